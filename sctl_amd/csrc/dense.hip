@@ -5,7 +5,8 @@
 // contiguous range of sources in tiles of TILE sources staged through LDS;
 // every lane of a wave reads the same source record (an LDS broadcast).  When
 // there are too few target blocks to fill the 256 CUs, the source range is
-// split over gridDim.y and the per-split sums are reduced in split order by a
+// split over the grid, down to a fraction of a tile per workgroup
+// (split_sources), and the per-split sums are reduced in split order by a
 // second kernel.  No MFMA: a pairwise sum is not a contraction.
 //
 // FP64 path: the accumulator runs over the sources in index order, as the
@@ -26,6 +27,7 @@ namespace sctl_amd {
 
 constexpr int WG = 256;
 constexpr int TILE = 256;
+constexpr int UNROLL = 2;  // sources per step of the pair loop; divides TILE
 
 // Far-away padding for the unused slots of a partial tile: the contribution is
 // a finite, vanishing kernel value times a zero density.
@@ -88,8 +90,9 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
 #pragma unroll
       for (int k = 0; k < K1; k++) saved[j][k] = acc[j][k];
 
-#pragma unroll 2
-    for (int i = 0; i < TILE; i++) {
+    // One source of the tile; `masked`: r2 == 0 contributes 0.
+    auto source = [&](int i, auto masked) {
+      constexpr bool MASK = decltype(masked)::value;
       const double* rec = lds + i * R;
       const double sx = rec[0], sy = rec[1], sz = rec[2];
       double n[3] = {0, 0, 0}, f[K0];
@@ -98,7 +101,13 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
 #pragma unroll
       for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
 #pragma unroll
-      for (int j = 0; j < TPL; j++) interact<KER, NEWTON, false>(acc[j], tx[j] - sx, ty[j] - sy, tz[j] - sz, n, f, mu);
+      for (int j = 0; j < TPL; j++) interact<KER, NEWTON, MASK>(acc[j], tx[j] - sx, ty[j] - sy, tz[j] - sz, n, f, mu);
+    };
+    // up to the first multiple of UNROLL at or past the tile's last source
+    // (the staged padding covers the rest)
+    for (int i = 0; i < len; i += UNROLL) {
+#pragma unroll
+      for (int u = 0; u < UNROLL; u++) source(i + u, std::false_type());
     }
 
     bool bad = false;
@@ -111,15 +120,7 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
       for (int j = 0; j < TPL; j++)
 #pragma unroll
         for (int k = 0; k < K1; k++) acc[j][k] = saved[j][k];
-      for (int i = 0; i < len; i++) {
-        const double* rec = lds + i * R;
-        double n[3] = {0, 0, 0}, f[K0];
-        for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
-        for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
-#pragma unroll
-        for (int j = 0; j < TPL; j++)
-          interact<KER, NEWTON, true>(acc[j], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], n, f, mu);
-      }
+      for (int i = 0; i < len; i++) source(i, std::true_type());
     }
   }
 
@@ -206,22 +207,34 @@ KMatFn kmat_fn(int ker, int newton) {
   });
 }
 
-// Splits the source range over gridDim.y when the target blocks alone cannot
-// fill the device (aim for >= 8 workgroups per CU, each split >= 4 tiles),
-// and so that no split exceeds SPLIT_TILES tiles (2 MiB of Laplace sources):
-// the workgroups resident at a time (dispatched in linear-index order) then
-// share one split in L2 rather than each streaming the whole source array.
-void split_sources(int64_t target_blocks, int64_t ntiles, int num_cus, int64_t* nsplit, int64_t* tiles_per_split) {
-  constexpr int64_t SPLIT_TILES = 256;
-  const int64_t want = 8LL * std::max(num_cus, 1);
-  int64_t ns_ = 1;
-  if (target_blocks < want) ns_ = (want + target_blocks - 1) / target_blocks;
-  ns_ = std::min<int64_t>(ns_, std::max<int64_t>(1, ntiles / 4));
-  ns_ = std::max<int64_t>(ns_, (ntiles + SPLIT_TILES - 1) / SPLIT_TILES);
-  ns_ = std::min<int64_t>(ns_, 65535);
-  int64_t tps = (ntiles + ns_ - 1) / ns_;
-  *tiles_per_split = tps;
-  *nsplit = (ntiles + tps - 1) / tps;
+// Splits the source range over the grid: *nsplit chunks of *chunk sources
+// (the last may be shorter), for about 32 workgroups per CU.  A chunk longer
+// than a tile is a whole number of tiles; a shorter one is a multiple of 64
+// sources.  Device time of one apply on MI355X, before and after small
+// problems were cut below four tiles per workgroup and large ones finer than
+// eight workgroups per CU (whose last ones left CUs idle):
+//   Laplace FxU 2000 x 3000     57.1 -> 11.2 us (8 target blocks: 24 -> 376 workgroups)
+//   Laplace DxU 2503 x 3001     74.2 -> 12.7 us
+//   Stokes FxU 5000 x 7000      79.4 -> 43 us
+//   Laplace DxU 100003 x 130001 8.84 -> 8.29 ms
+// At 16 workgroups per CU 20 000 x 20 000 took 4 % longer and nothing else
+// more than 1 % less; 32 instead of 64 sources gave nothing from 2000 points
+// on, where the per-workgroup latency and the reduction of more splits weigh
+// as much as the shorter loop.  No split is longer than SPLIT_TILES tiles
+// (2 MiB of Laplace sources): the workgroups resident at a time (dispatched in
+// linear-index order) then share one split in L2 rather than each streaming
+// the whole source array.
+void split_sources(int64_t target_blocks, int64_t ns, int num_cus, int64_t* nsplit, int64_t* chunk) {
+  constexpr int64_t SPLIT_TILES = 256, MIN_CHUNK = 64;
+  const int64_t want = 32LL * std::max(num_cus, 1);
+  int64_t n = target_blocks < want ? (want + target_blocks - 1) / target_blocks : 1;
+  n = std::max<int64_t>(n, (ns + SPLIT_TILES * TILE - 1) / (SPLIT_TILES * TILE));
+  n = std::min<int64_t>(n, 65535);
+  int64_t c = (ns + n - 1) / n;
+  const int64_t step = c > TILE ? TILE : MIN_CHUNK;
+  c = (c + step - 1) / step * step;
+  *chunk = c;
+  *nsplit = (ns + c - 1) / c;
 }
 
 }  // namespace
@@ -237,8 +250,8 @@ int f64_part_bytes(int ker, int64_t nt, int64_t ns, const DenseShape& shape, siz
   kernel_dims(ker, &K0, &K1, &ND);
   const int tpl = TPLS[std::min(tpl_index(shape.tpl), max_tpl_index(ker))];
   const int64_t tb = (nt + (int64_t)WG * tpl - 1) / ((int64_t)WG * tpl);
-  int64_t nsplit, tps;
-  split_sources(tb, (ns + TILE - 1) / TILE, dev.num_cus, &nsplit, &tps);
+  int64_t nsplit, chunk;
+  split_sources(tb, ns, dev.num_cus, &nsplit, &chunk);
   const size_t split_bytes = sizeof(double) * (size_t)nt * K1;
   const int64_t group = split_group(nsplit, split_bytes, part_budget);
   *bytes = group > 1 ? split_bytes * group : 0;
@@ -256,9 +269,8 @@ int f64_apply(int ker, int newton, const double* r_trg, int64_t nt, const double
   const int ti = std::min(tpl_index(shape.tpl), max_tpl_index(ker)), tpl = TPLS[ti];
   const int64_t tb = (nt + (int64_t)WG * tpl - 1) / ((int64_t)WG * tpl);
   SCTL_CHECK_ARG(tb <= 0x7fffffffLL, "too many targets for one launch");
-  const int64_t ntiles = (ns + TILE - 1) / TILE;
-  int64_t nsplit, tps;
-  split_sources(tb, ntiles, dev.num_cus, &nsplit, &tps);
+  int64_t nsplit, chunk;
+  split_sources(tb, ns, dev.num_cus, &nsplit, &chunk);
   const int64_t group = split_group(nsplit, sizeof(double) * (size_t)nt * K1, part_budget);
   SCTL_CHECK_ARG(group <= 1 || part, "no buffer for the split partial sums");
   const double scale = kernel_scale(ker) * fold_factor(ker, newton);
@@ -266,7 +278,6 @@ int f64_apply(int ker, int newton, const double* r_trg, int64_t nt, const double
   size_t dyn = 0;
   SCTL_TRY(occupancy_lds((const void*)fn, shape.occ, sizeof(double) * TILE * rec_words_f64(ker), &dyn));
   if (!stream_capturing(stream)) profile_count(ker, nt * ns);
-  const int64_t chunk = tps * TILE;
   // Groups of `group` splits: sources [y0*chunk, (y0+gy)*chunk) per launch.
   for (int64_t y0 = 0; y0 < nsplit; y0 += group) {
     const int64_t gy = std::min(group, nsplit - y0);
