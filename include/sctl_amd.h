@@ -196,8 +196,8 @@ int sctl_amd_dense_plan_destroy(sctl_amd_dense_plan plan);
  * Block b covers targets [trg_dsp[b], trg_dsp[b]+trg_cnt[b]) and sources
  * [src_dsp[b], src_dsp[b]+src_cnt[b]).  Target ranges of different blocks must
  * not overlap.  sctl_amd_plan_apply computes, for every block, the same
- * accumulation as sctl_amd_eval restricted to that block, in one persistent
- * launch fed by a work queue.
+ * accumulation as sctl_amd_eval restricted to that block, in one launch (and
+ * a second one that adds up the pieces of long source ranges).
  *
  * The offset/count arrays are host memory, copied at creation. */
 typedef struct sctl_amd_plan_s* sctl_amd_plan;

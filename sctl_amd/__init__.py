@@ -10,7 +10,7 @@ operations for Python hosts:
     and zeroes ``v_trg`` when its length is wrong, otherwise accumulates.
   * ``GenericKernel(kernel).KernelMatrix(r_trg, r_src, n_src)``
     -- ``GenericKernel<uKernel>::KernelMatrix`` (generic-kernel.txx:213-329).
-  * ``Plan`` -- batched near-field blocks in one persistent launch.
+  * ``Plan`` -- batched near-field blocks in one launch.
 
 The library is required: importing works without it, but every call raises
 ``LibraryNotBuilt`` (there is no CPU fallback).
@@ -344,7 +344,7 @@ class GenericKernel:
 
 # ------------------------------------------------------------------ batched
 class Plan:
-    """Batched (target-set, source-set) blocks evaluated in one persistent launch."""
+    """Batched (target-set, source-set) blocks evaluated in one launch."""
 
     def __init__(self, kernel, trg_dsp, trg_cnt, src_dsp, src_cnt, nt_total, ns_total, precision=FP64, digits=-1,
                  ctx=None):

@@ -3,12 +3,21 @@
 // BoundaryIntegralOp evaluates thousands of small, uneven (target-set,
 // source-set) blocks (boundary_integral.txx:1009-1032 builds them, :1169-1238
 // and :1342-1364 evaluate them one OpenMP task each).  Here all blocks of a
-// plan run in ONE persistent launch:
+// plan run in ONE launch (and one more that adds up cut chunks):
 //
-//  * Work items are (block, chunk of <= 64*TPL targets).  Items are ordered by
-//    cost Ns*Nt, largest first (longest-processing-time order), and every
-//    wave of the persistent grid takes the next item from a global atomic
-//    counter, so the tail of the launch is made of the smallest items.
+//  * Work items are (block, chunk of <= 64*TPL targets, piece of the block's
+//    sources), one per wave, ordered by cost, largest first, four to a
+//    workgroup.  The hardware's dispatcher hands the workgroups out in that
+//    order as others end, so the tail of the launch is made of the smallest
+//    items.  (Waves of a persistent grid taking items from one atomic counter
+//    got at most ~75 items per microsecond out of it, which bounded batches of
+//    short pieces: 512 torus blocks in 64-source pieces 390 us, dispatched 146.)
+//  * A chunk against a long source range would keep one wave busy after all
+//    others have ended (128 targets x 4096 sources: 300 us alone on a SIMD),
+//    so it is cut into pieces (build_items) whose sums k_sum_pieces adds up in
+//    piece order.  FP64 Laplace double layer, 4096 torus blocks 1.25 -> 1.08
+//    ms, 512 blocks 509 -> 146 us; mixed Stokes double layer 1.22 -> 1.03 ms
+//    and 508 -> 149 us.
 //  * A wave owns an item; each lane holds TPL targets.  Chunks of <= 16*TPL or
 //    <= 32*TPL targets use G = 4 or 2 lane groups (64/G lanes each): group g
 //    takes every G-th source and the groups' sums are combined with
@@ -26,9 +35,7 @@
 //
 // The knobs (SPL: LDS stage size, TPL: targets per lane, a cap on resident
 // workgroups per CU) are chosen per plan by the tuner (tune.cpp) or defaults.
-// Every wave leaves the loop when the counter passes the number of items, so
-// the grid always drains.  An apply allocates nothing and issues no memset
-// (the counter is cleared by a one-lane kernel), so it can be captured in a
+// An apply allocates nothing and issues no memset, so it can be captured in a
 // hipGraph.
 #include <hip/hip_runtime.h>
 
@@ -47,6 +54,7 @@ namespace sctl_amd {
 namespace {
 
 constexpr int BWG = 256;  // 4 waves per workgroup, each wave independent
+constexpr int SWG = 128;  // threads that add up a cut chunk's pieces
 
 // Padding of a partial source stage: the slots past the block's last source
 // repeat the stage's first source with zero density and normal.  Every
@@ -60,12 +68,6 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ int next_item(int* counter, int lane) {
-  int it = 0;
-  if (lane == 0) it = atomicAdd(counter, 1);
-  return __builtin_amdgcn_readfirstlane(it);
 }
 
 __device__ __forceinline__ double shfl_xor_d(double v, int m) {
@@ -95,28 +97,13 @@ template <int STAGE, class Body> __device__ __forceinline__ void group_sources(i
   }
 }
 
-__global__ void k_reset_counter(int* counter) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *counter = 0;
-}
-
 // ------------------------------------------------------------- FP64 blocks
-// The Laplace double layer with f n staged per source: z^3 (f n).r, one
-// multiplication per pair fewer than n.r z^3 f.
-template <int NEWTON, bool MASK>
-__device__ __forceinline__ void lap_dxu_fn(double& acc, double rx, double ry, double rz, const double* fn) {
-  const double r2 = fmad(rz, rz, fmad(ry, ry, rx * rx));
-  double z = rsq_deferred<NEWTON>(r2);
-  if constexpr (MASK) z = r2 > 0.0 ? z : 0.0;
-  const double nd = fmad(rz, fn[2], fmad(ry, fn[1], rx * fn[0]));
-  acc = fmad(nd, z * z * z, acc);
-}
-
 template <int KER, int NEWTON, int SPL, int TPL>
 __global__ void __launch_bounds__(BWG)
-k_blocks_f64(const Item* __restrict__ items, int nitems, int* __restrict__ counter,
+k_blocks_f64(const Item* __restrict__ items, int nitems,
              const int64_t* __restrict__ trg_dsp, const int64_t* __restrict__ src_dsp,
-             const int32_t* __restrict__ src_cnt, const double* __restrict__ xt, const double* __restrict__ xs,
-             const double* __restrict__ xn, const double* __restrict__ fs, double* __restrict__ out, double scale,
+             const double* __restrict__ xt, const double* __restrict__ xs, const double* __restrict__ xn,
+             const double* __restrict__ fs, double* __restrict__ out, double* __restrict__ part, double scale,
              double mu) {
   using K = Ker<KER>;
   constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, R = rec_f64<KER>(), STAGE = 64 * SPL;
@@ -124,14 +111,15 @@ k_blocks_f64(const Item* __restrict__ items, int nitems, int* __restrict__ count
   const int lane = threadIdx.x & 63;
   double* lds = lds_all + (threadIdx.x >> 6) * (STAGE * R);
 
-  for (int it = next_item(counter, lane); it < nitems; it = next_item(counter, lane)) {
+  const int first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (BWG / 64) + (threadIdx.x >> 6)));
+  for (int64_t it = first; it < nitems; it += (int64_t)gridDim.x * (BWG / 64)) {
     const Item I = items[it];
     const int lg = I.lg, G = 1 << lg, L = 64 >> lg;
     const int g = lane >> (6 - lg), tl = lane & (L - 1);
     const int64_t tb = trg_dsp[I.block] + I.t_off;
     bool tv[TPL];
     int64_t t[TPL];
-    double tx[TPL], ty[TPL], tz[TPL], acc[TPL][K1];
+    double tx[TPL], ty[TPL], tz[TPL], tot[TPL][K1];
 #pragma unroll
     for (int j = 0; j < TPL; j++) {
       tv[j] = tl + j * L < I.t_cnt;
@@ -140,10 +128,10 @@ k_blocks_f64(const Item* __restrict__ items, int nitems, int* __restrict__ count
       ty[j] = xt[t[j] * 3 + 1];
       tz[j] = xt[t[j] * 3 + 2];
 #pragma unroll
-      for (int k = 0; k < K1; k++) acc[j][k] = 0.0;
+      for (int k = 0; k < K1; k++) tot[j][k] = 0.0;
     }
-    const int64_t sb = src_dsp[I.block];
-    const int nsb = src_cnt[I.block];
+    const int64_t sb = src_dsp[I.block] + I.s_off;
+    const int nsb = I.s_cnt;
 
     for (int s0 = 0; s0 < nsb; s0 += STAGE) {
       const int len = min(STAGE, nsb - s0);
@@ -161,16 +149,16 @@ k_blocks_f64(const Item* __restrict__ items, int nitems, int* __restrict__ count
 #pragma unroll
         for (int k = 0; k < ND; k++) rec[3 + k] = real ? fn * xn[s * 3 + k] : 0.0;
 #pragma unroll
-        for (int k = 0; k < K0; k++) rec[3 + ND + k] = real ? fs[s * K0 + k] : 0.0;
+        for (int k = 0; k < (KER == LAP_DXU ? 0 : K0); k++) rec[3 + ND + k] = real ? fs[s * K0 + k] : 0.0;
 #pragma unroll
         for (int k = 3 + ND + K0; k < R; k++) rec[k] = 0.0;
       }
       wave_sync();
-      double saved[TPL][K1];
+      double acc[TPL][K1];  // this stage's sums
 #pragma unroll
       for (int j = 0; j < TPL; j++)
 #pragma unroll
-        for (int k = 0; k < K1; k++) saved[j][k] = acc[j][k];
+        for (int k = 0; k < K1; k++) acc[j][k] = 0.0;
       group_sources<STAGE>(lg, g, len, [&](int i) {
         const double* rec = lds + i * R;
         if constexpr (KER == LAP_DXU) {
@@ -197,7 +185,7 @@ k_blocks_f64(const Item* __restrict__ items, int nitems, int* __restrict__ count
 #pragma unroll
         for (int j = 0; j < TPL; j++)
 #pragma unroll
-          for (int k = 0; k < K1; k++) acc[j][k] = saved[j][k];
+          for (int k = 0; k < K1; k++) acc[j][k] = 0.0;
         for (int i = g; i < len; i += G) {
           const double* rec = lds + i * R;
           if constexpr (KER == LAP_DXU) {
@@ -214,15 +202,22 @@ k_blocks_f64(const Item* __restrict__ items, int nitems, int* __restrict__ count
           }
         }
       }
+#pragma unroll
+      for (int j = 0; j < TPL; j++)
+#pragma unroll
+        for (int k = 0; k < K1; k++) tot[j][k] += acc[j][k];
     }
 #pragma unroll
     for (int j = 0; j < TPL; j++) {
       for (int m = L; m < 64; m <<= 1)
 #pragma unroll
-        for (int k = 0; k < K1; k++) acc[j][k] += shfl_xor_d(acc[j][k], m);
+        for (int k = 0; k < K1; k++) tot[j][k] += shfl_xor_d(tot[j][k], m);
       if (g == 0 && tv[j]) {
 #pragma unroll
-        for (int k = 0; k < K1; k++) out[t[j] * K1 + k] += acc[j][k] * scale;
+        for (int k = 0; k < K1; k++) {
+          if (I.part < 0) out[t[j] * K1 + k] += tot[j][k] * scale;
+          else part[I.part + (int64_t)(tl + j * L) * K1 + k] = tot[j][k];
+        }
       }
     }
   }
@@ -270,11 +265,11 @@ __device__ __forceinline__ void lap_pair_r2d(float& p, double tx, double ty, dou
 
 template <int KER, int NEWTON, int SPL, int TPL>
 __global__ void __launch_bounds__(BWG)
-k_blocks_mixed(const Item* __restrict__ items, int nitems, int* __restrict__ counter,
+k_blocks_mixed(const Item* __restrict__ items, int nitems,
                const int64_t* __restrict__ trg_dsp, const int64_t* __restrict__ src_dsp,
-               const int32_t* __restrict__ src_cnt, const double* __restrict__ xt, const double* __restrict__ xs,
-               const double* __restrict__ xn, const double* __restrict__ fs, double* __restrict__ out,
-               double scale, double ctx) {
+               const double* __restrict__ xt, const double* __restrict__ xs, const double* __restrict__ xn,
+               const double* __restrict__ fs, double* __restrict__ out, double* __restrict__ part, double scale,
+               double ctx) {
   const float mu = (float)ctx;
   using K = Ker<KER>;
   constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, STAGE = 64 * SPL;
@@ -287,7 +282,8 @@ k_blocks_mixed(const Item* __restrict__ items, int nitems, int* __restrict__ cou
   double* pos = pos_all + (threadIdx.x >> 6) * (STAGE * PW);
   float* aux = aux_all + (threadIdx.x >> 6) * (STAGE * AW);
 
-  for (int it = next_item(counter, lane); it < nitems; it = next_item(counter, lane)) {
+  const int first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (BWG / 64) + (threadIdx.x >> 6)));
+  for (int64_t it = first; it < nitems; it += (int64_t)gridDim.x * (BWG / 64)) {
     const Item I = items[it];
     const int lg = I.lg, G = 1 << lg, L = 64 >> lg;
     const int g = lane >> (6 - lg), tl = lane & (L - 1);
@@ -305,8 +301,8 @@ k_blocks_mixed(const Item* __restrict__ items, int nitems, int* __restrict__ cou
 #pragma unroll
       for (int k = 0; k < K1; k++) acc[j][k] = comp[j][k] = 0.0;
     }
-    const int64_t sb = src_dsp[I.block];
-    const int nsb = src_cnt[I.block];
+    const int64_t sb = src_dsp[I.block] + I.s_off;
+    const int nsb = I.s_cnt;
 
     for (int s0 = 0; s0 < nsb; s0 += STAGE) {
       const int len = min(STAGE, nsb - s0);
@@ -406,14 +402,46 @@ k_blocks_mixed(const Item* __restrict__ items, int nitems, int* __restrict__ cou
         for (int k = 0; k < K1; k++) v[k] += shfl_xor_d(v[k], m);
       if (g == 0 && tv[j]) {
 #pragma unroll
-        for (int k = 0; k < K1; k++) out[t[j] * K1 + k] += v[k] * scale;
+        for (int k = 0; k < K1; k++) {
+          if (I.part < 0) out[t[j] * K1 + k] += v[k] * scale;
+          else part[I.part + (int64_t)(tl + j * L) * K1 + k] = v[k];
+        }
       }
     }
   }
 }
 
-using BlocksFn = void (*)(const Item*, int, int*, const int64_t*, const int64_t*, const int32_t*, const double*,
-                          const double*, const double*, const double*, double*, double, double);
+// One workgroup per chunk that was cut into pieces: out += scale * (the sum of
+// the pieces' partial sums, in piece order).
+__global__ void __launch_bounds__(SWG)
+k_sum_pieces(const SplitChunk* __restrict__ chunks, int K1, const double* __restrict__ part, double* __restrict__ out,
+             double scale) {
+  const SplitChunk C = chunks[blockIdx.x];
+  const int n = C.t_cnt * K1;
+  if (C.pieces > 32) {  // few targets, many pieces: four lanes per value
+    for (int i0 = 0; i0 < n; i0 += SWG / 4) {
+      const int i = i0 + (int)(threadIdx.x >> 2);
+      const double s = sum_splits_quad(part + C.part, n, C.pieces, i, i < n);
+      if (i < n && (threadIdx.x & 3) == 0) out[C.t_base * K1 + i] += s * scale;
+    }
+    return;
+  }
+  for (int i = threadIdx.x; i < n; i += SWG) {
+    const double* p = part + C.part + i;
+    double s = 0.0;
+    for (int y = 0; y < C.pieces; y += 8) {
+      double v[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) v[k] = y + k < C.pieces ? p[(int64_t)(y + k) * n] : 0.0;
+#pragma unroll
+      for (int k = 0; k < 8; k++) s += v[k];
+    }
+    out[C.t_base * K1 + i] += s * scale;
+  }
+}
+
+using BlocksFn = void (*)(const Item*, int, const int64_t*, const int64_t*, const double*, const double*,
+                          const double*, const double*, double*, double*, double, double);
 
 // Targets per lane: 1 or 2 (2 only where max_tpl allows it).
 template <int KER, int NEWTON, int SPL> BlocksFn f64_blocks_t(int tpl) {
@@ -461,7 +489,7 @@ size_t blocks_lds(int ker, int precision, int spl) {
     if (ker == LAP_DXU) return stage * (6 * sizeof(double) + sizeof(float));  // s, f n; one unused float
     return stage * (4 * sizeof(double) + (((ND + K0) + 3) & ~3) * sizeof(float));
   }
-  return stage * (((3 + ND + K0) + 1) & ~1) * sizeof(double);
+  return stage * (ker == LAP_DXU ? 6 : ((3 + ND + K0) + 1) & ~1) * sizeof(double);
 }
 }  // namespace
 }  // namespace sctl_amd
@@ -473,27 +501,53 @@ namespace sctl_amd {
 namespace {
 
 // Work items for `tpl` targets per lane: chunks of <= 64*tpl targets, lane
-// groups for small chunks, longest (Ns x lanes) first.
-std::vector<Item> build_items(const sctl_amd_plan_s* p, int tpl) {
+// groups for small chunks, longest first.  Cost: sources x lanes x tpl.  A
+// chunk is cut into pieces of a third of what one wave of twelve per CU has to
+// do on average, and of at least 128 sources of a full chunk: finer pieces
+// (a 6th, a 12th) were 1-2 % slower on 4096 blocks, a 64- or 256-source bound
+// within 2 % on 512.
+constexpr int PIECES_PER_WAVE = 3, MIN_PIECE = 128;
+struct WorkList {
+  std::vector<Item> items;
+  std::vector<SplitChunk> split;
+  int64_t part_words = 0;
+};
+WorkList build_items(const sctl_amd_plan_s* p, int tpl, int num_cus) {
+  WorkList w;
+  const int64_t chunk = 64LL * tpl;
+  auto groups = [&](int64_t cnt) { return cnt <= 16 * tpl ? 2 : (cnt <= 32 * tpl ? 1 : 0); };
+  int64_t total = 0;
+  for (int64_t b = 0; b < p->nblocks; b++)
+    for (int64_t t0 = 0; t0 < p->trg_cnt[b]; t0 += chunk)
+      total += (chunk >> groups(std::min<int64_t>(chunk, p->trg_cnt[b] - t0))) * p->src_cnt[b];
+  const int64_t piece_cost = std::max<int64_t>(chunk * MIN_PIECE, total / (12LL * num_cus * PIECES_PER_WAVE));
   std::vector<Item> items;
   std::vector<int64_t> cost;
-  const int64_t chunk = 64LL * tpl;
   for (int64_t b = 0; b < p->nblocks; b++) {
     const int64_t tc = p->trg_cnt[b], sc = p->src_cnt[b];
     if (!tc || !sc) continue;
     for (int64_t t0 = 0; t0 < tc; t0 += chunk) {
       const int cnt = (int)std::min<int64_t>(chunk, tc - t0);
-      const int lg = cnt <= 16 * tpl ? 2 : (cnt <= 32 * tpl ? 1 : 0);
-      items.push_back(Item{(int32_t)b, (int32_t)t0, cnt, lg});
-      cost.push_back((int64_t)(64 >> lg) * tpl * sc);
+      const int lg = groups(cnt);
+      const int64_t lanes = chunk >> lg;
+      int64_t n = (lanes * sc + piece_cost - 1) / piece_cost;
+      const int64_t len = ((sc + n - 1) / n + 63) / 64 * 64;
+      n = (sc + len - 1) / len;
+      if (n > 1) w.split.push_back(SplitChunk{p->trg_dsp[b] + t0, w.part_words, cnt, (int32_t)n});
+      for (int64_t i = 0; i < n; i++) {
+        const int64_t s0 = i * len, sn = std::min<int64_t>(len, sc - s0);
+        items.push_back(Item{(int32_t)b, (int32_t)t0, cnt, lg, (int32_t)s0, (int32_t)sn, n > 1 ? w.part_words : -1});
+        cost.push_back(lanes * sn);
+        if (n > 1) w.part_words += (int64_t)cnt * p->K1;
+      }
     }
   }
   std::vector<size_t> idx(items.size());
   std::iota(idx.begin(), idx.end(), 0);
   std::stable_sort(idx.begin(), idx.end(), [&](size_t a, size_t b) { return cost[a] > cost[b]; });
-  std::vector<Item> sorted(items.size());
-  for (size_t i = 0; i < idx.size(); i++) sorted[i] = items[idx[i]];
-  return sorted;
+  w.items.resize(items.size());
+  for (size_t i = 0; i < idx.size(); i++) w.items[i] = items[idx[i]];
+  return w;
 }
 
 BlocksFn plan_fn(const sctl_amd_plan_s* p, const PlanShape& s) {
@@ -504,7 +558,7 @@ BlocksFn plan_fn(const sctl_amd_plan_s* p, const PlanShape& s) {
 }  // namespace
 
 // Applies knobs to a plan: rebuilds the work items for the targets per lane
-// and sizes the persistent grid from the occupancy calculator (with the cap).
+// and sizes the dynamic LDS that enforces the cap on resident workgroups.
 int plan_configure(sctl_amd_plan_s* p, PlanShape s) {
   DeviceInfo dev;
   SCTL_TRY(device_info(&dev));
@@ -512,19 +566,24 @@ int plan_configure(sctl_amd_plan_s* p, PlanShape s) {
   s.tpl = s.tpl >= 2 && plan_max_tpl(p->kernel) >= 2 ? 2 : 1;
   s.occ = std::max(0, s.occ);
   if (!p->d_items || s.tpl != p->shape.tpl) {
-    const std::vector<Item> items = build_items(p, s.tpl);
-    SCTL_CHECK_ARG(items.size() < 0x7fffffffULL, "too many work items");
-    if (p->d_items) SCTL_HIP_TRY(hipFree(p->d_items));
+    const WorkList w = build_items(p, s.tpl, std::max(dev.num_cus, 1));
+    SCTL_CHECK_ARG(w.items.size() < 0x7fffffffULL, "too many work items");
+    p->nitems = p->nsplit = 0;
+    void* old[] = {p->d_items, p->d_split, p->d_part};
     p->d_items = nullptr;
-    SCTL_TRY(dev_upload(&p->d_items, items));
-    p->nitems = (int)items.size();
+    p->d_split = nullptr;
+    p->d_part = nullptr;
+    for (void* q : old)
+      if (q) SCTL_HIP_TRY(hipFree(q));
+    SCTL_TRY(dev_upload(&p->d_items, w.items));
+    SCTL_TRY(dev_upload(&p->d_split, w.split));
+    if (w.part_words) SCTL_HIP_TRY(hipMalloc(&p->d_part, sizeof(double) * w.part_words));
+    p->nitems = (int)w.items.size();
+    p->nsplit = (int)w.split.size();
   }
   const BlocksFn fn = plan_fn(p, s);
   size_t dyn = 0;
   SCTL_TRY(occupancy_lds((const void*)fn, s.occ, blocks_lds(p->kernel, p->precision, s.spl), &dyn));
-  int per_cu = 0;
-  SCTL_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, BWG, dyn));
-  p->grid = std::max(1, per_cu) * dev.num_cus;
   p->dyn_lds = dyn;
   p->shape = s;
   p->generation++;
@@ -548,17 +607,22 @@ PlanShape plan_shape(sctl_amd_plan p) { return p ? p->shape : PlanShape(); }
 
 int plan_launch(sctl_amd_plan_s* p, const double* v_src, double* v_trg, hipStream_t s) {
   if (p->nitems == 0) return SCTL_AMD_SUCCESS;
-  hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, s, p->d_counter);
-  SCTL_HIP_TRY(hipGetLastError());
-  const double scale = kernel_scale(p->kernel) * fold_factor(p->kernel, p->newton);
-  const int grid = (int)std::min<int64_t>(p->grid, ((int64_t)p->nitems + 3) / 4);
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   SCTL_HIP_TRY(hipStreamIsCapturing(s, &cs));
+  const double scale = (double)(kernel_scale(p->kernel) * fold_factor(p->kernel, p->newton));
+  // Four items per workgroup; past 2^22 workgroups (a grid of 2^30 threads) they loop.
+  const unsigned grid = (unsigned)std::min<int64_t>(1 << 22, ((int64_t)p->nitems + BWG / 64 - 1) / (BWG / 64));
   if (cs == hipStreamCaptureStatusNone) profile_count(p->kernel, p->interactions);  // graphs count per launch
-  ProfileScope prof(s);
-  hipLaunchKernelGGL(plan_fn(p, p->shape), dim3(grid), dim3(BWG), p->dyn_lds, s, p->d_items, p->nitems, p->d_counter,
-                     p->d_trg_dsp, p->d_src_dsp, p->d_src_cnt, p->d_xt, p->d_xs, p->d_xn, v_src, v_trg, scale, p->ctx);
+  {
+    ProfileScope prof(s);
+    hipLaunchKernelGGL(plan_fn(p, p->shape), dim3(grid), dim3(BWG), p->dyn_lds, s, p->d_items, p->nitems,
+                       p->d_trg_dsp, p->d_src_dsp, p->d_xt, p->d_xs, p->d_xn, v_src, v_trg, p->d_part, scale, p->ctx);
+  }
   SCTL_HIP_TRY(hipGetLastError());
+  if (p->nsplit) {
+    hipLaunchKernelGGL(k_sum_pieces, dim3(p->nsplit), dim3(SWG), 0, s, p->d_split, p->K1, p->d_part, v_trg, scale);
+    SCTL_HIP_TRY(hipGetLastError());
+  }
   return SCTL_AMD_SUCCESS;
 }
 
@@ -634,22 +698,16 @@ int sctl_amd_plan_create(sctl_amd_plan* plan, int kernel, int precision, int dig
   if (!rc) rc = dev_upload(&p->d_src_cnt, v_sc);
   if (!rc) rc = dev_upload(&p->d_trg_cnt, v_tc);
   if (!rc) {
-    hipError_t e = hipMalloc(&p->d_counter, sizeof(int));
-    if (e != hipSuccess) {
-      set_error(std::string("hipMalloc(counter): ") + hipGetErrorString(e));
-      rc = SCTL_AMD_ERROR_OUT_OF_MEMORY;
-    }
-  }
-  if (!rc) {
     PlanShape s;
     if (!lookup_plan_shape(kernel, precision, p->interactions, p->nonempty, &s)) {
-      // Untuned default, from sweeps of 4096- and 2048-block surface
-      // batches (Laplace and Stokes double layers) on MI355X: 256-source
-      // stages and two targets per lane; at most two workgroups per CU for
-      // mixed scalar outputs, four otherwise.
-      s.spl = 4;
+      // Untuned default, from sweeps of 4096- and 512-block surface batches
+      // (Laplace and Stokes double layers) on MI355X: two targets per lane and
+      // 128-source stages (64 for mixed scalar outputs), whose LDS leaves room
+      // for the waves that the registers allow; 256-source stages are 2-20 %
+      // slower in mixed precision and even in FP64, a cap never helps.
+      s.spl = (precision == SCTL_AMD_MIXED && K1 == 1) ? 1 : 2;
       s.tpl = 2;
-      s.occ = (precision == SCTL_AMD_MIXED && K1 == 1) ? 2 : 4;
+      s.occ = 0;
     }
     rc = plan_configure(p, s);
   }

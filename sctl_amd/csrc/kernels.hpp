@@ -20,7 +20,7 @@
 // refined by one deferred-scaling Newton step, the scheme of
 // intrin-wrapper.hpp:540-559 (z <- z * (x*z*z - 3), the constant -1/2 applied
 // once), for about 14 digits, or by one third-order step for full FP64
-// precision (rsq_deferred).  The Newton constant is folded into the
+// precision (rsq_deferred).  The constant of either step is folded into the
 // per-target scale wherever the kernel value is a single power of 1/r
 // (Laplace FxU: r^-1, Laplace DxU and FxdU, BiotSavart FxU: r^-3, Stokes DxU
 // and FxT: r^-5); the other kernels scale 1/r once per pair.
@@ -98,7 +98,9 @@ template <int KER> constexpr int max_tpl() { return Ker<KER>::K1 <= 3 ? 4 : (Ker
 // Words per packed source record: position, normal (if any), density.
 template <int KER> constexpr int src_words() { return 3 + Ker<KER>::ND + Ker<KER>::K0; }
 // Record widths padded to 16 bytes (LDS reads of 128 bits).
-template <int KER> constexpr int rec_f64() { return (src_words<KER>() + 1) & ~1; }
+// The Laplace double layer's FP64 record holds f n in place of n and f
+// (lap_dxu_fn).
+template <int KER> constexpr int rec_f64() { return KER == LAP_DXU ? 6 : (src_words<KER>() + 1) & ~1; }
 template <int KER> constexpr int rec_f32() { return (src_words<KER>() + 3) & ~3; }
 
 __device__ __forceinline__ double hw_rsq(double x) { return __builtin_amdgcn_rsq(x); }
@@ -268,40 +270,68 @@ __device__ __forceinline__ void helmholtz_factor(T r2, T z, T mu, T* G0, T* G1) 
   }
 }
 
-// Deferred-scaling Newton constants (intrin-wrapper.hpp:540-559).  NEWTON = 2
-// (full FP64 precision) is not two deferred steps here but one third-order
-// step, which needs no final constant (newton_c2(2) = 1; see rsq_deferred).
+// Deferred-scaling constants.  NEWTON = 1: intrin-wrapper.hpp:540-559.
+// NEWTON = 2 (full FP64 precision) is not two deferred steps here but one
+// third-order step in one of two forms (rsq_deferred): FOLD = true leaves the
+// factor 1 / h0 of the completed square to the caller, FOLD = false needs no
+// factor.
+constexpr double CUBIC_E = 5.0 / 3.0, CUBIC_H = 20.0 / 9.0;
 __host__ __device__ constexpr double newton_c1(int j) { return j == 0 ? -3.0 : (j == 1 ? -12.0 : -768.0); }
 __host__ __device__ constexpr double newton_c2(int n) { return n == 1 ? -0.5 : 1.0; }
-__host__ __device__ constexpr double ipow(double x, int p) { return p == 0 ? 1.0 : x * ipow(x, p - 1); }
+__host__ __device__ constexpr long double ipow(long double x, int p) { return p == 0 ? 1.0L : x * ipow(x, p - 1); }
 
-// Unscaled rsqrt: equals newton_c2(NEWTON)^-1 / sqrt(x) up to rounding.
+// Unscaled rsqrt: equals c^-1 / sqrt(x) up to rounding, with c =
+// newton_c2(NEWTON), or 1 / h0 for NEWTON 2 with FOLD.
 //   NEWTON 0: the hardware estimate (v_rsq_f64 / v_rsq_f32, ~2^-23 relative);
 //   NEWTON 1: one deferred Newton step z (x z^2 - 3) (= -2 / sqrt(x), ~2^-47);
 //   NEWTON 2: the third-order step z (1 + e/2 + 3 e^2 / 8), e = 1 - x z^2,
 //             the first terms of (1 - e)^(-1/2) (Householder's method of
 //             order 3): error ~ (5/16) e^3 ~ 2^-70, i.e. rounding only, in 5
 //             operations instead of the 6 of two deferred Newton steps.
-template <int NEWTON, class T> __device__ __forceinline__ T rsq_deferred(T x) {
+//             With FOLD the polynomial's square is completed,
+//               1 + e/2 + 3 e^2 / 8 = ((e + 2/3)^2 + 20/9) 3/8,
+//             and the 3/8 left out: 4 operations (x z, e + 2/3 in one FMA,
+//             the square in another, the product).  Its value at e = 0, h0 =
+//             (CUBIC_E - 1)^2 + CUBIC_H = 8/3 up to rounding, is divided out
+//             by fold_factor.  The FP64 kernels of one power of 1/r are bound
+//             by VALU issue, so the operation counts in time: Laplace FxU 16
+//             -> 15 issue slots per pair (v_rsq_f64 takes four).
+template <int NEWTON, bool FOLD = false, class T> __device__ __forceinline__ T rsq_deferred(T x) {
   T z = hw_rsq(x);
   if constexpr (NEWTON == 1) z = z * fmad(x, z * z, (T)newton_c1(0));
-  if constexpr (NEWTON >= 2) {
+  if constexpr (NEWTON >= 2 && FOLD) {
+    const T e = fmad(-(x * z), z, (T)CUBIC_E);
+    z = z * fmad(e, e, (T)CUBIC_H);
+  } else if constexpr (NEWTON >= 2) {
     const T e = fmad(-(x * z), z, (T)1);
     z = fmad(z * e, fmad(e, (T)0.375, (T)0.5), z);
   }
   return z;
 }
 
-// Factor that turns the accumulated (unscaled) sum into the kernel value:
-// newton_c2^POW for single-power kernels, 1 for the others (scaled in-loop).
-template <int KER, int NEWTON> __host__ __device__ constexpr double fold_factor() {
-  return Ker<KER>::POW ? ipow(newton_c2(NEWTON), Ker<KER>::POW) : 1.0;
+// Factor that turns the accumulated (unscaled) sum into the kernel value: the
+// rsqrt's constant to the kernel's power for single-power kernels, 1 for the
+// others (scaled in-loop).
+template <int KER, int NEWTON> __host__ __device__ constexpr long double fold_factor() {
+  constexpr long double e0 = (long double)CUBIC_E - 1, h0 = e0 * e0 + (long double)CUBIC_H;
+  return Ker<KER>::POW ? ipow(NEWTON >= 2 ? 1 / h0 : (long double)newton_c2(NEWTON), Ker<KER>::POW) : 1.0L;
 }
-inline double fold_factor(int ker, int newton) {
+inline long double fold_factor(int ker, int newton) {
   return with_kernel(ker, [&](auto kc) {
     constexpr int K = decltype(kc)::value;
     return newton == 0 ? fold_factor<K, 0>() : (newton == 1 ? fold_factor<K, 1>() : fold_factor<K, 2>());
   });
+}
+
+// The FP64 Laplace double layer with f n per source: z^3 (f n).r, one
+// multiplication per pair fewer than n.r z^3 f, and two words less per record.
+template <int NEWTON, bool MASK>
+__device__ __forceinline__ void lap_dxu_fn(double& acc, double rx, double ry, double rz, const double* fn) {
+  const double r2 = fmad(rz, rz, fmad(ry, ry, rx * rx));
+  double z = rsq_deferred<NEWTON, true>(r2);
+  if constexpr (MASK) z = r2 > 0.0 ? z : 0.0;
+  const double nd = fmad(rz, fn[2], fmad(ry, fn[1], rx * fn[0]));
+  acc = fmad(nd, z * z * z, acc);
 }
 
 // acc[K1] += K(r, n) * f  (fused apply, unscaled).  r = x_t - x_s.
@@ -310,7 +340,7 @@ inline double fold_factor(int ker, int newton) {
 template <int KER, int NEWTON, bool MASK, class T>
 __device__ __forceinline__ void interact(T* acc, T rx, T ry, T rz, const T* n, const T* f, T mu = (T)0) {
   const T r2 = fmad(rz, rz, fmad(ry, ry, rx * rx));
-  T z = rsq_deferred<NEWTON>(r2);
+  T z = rsq_deferred<NEWTON, Ker<KER>::POW != 0>(r2);
   if constexpr (MASK) z = (r2 > (T)0) ? z : (T)0;
   if constexpr (KER == LAP_FXU) {
     acc[0] = fmad(z, f[0], acc[0]);

@@ -594,7 +594,7 @@ int mixed_apply(int ker, int newton, const MixedGeometry& g, const DenseShape& s
   hipLaunchKernelGGL(pack_fn(ker), dim3((unsigned)(g.ntiles + (nt + WG - 1) / WG)), dim3(WG), 0, stream, r_src, n_src,
                      v_src, ns, sperm, packed, meta, sub, g.ntiles, r_trg, nt, tperm, xt_sorted);
   SCTL_HIP_TRY(hipGetLastError());
-  const double scale = kernel_scale(ker) * fold_factor(ker, newton ? 1 : 0);
+  const double scale = (double)(kernel_scale(ker) * fold_factor(ker, newton ? 1 : 0));
   const EvalMixFn fn = mix_fn(ker, newton, g.ti);
   size_t dyn = 0;
   SCTL_TRY(occupancy_lds((const void*)fn, shape.occ, sizeof(float4) * TILE * g.Q, &dyn));

@@ -11,12 +11,24 @@
 
 namespace sctl_amd {
 
-// One work item of the batched Eval: a chunk of one block's targets.
+// One work item of the batched Eval: a chunk of one block's targets against a
+// piece of the block's sources.
 struct Item {
   int32_t block;  // block index
   int32_t t_off;  // first target of the chunk, relative to the block
   int32_t t_cnt;  // targets in the chunk (<= 64*TPL)
   int32_t lg;     // log2 of the number of lane groups
+  int32_t s_off;  // first source of the piece, relative to the block
+  int32_t s_cnt;  // sources in the piece
+  int64_t part;   // where the piece's sums go in the partial sums; -1: the only piece, added to the output
+};
+
+// A chunk cut into pieces: its targets' sums are those of the pieces' partial
+// sums, t_cnt * K1 words each, in order.
+struct SplitChunk {
+  int64_t t_base;  // first target of the chunk in the plan's target array
+  int64_t part;    // the first piece's partial sums
+  int32_t t_cnt, pieces;
 };
 
 // Wave tiles of the near-field operators, as a flattened list: tile i
@@ -45,7 +57,6 @@ struct sctl_amd_plan_s {
   std::vector<int64_t> trg_dsp, trg_cnt, src_dsp, src_cnt;  // host copies
   int nitems = 0;
   sctl_amd::PlanShape shape;  // resolved knobs
-  int grid = 0;               // persistent grid (workgroups)
   size_t dyn_lds = 0;         // dynamic LDS that enforces shape.occ
   bool has_geometry = false;
   double ctx = 0.0;     // wavenumber of the Helmholtz kernels (sctl_amd_plan_set_ctx)
@@ -55,9 +66,11 @@ struct sctl_amd_plan_s {
   // refuse to launch once it differs.
   uint64_t generation = 0;
   sctl_amd::Item* d_items = nullptr;
+  sctl_amd::SplitChunk* d_split = nullptr;
+  int nsplit = 0;             // chunks cut into pieces
+  double* d_part = nullptr;   // their partial sums
   int64_t *d_trg_dsp = nullptr, *d_src_dsp = nullptr;
   int32_t *d_src_cnt = nullptr, *d_trg_cnt = nullptr;
-  int* d_counter = nullptr;
   double *d_xt = nullptr, *d_xs = nullptr, *d_xn = nullptr;
 
   // Near-field matrix layout (sctl_amd_plan_near_layout): per-block offsets
@@ -88,7 +101,7 @@ struct sctl_amd_plan_s {
     (void)hipGetDevice(&cur);
     if (cur != device) (void)hipSetDevice(device);
     free_near();
-    void* ptrs[] = {d_items, d_trg_dsp, d_src_dsp, d_src_cnt, d_trg_cnt, d_counter, d_xt, d_xs, d_xn};
+    void* ptrs[] = {d_items, d_split, d_part, d_trg_dsp, d_src_dsp, d_src_cnt, d_trg_cnt, d_xt, d_xs, d_xn};
     for (void* p : ptrs)
       if (p) (void)hipFree(p);
     if (cur >= 0 && cur != device) (void)hipSetDevice(cur);
