@@ -482,6 +482,256 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
   }
 }
 
+// ---- Laplace kernels: the far form on the matrix cores ---------------------
+// The far form's r^2 = |t'|^2 + |s'|^2 - 2 t'.s' (and the double layer's
+// f n.r = t'.nq - s'.nq) is a contraction over the three axes.  FP32 values are
+// cut into three bf16 parts (8 of the 24 mantissa bits each, by truncation, so
+// the parts' sum is exact), and a product of two such values is the sum of
+// eight products of parts (all but the last parts' product, 2^-32 of it): the
+// 8 k-slots that one lane group holds of v_mfma_f32_16x16x32_bf16.  Lane groups
+// 0-2 take the axes; group 3 takes |t'|^2 (three parts against ones), and
+// |s'|^2 comes in as the FP32 addend, one per row.  So one instruction forms
+// r^2 for 16 sources x 16 targets in FP32 accumulation: rms error 6.5e-8
+// relative where the FP32 FMA chain has 6.9e-8 (|t'| = 3H, 10^6 pairs).
+//
+// Cycles per 256 pairs of one SIMD on MI355X (8 waves, 2.4 GHz): 17 for the
+// instruction, 33 for four v_rsq_f32, 12 for four FMAs, 55 together; the
+// FP32 form needs 94.  Dense plan applies, 524288 x 524288 sphere and shell
+// (FP32 form -> this): Laplace FxU 46.5 -> 30.4 ms (9.0e12 pairs/s), DxU 70.7
+// -> 48.6 ms; 131072 x 131072 cube 3.36 -> 2.66 and 5.04 -> 3.98 ms.
+//
+// The matrix cores round sums toward minus infinity somewhere below 2^-29 of
+// their largest term: a bias of one sign, which 130 001 double layer terms of
+// random sign do not average out (error against 64 bits 2.0e-7 -> 6.8e-7).
+// The odd sources' nq and s'.nq are therefore staged with the opposite sign
+// and turned back by the FMA, so that the bias cancels between neighbours
+// (2.0e-7 again).  r^2's bias is multiplied by the density, whose sign varies.
+//
+// D's layout (lane l: target column l & 15, source rows 4 (l >> 4) + i) leaves
+// each lane with 4 sources of one target, whose densities and |s'|^2 are one
+// 16-byte LDS read each, shared by the wave's four target groups.
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+
+template <int KER> constexpr bool far_mfma() { return KER == LAP_FXU || KER == LAP_DXU; }
+// |t'|^2 below this takes the FP32 forms: the matrix cores may flush parts
+// below 2^-126, which are 2^-16 of |t'|^2.
+constexpr float MFMA_MIN_T = 0x1p-100f;
+
+struct Parts {
+  float a, b, c;  // each used by its upper 16 bits
+};
+__device__ __forceinline__ float upper(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+__device__ __forceinline__ Parts parts3(float x) {
+  const float r = x - upper(x);
+  return {x, r, r - upper(r)};
+}
+// The upper halves of two words: lo's in bits 0-15, hi's in bits 16-31.
+__device__ __forceinline__ uint32_t halves(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+// k-slots of a row (source) and of a column (target): slot by slot the eight products.
+__device__ __forceinline__ u32x4 row_slots(float x) {
+  const Parts p = parts3(x);
+  return u32x4{halves(p.a, p.a), halves(p.a, p.b), halves(p.b, p.b), halves(p.c, p.c)};
+}
+__device__ __forceinline__ u32x4 column_slots(float x) {
+  const Parts p = parts3(x);
+  const uint32_t ab = halves(p.a, p.b);
+  return u32x4{ab, halves(p.c, p.a), halves(p.b, p.c), ab};
+}
+__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                 0);
+}
+
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Mixed Eval of the Laplace kernels, 64 targets per wave.  Each tile's sources
+// are staged as k-slots; the classes are those of k_eval_mixed at one target
+// per lane (whole tile, else 64-source sub-tiles).  Far pairs are summed in the
+// matrix layout (at most 64 per FP32 sum), mid and near ones with one target
+// per lane from records that the wave stages for itself, NEAR_ST at a time.
+//
+// Four waves per SIMD are asked for: left alone the compiler takes 148
+// registers for the double layer (three waves), 58.6 instead of 48.6 ms at
+// 524288 x 524288; at six waves the single layer spills (32.1 against 30.4 ms).
+template <int KER, int NEWTON>
+__global__ void __launch_bounds__(WG, 4)
+k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __restrict__ tperm,
+                  const float4* __restrict__ packed, const double4* __restrict__ meta, const float4* __restrict__ sub,
+                  int64_t ntiles, int64_t tiles_per_split, double* __restrict__ out, int direct, double scale,
+                  double) {
+  constexpr int Q = MixLayout<KER>::Q, R = 4 * Q, NEAR_ST = 32, GROUPS = 4, CHUNKS = TILE / 16;
+  constexpr bool DXU = KER == LAP_DXU;
+  __shared__ u32x4 rs[TILE * 4];                  // -2 s' (group 3: ones against |t'|^2)
+  __shared__ u32x4 rn[DXU ? TILE * 4 : 1];        // nq (group 3: zeros)
+  __shared__ float sS[TILE], sq[DXU ? 1 : TILE];  // |s'|^2, density
+  __shared__ float sn[DXU ? TILE : 1];            // -s'.nq
+  __shared__ float4 near_all[(WG / 64) * NEAR_ST * Q];
+
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
+  float4* nst = near_all + (tid >> 6) * (NEAR_ST * Q);
+  const SplitCoord wg = split_coord((nt + WG - 1) / WG);
+  const int64_t tile_begin = wg.split * tiles_per_split;
+  const int64_t tile_end = tile_begin + tiles_per_split < ntiles ? tile_begin + tiles_per_split : ntiles;
+  const int64_t q0 = wg.block * WG + (tid & ~63);  // the wave's first target
+
+  // t64: this lane's target (q0 + lane); tg: axis g of the targets q0 + 16 m + c16
+  double t64[3], tg[GROUPS], accn = 0.0, accf[GROUPS];
+#pragma unroll
+  for (int k = 0; k < 3; k++) t64[k] = q0 + lane < nt ? xt[(q0 + lane) * 3 + k] : 0.0;
+#pragma unroll
+  for (int m = 0; m < GROUPS; m++) {
+    const int64_t q = q0 + 16 * m + c16;
+    tg[m] = q < nt && g < 3 ? xt[q * 3 + g] : 0.0;
+    accf[m] = 0.0;
+  }
+  // group 3's slots never change: this thread's row of chunk tid / 16
+  rs[(tid >> 4) * 64 + 48 + (tid & 15)] = u32x4{0x3f803f80u, 0x00003f80u, 0u, 0u};
+  if constexpr (DXU) rn[(tid >> 4) * 64 + 48 + (tid & 15)] = u32x4{0u, 0u, 0u, 0u};
+
+  for (int64_t tile = tile_begin; tile < tile_end; tile++) {
+    const float4* src = packed + tile * (TILE * Q);
+    float rec[R];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      if (DXU && q == 2) continue;  // the residuals: read only by near waves
+      const float4 v = src[tid * Q + q];
+      rec[4 * q] = v.x;
+      rec[4 * q + 1] = v.y;
+      rec[4 * q + 2] = v.z;
+      rec[4 * q + 3] = v.w;
+    }
+    const double4 m = meta[tile];
+    const double cg = g == 0 ? m.x : (g == 1 ? m.y : m.z);
+    __syncthreads();  // the previous tile's readers
+#pragma unroll
+    for (int k = 0; k < 3; k++) rs[(tid >> 4) * 64 + 16 * k + (tid & 15)] = row_slots(-2.0f * rec[k]);
+    sS[tid] = rec[3];
+    if constexpr (DXU) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) rn[(tid >> 4) * 64 + 16 * k + (tid & 15)] = row_slots(tid & 1 ? -rec[4 + k] : rec[4 + k]);
+      sn[tid] = tid & 1 ? -rec[7] : rec[7];
+    } else {
+      sq[tid] = rec[4];
+    }
+    __syncthreads();
+
+    const float th[3] = {(float)(t64[0] - m.x), (float)(t64[1] - m.y), (float)(t64[2] - m.z)};
+    const float T = fmad(th[2], th[2], fmad(th[1], th[1], th[0] * th[0]));
+    const float H2 = (float)m.w;
+    u32x4 col[GROUPS];
+#pragma unroll
+    for (int j = 0; j < GROUPS; j++) {
+      const float Tj = __shfl(T, 16 * j + c16, 64);
+      col[j] = column_slots(g < 3 ? (float)(tg[j] - cg) : Tj);
+    }
+    float pf[GROUPS], pn[1] = {0.0f};
+    double ptn = 0.0;
+#pragma unroll
+    for (int j = 0; j < GROUPS; j++) pf[j] = 0.0f;
+    auto far = [&](int ch0, auto count) {
+#pragma unroll 4
+      for (int ch = ch0; ch < ch0 + decltype(count)::value; ch++) {
+        const u32x4 a = rs[ch * 64 + lane];
+        const f32x4 S4 = *reinterpret_cast<const f32x4*>(sS + ch * 16 + 4 * g);
+        if constexpr (DXU) {
+          const u32x4 an = rn[ch * 64 + lane];
+          const f32x4 n4 = *reinterpret_cast<const f32x4*>(sn + ch * 16 + 4 * g);
+#pragma unroll
+          for (int j = 0; j < GROUPS; j++) {
+            const f32x4 r2 = mfma16(a, col[j], S4), rnq = mfma16(an, col[j], n4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const float z = rsq_deferred<NEWTON>(r2[i]);
+              pf[j] = fmad((i & 1 ? -rnq[i] : rnq[i]) * z, z * z, pf[j]);
+            }
+          }
+        } else {
+          const f32x4 f4 = *reinterpret_cast<const f32x4*>(sq + ch * 16 + 4 * g);
+#pragma unroll
+          for (int j = 0; j < GROUPS; j++) {
+            const f32x4 r2 = mfma16(a, col[j], S4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) pf[j] = fmad(rsq_deferred<NEWTON>(r2[i]), f4[i], pf[j]);
+          }
+        }
+      }
+    };
+    // Sub-tile sq0 / 64 with one target per lane: the mid form, or the near form.
+    auto by_lane = [&](int sq0, bool near) {
+      const float tl[3] = {(float)((t64[0] - m.x) - (double)th[0]), (float)((t64[1] - m.y) - (double)th[1]),
+                           (float)((t64[2] - m.z) - (double)th[2])};
+#pragma unroll 1
+      for (int s0 = sq0; s0 < sq0 + 64; s0 += NEAR_ST) {
+        wave_sync();
+        for (int i = lane; i < NEAR_ST * Q; i += 64) nst[i] = src[s0 * Q + i];
+        wave_sync();
+        const float* recs = reinterpret_cast<const float*>(nst);
+        if (near) {
+#pragma unroll 2
+          for (int i = 0; i < NEAR_ST; i++) mix_near<KER, NEWTON>(pn, th, tl, recs + i * R, 0.0f);
+        } else {
+#pragma unroll 4
+          for (int i = 0; i < NEAR_ST; i++) mix_mid<KER, NEWTON>(pn, th, recs + i * R);
+        }
+      }
+      ptn += (double)pn[0];
+      pn[0] = 0.0f;
+    };
+    const bool tiny = __builtin_amdgcn_ballot_w64(T < MFMA_MIN_T) != 0;
+    if (__builtin_amdgcn_ballot_w64(T < 9.0f * H2) == 0 && !tiny) {
+      far(0, std::integral_constant<int, CHUNKS>());
+    } else {
+      const float H = sqrtf(H2);
+#pragma unroll 1
+      for (int q = 0; q < TILE / 64; q++) {
+        const float4 b = sub[tile * (TILE / 64) + q];
+        const float h = sqrtf(b.w), X = sqrtf(T) + H;
+        const float dx = th[0] - b.x, dy = th[1] - b.y, dz = th[2] - b.z;
+        const float d2 = fmad(dz, dz, fmad(dy, dy, dx * dx));
+        const float ef = fmad(0.5f, X, h), em = fmad(1.0f / 3.0f, X, h);
+        if (__builtin_amdgcn_ballot_w64(d2 < ef * ef) == 0 && !tiny)
+          far(q * (CHUNKS / 4), std::integral_constant<int, CHUNKS / 4>());
+        else by_lane(q * 64, __builtin_amdgcn_ballot_w64(d2 < em * em) != 0);
+      }
+    }
+    bool bad = !__builtin_isfinite(ptn);
+#pragma unroll
+    for (int j = 0; j < GROUPS; j++) bad |= !__builtin_isfinite(pf[j]);
+    if (__builtin_amdgcn_ballot_w64(bad) != 0) {  // the whole tile in the near form
+#pragma unroll
+      for (int j = 0; j < GROUPS; j++) pf[j] = 0.0f;
+      ptn = 0.0;
+      for (int q = 0; q < TILE / 64; q++) by_lane(q * 64, true);
+    }
+    accn += ptn;
+#pragma unroll
+    for (int j = 0; j < GROUPS; j++) accf[j] += (double)pf[j];
+  }
+
+  // Target 16 j + c16's far sums: over the four lane groups, to the lane of that target.
+  double v = accn;
+#pragma unroll
+  for (int j = 0; j < GROUPS; j++) {
+    double f = accf[j];
+    f += __shfl_xor(f, 16, 64);
+    f += __shfl_xor(f, 32, 64);
+    if (g == j) v += f;
+  }
+  const int64_t q = q0 + lane;
+  if (q < nt) {
+    if (direct) out[tperm[q]] += v * scale;
+    else out[wg.split * nt + q] = v;
+  }
+}
+
 // v_trg[tperm[q]*K1+k] += scale * sum_y part[y][q*K1+k]; one lane quad per
 // element (sum_splits_quad).
 __global__ void __launch_bounds__(WG)
@@ -503,7 +753,11 @@ using PackFn = void (*)(const double*, const double*, const double*, int64_t, co
 constexpr int TPLS[3] = {1, 2, 4};
 int tpl_index(int tpl) { return tpl >= 4 ? 2 : (tpl >= 2 ? 1 : 0); }
 
+// Targets per lane of the mixed kernels (the matrix-core ones have one form).
+template <int KER> constexpr int mixed_max_tpl() { return far_mfma<KER>() ? 1 : max_tpl<KER>(); }
+
 template <int KER, int NEWTON> EvalMixFn mix_fn(int ti) {
+  if constexpr (far_mfma<KER>()) return k_eval_mixed_mfma<KER, NEWTON>;
   constexpr int MT = max_tpl<KER>();
   if (ti >= 2 && MT >= 4) return k_eval_mixed<KER, (MT >= 4 ? 4 : 1), NEWTON>;
   if (ti >= 1 && MT >= 2) return k_eval_mixed<KER, (MT >= 2 ? 2 : 1), NEWTON>;
@@ -522,7 +776,7 @@ int layout_q(int ker) {
   return with_kernel(ker, [](auto kc) { return MixLayout<decltype(kc)::value>::Q; });
 }
 int max_tpl_index(int ker) {
-  return with_kernel(ker, [](auto kc) { return tpl_index(max_tpl<decltype(kc)::value>()); });
+  return with_kernel(ker, [](auto kc) { return tpl_index(mixed_max_tpl<decltype(kc)::value>()); });
 }
 
 }  // namespace
