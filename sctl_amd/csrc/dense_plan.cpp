@@ -25,6 +25,7 @@ using namespace sctl_amd;
 
 struct sctl_amd_dense_plan_s {
   int kernel = 0, precision = SCTL_AMD_FP64, newton = 2, K0 = 1, K1 = 1, ND = 0, device = 0;
+  bool f64 = true;  // runs the FP64 kernels (mixed_runs_f64 for a mixed plan)
   int64_t nt = 0, ns = 0;
   double ctx = 0.0;
   DenseShape shape;
@@ -56,7 +57,7 @@ int dev_alloc(void** p, size_t bytes) {
 
 int dense_plan_apply_dev(sctl_amd_dense_plan_s* p, const double* v_src, double* v_trg, hipStream_t s) {
   if (p->nt == 0 || p->ns == 0) return SCTL_AMD_SUCCESS;
-  if (p->precision == SCTL_AMD_FP64)
+  if (p->f64)
     return f64_apply(p->kernel, p->newton, p->d_xt, p->nt, p->d_xs, p->d_xn, v_src, p->ns, v_trg, p->shape, p->ctx,
                      p->d_part, s);
   return mixed_apply(p->kernel, p->newton, p->geo, p->shape, p->d_xt, p->nt, p->d_tperm, p->d_xs, p->d_xn, v_src,
@@ -112,6 +113,7 @@ int sctl_amd_dense_plan_create(sctl_amd_dense_plan* out, int kernel, int precisi
   p->kernel = kernel;
   p->precision = precision;
   p->newton = precision == SCTL_AMD_FP64 ? newton_steps_f64(digits) : ((flags & SCTL_AMD_MIXED_NEWTON) ? 1 : 0);
+  p->f64 = precision == SCTL_AMD_FP64 || mixed_runs_f64(kernel, nt, ns);
   p->K0 = K0;
   p->K1 = K1;
   p->ND = ND;
@@ -132,7 +134,7 @@ int sctl_amd_dense_plan_create(sctl_amd_dense_plan* out, int kernel, int precisi
   if (!rc && ND) rc = copy(&p->d_xn, n_src, ns * 3);
   if (!rc && nt > 0 && ns > 0) {
     size_t part = 0;
-    if (precision == SCTL_AMD_FP64) {
+    if (p->f64) {
       rc = f64_part_bytes(kernel, nt, ns, p->shape, &part);
     } else {
       rc = mixed_geometry(kernel, nt, ns, p->shape, &p->geo);

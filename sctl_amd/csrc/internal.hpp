@@ -139,6 +139,11 @@ int f64_part_bytes(int ker, int64_t nt, int64_t ns, const DenseShape& shape, siz
 int f64_apply(int ker, int newton, const double* r_trg, int64_t nt, const double* r_src, const double* n_src,
               const double* v_src, int64_t ns, double* v_trg, const DenseShape& shape, double ctx, double* part,
               hipStream_t stream, size_t part_budget = PART_BUDGET);
+// Whether a mixed Eval of this size runs the FP64 kernels, with the rsqrt as
+// far refined as its own would be (the estimate, good to 2^-24, or one Newton
+// step with SCTL_AMD_MIXED_NEWTON): below a size the mixed path's orders, packing
+// and short tiles cost more than its cheaper pairs save.  mixed.hip.
+bool mixed_runs_f64(int ker, int64_t nt, int64_t ns);
 struct MixedGeometry {
   int ti = 0, Q = 0;
   int64_t tb = 0, ntiles = 0, nsplit = 1, tps = 0;

@@ -781,6 +781,26 @@ int max_tpl_index(int ker) {
 
 }  // namespace
 
+// Measured on MI355X, uniform cubes, us, FP64 kernels with the rsqrt estimate /
+// mixed path:
+//                    dense plan apply                     Eval
+//   Laplace FxU      8000^2 34 / 39, 12000^2 59 / 62      8000^2 36 / 67, 17000^2 109 / 125
+//   Laplace DxU      8000^2 44 / 59, 12000^2 83 / 92      8000^2 47 / 87, 17000^2 160 / 166
+//   Stokes FxU       5000^2 30 / 35, 6500^2 44 / 43       5000^2 33 / 63, 8000^2 64 / 80
+//   Helmholtz FxU    6500^2 104 / 118, 8000^2 147 / 141   8000^2 150 / 169
+//   BiotSavart FxdU  2000 x 3000 22 / 39, 5000^2 53 / 50  5000^2 56 / 77
+// The line is where an apply, which keeps its orders, is even, so that a plan
+// and an Eval of one size run the same kernels (their results are equal bit
+// for bit).  The estimate is good to 2^-24 and all else is FP64: errors are a
+// tenth to a half of the mixed path's.
+bool mixed_runs_f64(int ker, int64_t nt, int64_t ns) {
+  int K0, K1, ND;
+  kernel_dims(ker, &K0, &K1, &ND);
+  const double pairs = (double)nt * (double)ns;
+  if (ker == LAP_FXU || ker == LAP_DXU) return pairs <= 1.5e8;
+  return pairs <= (needs_ctx(ker) ? 6e7 : (K1 > 4 ? 2e7 : 4.2e7));
+}
+
 // Launch geometry of one mixed Eval: target blocks and the source splits.
 // Split the sources over gridDim.y when the target blocks cannot fill the
 // device (>= 8 workgroups per CU, each split >= 4 tiles), and so that no
@@ -915,6 +935,8 @@ int launch_eval_mixed(int ker, int newton, const double* r_trg, int64_t nt, cons
                       const double* n_src, const double* v_src, int64_t ns, double* v_trg, const DenseShape& shape,
                       double ctx, hipStream_t stream) {
   if (nt <= 0 || ns <= 0) return SCTL_AMD_SUCCESS;
+  if (mixed_runs_f64(ker, nt, ns))
+    return launch_eval_f64(ker, newton, r_trg, nt, r_src, n_src, v_src, ns, v_trg, shape, ctx, stream);
   MixedGeometry g;
   SCTL_TRY(mixed_geometry(ker, nt, ns, shape, &g));
   // One allocation for the call: orders, packed tiles, the sorts' workspace

@@ -72,7 +72,7 @@ int sctl_amd_eval_noalloc(int kernel, const double* ctx, int precision, int digi
       precision == SCTL_AMD_FP64 ? newton_steps_f64(digits) : ((flags & SCTL_AMD_MIXED_NEWTON) ? 1 : 0);
   const DenseShape shape = pick_dense_shape(kernel, precision, newton, nt, ns);
   const double mu = eval_ctx_value(kernel, ctx);
-  if (precision == SCTL_AMD_FP64) {
+  if (precision == SCTL_AMD_FP64 || mixed_runs_f64(kernel, nt, ns)) {
     // Split partial sums only; with the whole array as their budget.
     return f64_apply(kernel, newton, r_trg, nt, r_src, n_src, v_src, ns, v_trg, shape, mu,
                      reinterpret_cast<double*>(w), s, NOALLOC_SCRATCH_BYTES);
