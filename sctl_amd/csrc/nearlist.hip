@@ -14,48 +14,60 @@
 //
 // The reference finds candidates through a Morton tree of the nodes.  Here:
 //   1. targets get 63-bit Morton keys over the reference's bounding cube
-//      (all points, grown by 5 % per side, :104-154) and are radix sorted;
-//   2. one wave per element (its nodes in the lanes) takes the bounding box
-//      of its nodes grown by the largest radius, picks the finest Morton
-//      depth at which that box spans at most 64 cells, finds each cell's
-//      targets by binary search in the sorted keys, queues the candidates
-//      inside the grown box and tests them 64 at a time exactly against the
-//      element's nodes (one ballot per candidate and 64 nodes, each node
-//      chunk loaded once per batch, first hit wins);
-//   3. a first pass counts the candidates inside the grown boxes only (an
-//      upper bound of the pairs, without the node tests), the second tests
-//      them and appends the (element, target) keys of the near ones through
-//      an atomic counter; the keys are radix sorted (so the list does not
-//      depend on the order of the appends), each element's range is found
-//      by binary search, and a second sort by (target, pair) gives the
-//      scatter index.
-// Each element is one workgroup of 4 waves that take turns over its
-// 64-candidate groups; elements are launched largest first.
+//      (all points, grown by 5 % per side, :104-154), are radix sorted and
+//      copied into that order;
+//   2. one workgroup per element takes the bounding boxes of its nodes, 64 at a
+//      time, and of all of them grown by the largest radius, picks the finest
+//      Morton depth at which that box spans at most 64 cells, finds the cells'
+//      targets by binary search in the sorted keys (one cell per lane), and
+//      its four waves take the cells' targets 64 at a time as one list: those
+//      inside the grown box are queued and tested in batches (k_nl_elements);
+//   3. the near ones go out as (element, target) keys, gathered in LDS and
+//      appended through an atomic counter once per element (one atomic per
+//      batch of 64 tests was most of this kernel's time: a single address
+//      takes ~75 per microsecond); the buffer holds 24 pairs per target, and a
+//      list that has more is filled again into one of the size then known;
+//   4. the keys are radix sorted (so the list does not depend on the order of
+//      the appends), in 32 bits where an element and a target number fit; each
+//      element's range is found by binary search, and a stable sort of the
+//      pairs by target gives the scatter index.
 // Every target within a node's radius lies in the grown box, hence in one of
 // the cells (the cell range is computed with the same quantisation as the
 // target keys), so the list is exact.
+//
+// Build, get and destroy for 2048 elements (0.9 M nodes) and 500 009 targets on
+// MI355X: 5.76 -> 1.59 ms; the passes over the elements, two of them before
+// (candidates counted, then tested), 1.78 -> 0.36 ms, the sorts of the pairs 0.38
+// -> 0.19.  All results live in one buffer of the library's pool: seven
+// hipMalloc and hipFree each, and their waits, were half of the time.
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/device/device_scan.hpp>
 
 #include <algorithm>
 #include <string>
 
 #include "internal.hpp"
+#include "wave.hpp"
 
 struct sctl_amd_near_list_s {
   int device = 0;
   int64_t ntrg = 0, nelem = 0, n_near = 0;
   bool has_normal = false;
+  char* buf = nullptr;         // all results, from the library's pool
+  size_t counts = 0, counts_bytes = 0;  // the four count and offset arrays within buf, adjacent
   double *d_xtn = nullptr, *d_xntn = nullptr;
   int64_t *d_ecnt = nullptr, *d_edsp = nullptr, *d_scatter = nullptr, *d_tcnt = nullptr, *d_tdsp = nullptr;
+  hipEvent_t last = nullptr;  // the latest read of the results, on whichever stream
   ~sctl_amd_near_list_s() {
     int cur = -1;
     (void)hipGetDevice(&cur);
     if (cur != device) (void)hipSetDevice(device);
-    void* ptrs[] = {d_xtn, d_xntn, d_ecnt, d_edsp, d_scatter, d_tcnt, d_tdsp};
-    for (void* p : ptrs)
-      if (p) (void)hipFree(p);
+    if (buf) {
+      // Freed in this thread's stream after the last read.
+      if (last) (void)hipStreamWaitEvent(hipStreamPerThread, last, 0);
+      (void)hipFreeAsync(buf, hipStreamPerThread);
+    }
+    if (last) (void)hipEventDestroy(last);
     if (cur >= 0 && cur != device) (void)hipSetDevice(cur);
   }
 };
@@ -118,18 +130,6 @@ __device__ __forceinline__ int64_t lower_bound_u64(const uint64_t* __restrict__ 
   return lo;
 }
 
-__device__ __forceinline__ double wave_min(double v) {
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) v = fmin(v, __shfl_xor(v, m, 64));
-  return v;
-}
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) v = fmax(v, __shfl_xor(v, m, 64));
-  return v;
-}
-
-
 // |d|^2 rounded as node_dist2 sums it (boundary_integral.txx:72-79), without
 // fused multiply-adds, so the radius test matches the reference's bit for bit.
 __device__ __forceinline__ double dist2(double dx, double dy, double dz) {
@@ -137,13 +137,14 @@ __device__ __forceinline__ double dist2(double dx, double dy, double dz) {
   return (dx * dx + dy * dy) + dz * dz;
 }
 
-constexpr int NODE_REGS = 4;  // node chunks of 64 kept in registers (larger elements load the rest per batch)
-constexpr int QCAP = 128;     // per-wave queue of candidates inside the grown box
+constexpr int QCAP = 128;          // per-wave queue of candidates inside the grown box
 constexpr int NWAVE = NL_WG / 64;  // waves sharing one element's candidates
+constexpr int MAX_BOXES = 64;      // node boxes of an element: one per 64 nodes up to 4096 nodes, larger ones beyond
+constexpr int HITS = 512;          // near targets a wave gathers before it appends them
 
 struct Cand {
   double x, y, z;
-  uint64_t t;
+  uint32_t t;
 };
 
 __device__ __forceinline__ void wave_sync() {
@@ -151,234 +152,281 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+__device__ __forceinline__ int lanes_below(uint64_t mask) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+}
+__device__ __forceinline__ uint64_t uniform64(uint64_t v, int lane) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+}
 
-// One workgroup per element.  FILL = false: counts[e * NWAVE + w] = the
-// candidates inside the element's grown box that wave w fetched (no node
-// tests); FILL = true: appends (e << 32 | t) of each near target at
-// out[atomicAdd(counter)], cap entries at most.
-// Lanes hold the element's nodes (64 per chunk, the first NODE_REGS chunks in
-// registers).  Candidate targets are fetched 64 at a time; those inside the
-// grown box are appended to a per-wave LDS queue, and every 64 queued
-// candidates are tested as a batch: node chunk by node chunk (each chunk
-// loaded once per batch), each undecided candidate broadcast from LDS and
-// tested against the chunk's 64 nodes with one ballot, decided at its first
-// hit.
-template <bool FILL>
+// One workgroup per element: appends the key (e << tbits | t) of each near
+// target at out[atomicAdd(counter)], cap entries at most (the counter goes on
+// counting).
+//
+// A candidate inside the grown box is near when it is within some node's
+// radius.  Each batch of 64 is decided in three steps, cheapest first:
+//   lane per candidate   the node boxes within reach: a box whose nearest point
+//                        is not within its largest radius holds no node that
+//                        is (dist2 is monotone in each |difference|, so this
+//                        is exact).  No box: not near.
+//   wave per candidate   64 of the element's nodes, spread over it, one per
+//                        lane, one ballot.  Radii of several node spacings
+//                        decide nearly every near candidate here.
+//   wave per candidate   box by box, those left with the box within reach, 64
+//                        nodes a ballot.
+// Testing every candidate against the element's nodes chunk by chunk took ~8
+// ballots each.
+template <class Key>
 __global__ void __launch_bounds__(NL_WG)
-k_nl_elements(const uint32_t* __restrict__ eorder, const int64_t* __restrict__ ecnt,
-              const int64_t* __restrict__ edsp, int64_t nsrc, const double* __restrict__ xs,
-              const double* __restrict__ rad, int64_t nt, const double* __restrict__ xt,
-              const uint64_t* __restrict__ skeys, const uint32_t* __restrict__ sidx, const double* __restrict__ box,
-              int64_t* __restrict__ counts, unsigned long long* __restrict__ counter, int64_t cap,
-              uint64_t* __restrict__ out) {
+k_nl_elements(const int64_t* __restrict__ ecnt, const int64_t* __restrict__ edsp, int64_t nsrc,
+              const double* __restrict__ xs, const double* __restrict__ rad, int64_t nt,
+              const double* __restrict__ xsorted, const uint64_t* __restrict__ skeys,
+              const uint32_t* __restrict__ sidx, const double* __restrict__ cube, int tbits,
+              unsigned long long* __restrict__ counter, int64_t cap, Key* __restrict__ out) {
   __shared__ Cand queue_all[NWAVE][QCAP];
+  __shared__ uint32_t hits_all[NWAVE][HITS];
+  __shared__ double box[7][MAX_BOXES];  // lo, hi, largest radius^2
+  __shared__ int64_t cell_first[MAX_CELLS];
+  __shared__ uint64_t cell_before[MAX_CELLS + 1];
+  __shared__ int nhits[NWAVE];
+  __shared__ unsigned long long out_base;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   Cand* queue = queue_all[w];
-  const double x0[3] = {box[0], box[1], box[2]}, scale = box[3];
-  {
-    const int64_t e = eorder[blockIdx.x];
-    const int64_t s0 = edsp[e], sc = ecnt[e];
-    int64_t count = 0;
-    if (s0 >= 0 && sc > 0 && s0 <= nsrc && sc <= nsrc - s0 && nt > 0) {
-      const int nch = (int)((sc + 63) / 64);
-      // nodes of the first chunks in registers; r2 = -1 marks a lane without a node
-      double nx[NODE_REGS], ny[NODE_REGS], nz[NODE_REGS], nr2[NODE_REGS];
-      double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY}, rmax = 0;
-#pragma unroll
-      for (int c = 0; c < NODE_REGS; c++) {
-        nx[c] = ny[c] = nz[c] = 0.0;
-        nr2[c] = -1.0;
-      }
-      for (int64_t s = lane; s < sc; s += 64) {
-        const double x = xs[(s0 + s) * 3 + 0], y = xs[(s0 + s) * 3 + 1], z = xs[(s0 + s) * 3 + 2];
-        const double r = rad[s0 + s];
-        lo[0] = fmin(lo[0], x);
-        lo[1] = fmin(lo[1], y);
-        lo[2] = fmin(lo[2], z);
-        hi[0] = fmax(hi[0], x);
-        hi[1] = fmax(hi[1], y);
-        hi[2] = fmax(hi[2], z);
-        rmax = fmax(rmax, fabs(r));
-        const int c = (int)(s >> 6);
-#pragma unroll
-        for (int k = 0; k < NODE_REGS; k++)
-          if (c == k) {
-            nx[k] = x;
-            ny[k] = y;
-            nz[k] = z;
-            nr2[k] = r * r;
-          }
-      }
+  uint32_t* hits = hits_all[w];
+  const int64_t e = blockIdx.x;
+  const int64_t s0 = edsp[e], sc = ecnt[e];
+  if (!(s0 >= 0 && sc > 0 && s0 <= nsrc && sc <= nsrc - s0 && nt > 0)) return;  // the whole workgroup
+
+  // Node boxes: per_box nodes each, a whole number of 64-node chunks.
+  const int64_t nch = (sc + 63) / 64, per_box = (nch + MAX_BOXES - 1) / MAX_BOXES * 64;
+  const int nbox = (int)((sc + per_box - 1) / per_box);
+  for (int b = w; b < nbox; b += NWAVE) {
+    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY}, rmax = 0;
+    const int64_t end = (b + 1) * per_box < sc ? (b + 1) * per_box : sc;
+    for (int64_t s = b * per_box + lane; s < end; s += 64) {
 #pragma unroll
       for (int k = 0; k < 3; k++) {
-        lo[k] = wave_min(lo[k]);
-        hi[k] = wave_max(hi[k]);
+        const double x = xs[(s0 + s) * 3 + k];
+        lo[k] = fmin(lo[k], x);
+        hi[k] = fmax(hi[k], x);
       }
-      rmax = wave_max(rmax);
+      rmax = fmax(rmax, fabs(rad[s0 + s]));
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      lo[k] = sctl_amd::wave_min(lo[k]);
+      hi[k] = sctl_amd::wave_max(hi[k]);
+    }
+    rmax = sctl_amd::wave_max(rmax);
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        box[k][b] = lo[k];
+        box[3 + k][b] = hi[k];
+      }
+      box[6][b] = rmax * rmax;
+    }
+  }
+  __syncthreads();
+  // The element's own box and largest radius.
+  double glo[3], ghi[3];
+  double rmax = sctl_amd::wave_max(lane < nbox ? box[6][lane] : 0.0);
+  if (!(rmax > 0)) return;  // uniform over the workgroup
+  rmax = sqrt(rmax);
+  const double grow = rmax * (1.0 + 1e-9);  // a margin above the rounding of the additions and of sqrt(r^2)
+  uint32_t qlo[3], qhi[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const double lo = sctl_amd::wave_min(lane < nbox ? box[k][lane] : INFINITY);
+    const double hi = sctl_amd::wave_max(lane < nbox ? box[3 + k][lane] : -INFINITY);
+    glo[k] = lo - grow - 1e-14 * fabs(lo);
+    ghi[k] = hi + grow + 1e-14 * fabs(hi);
+    qlo[k] = quant(glo[k], cube[k], cube[3]);
+    qhi[k] = quant(ghi[k], cube[k], cube[3]);
+  }
+  int shift = 0;
+  int64_t cells = 1;
+  for (int d = MAX_DEPTH; d >= 0; d--) {
+    shift = MAX_DEPTH - d;
+    cells = 1;
+#pragma unroll
+    for (int k = 0; k < 3; k++) cells *= (int64_t)(qhi[k] >> shift) - (qlo[k] >> shift) + 1;
+    if (cells <= MAX_CELLS) break;
+  }
+  // Targets of the cells, one cell per lane of wave 0: two binary searches.
+  if (w == 0) {
+    int64_t i0 = 0, i1 = 0;
+    if (lane < cells) {
+      const uint32_t nx = (qhi[0] >> shift) - (qlo[0] >> shift) + 1, ny = (qhi[1] >> shift) - (qlo[1] >> shift) + 1;
+      const uint32_t c = lane, bx = (qlo[0] >> shift) + c % nx, by = (qlo[1] >> shift) + c / nx % ny,
+                     bz = (qlo[2] >> shift) + c / nx / ny;
+      const uint64_t klo = interleave(bx, by, bz) << (3 * shift);
+      i0 = lower_bound_u64(skeys, nt, klo);
+      i1 = lower_bound_u64(skeys, nt, klo + (1ULL << (3 * shift)));
+    }
+    uint64_t inc = (uint64_t)(i1 - i0);
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+      const uint64_t o = __shfl_up(inc, m, 64);
+      if (lane >= m) inc += o;
+    }
+    cell_first[lane] = i0;
+    cell_before[lane + 1] = inc;
+    if (lane == 0) cell_before[0] = 0;
+  }
+  // Sample nodes, one per lane; r2 = -1 marks a lane without one.
+  double px = 0, py = 0, pz = 0, pr2 = -1.0;
+  {
+    const int64_t s = sc >= 64 ? (2 * lane + 1) * sc / 128 : lane;
+    if (s < sc) {
+      px = xs[(s0 + s) * 3 + 0];
+      py = xs[(s0 + s) * 3 + 1];
+      pz = xs[(s0 + s) * 3 + 2];
+      const double r = rad[s0 + s];
+      pr2 = r * r;
+    }
+  }
+  __syncthreads();
 
-      // Tests queue entries [0, n) (n <= 64); returns the mask of near ones
-      // and, with FILL, writes them.
-      auto batch = [&](int n) {
-        uint64_t rem = n >= 64 ? ~0ULL : ((1ULL << n) - 1);
-        uint64_t nearm = 0;
-        for (int k = 0; k < nch && rem; k++) {
-          double bx = 0, by = 0, bz = 0, br2 = -1.0;
-          if (k < NODE_REGS) {
+  int nh = 0;  // near targets gathered by this wave (uniform)
+  auto flush = [&]() {
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd(counter, (unsigned long long)nh);
+    base = uniform64(base, 0);
+    for (int i = lane; i < nh; i += 64)
+      if ((int64_t)base + i < cap) out[base + i] = ((Key)e << tbits) | (Key)hits[i];
+    nh = 0;
+  };
+  // Which of the queue entries in `mask` are within a node's radius, one node
+  // per lane; four at a time, so that their LDS reads and ballots overlap.
+  auto tested = [&](uint64_t mask, double x, double y, double z, double r2) -> uint64_t {
+    uint64_t hit = 0;
+    while (mask) {
+      int j[4];
+      double d2[4];
 #pragma unroll
-            for (int kk = 0; kk < NODE_REGS; kk++)
-              if (kk == k) {
-                bx = nx[kk];
-                by = ny[kk];
-                bz = nz[kk];
-                br2 = nr2[kk];
-              }
-          } else {
-            const int64_t s = (int64_t)k * 64 + lane;
-            if (s < sc) {
-              bx = xs[(s0 + s) * 3 + 0];
-              by = xs[(s0 + s) * 3 + 1];
-              bz = xs[(s0 + s) * 3 + 2];
-              const double r = rad[s0 + s];
-              br2 = r * r;
-            }
-          }
-          uint64_t todo = rem;
-          while (todo) {
-            const int j = __builtin_ctzll(todo);
-            todo &= todo - 1;
-            const double cx = queue[j].x, cy = queue[j].y, cz = queue[j].z;
-            if (__builtin_amdgcn_ballot_w64(dist2(bx - cx, by - cy, bz - cz) < br2) != 0) {
-              nearm |= 1ULL << j;
-              rem &= ~(1ULL << j);
-            }
-          }
-        }
-        if constexpr (FILL) {
-          const int nn = __builtin_popcountll(nearm);
-          if (nn) {
-            unsigned long long base = 0;
-            if (lane == 0) base = atomicAdd(counter, (unsigned long long)nn);
-            base = __shfl(base, 0, 64);
-            if ((nearm >> lane) & 1ULL) {
-              const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(nearm >> 32),
-                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)nearm, 0));
-              const int64_t pos = (int64_t)base + below;
-              if (pos < cap) out[pos] = ((uint64_t)e << 32) | queue[lane].t;
-            }
-          }
-        }
-      };
-
-      if (rmax > 0) {
-        // Grown box, with a margin above the rounding of the two additions.
-        const double grow = rmax * (1.0 + 1e-9);
-        double glo[3], ghi[3];
-        uint32_t qlo[3], qhi[3];
+      for (int k = 0; k < 4; k++) {  // fewer than four left: the last one again
+        j[k] = mask ? __builtin_ctzll(mask) : j[k - 1];
+        mask &= mask - 1;
+      }
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-          glo[k] = lo[k] - grow - 1e-14 * fabs(lo[k]);
-          ghi[k] = hi[k] + grow + 1e-14 * fabs(hi[k]);
-          qlo[k] = quant(glo[k], x0[k], scale);
-          qhi[k] = quant(ghi[k], x0[k], scale);
-        }
-        int shift = 0;
-        for (int d = MAX_DEPTH; d >= 0; d--) {
-          shift = MAX_DEPTH - d;
-          int64_t cells = 1;
+      for (int k = 0; k < 4; k++) d2[k] = dist2(x - queue[j[k]].x, y - queue[j[k]].y, z - queue[j[k]].z);
 #pragma unroll
-          for (int k = 0; k < 3; k++) cells *= (int64_t)(qhi[k] >> shift) - (qlo[k] >> shift) + 1;
-          if (cells <= MAX_CELLS) break;
+      for (int k = 0; k < 4; k++)
+        if (__builtin_amdgcn_ballot_w64(d2[k] < r2) != 0) hit |= 1ULL << j[k];
+    }
+    return hit;
+  };
+  // Tests queue entries [0, n) (n <= 64).
+  auto batch = [&](int n) {
+    const Cand q = queue[lane < n ? lane : 0];
+    uint64_t reach = 0;
+    for (int b = 0; b < nbox; b++) {
+      const double dx = fmax(fmax(box[0][b] - q.x, q.x - box[3][b]), 0.0);
+      const double dy = fmax(fmax(box[1][b] - q.y, q.y - box[4][b]), 0.0);
+      const double dz = fmax(fmax(box[2][b] - q.z, q.z - box[5][b]), 0.0);
+      if (dist2(dx, dy, dz) < box[6][b]) reach |= 1ULL << b;
+    }
+    if (lane >= n) reach = 0;
+    uint64_t rem = __builtin_amdgcn_ballot_w64(reach != 0), nearm = 0;
+    nearm = tested(rem, px, py, pz, pr2);
+    rem &= ~nearm;
+    if (sc > 64 && rem) {  // the samples were not all nodes
+      for (int b = 0; b < nbox && rem; b++) {
+        const uint64_t mine = __builtin_amdgcn_ballot_w64((reach >> b) & 1ULL) & rem;
+        if (!mine) continue;
+        const int64_t first = b * per_box, end = first + per_box < sc ? first + per_box : sc;
+        uint64_t left = mine;
+        for (int64_t s1 = first; s1 < end && left; s1 += 64) {
+          const int64_t s = s1 + lane < end ? s1 + lane : end - 1;  // the last node again past the end
+          const double r = rad[s0 + s];
+          left &= ~tested(left, xs[(s0 + s) * 3 + 0], xs[(s0 + s) * 3 + 1], xs[(s0 + s) * 3 + 2], r * r);
         }
-        const uint64_t span = 1ULL << (3 * shift);
-        int qn = 0;        // queued candidates (< 64 between batches)
-        int64_t group = 0; // 64-candidate groups fetched so far; wave w takes every NWAVE-th
-        for (uint32_t bz = qlo[2] >> shift; bz <= (qhi[2] >> shift); bz++)
-          for (uint32_t by = qlo[1] >> shift; by <= (qhi[1] >> shift); by++)
-            for (uint32_t bx = qlo[0] >> shift; bx <= (qhi[0] >> shift); bx++) {
-              const uint64_t klo = interleave(bx, by, bz) << (3 * shift);
-              const int64_t i0 = lower_bound_u64(skeys, nt, klo);
-              const int64_t i1 = lower_bound_u64(skeys, nt, klo + span);
-              for (int64_t c0 = i0; c0 < i1; c0 += 64) {
-                if ((group++ % NWAVE) != w) continue;
-                const int64_t c = c0 + lane;
-                bool inside = false;
-                double mx = 0, my = 0, mz = 0;
-                uint64_t mt = 0;
-                if (c < i1) {
-                  mt = sidx[c];
-                  mx = xt[mt * 3 + 0];
-                  my = xt[mt * 3 + 1];
-                  mz = xt[mt * 3 + 2];
-                  inside = mx >= glo[0] && mx <= ghi[0] && my >= glo[1] && my <= ghi[1] && mz >= glo[2] &&
-                           mz <= ghi[2];
-                }
-                const uint64_t in = __builtin_amdgcn_ballot_w64(inside);
-                if constexpr (!FILL) {
-                  count += __builtin_popcountll(in);
-                  continue;
-                }
-                if (inside) {
-                  const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(in >> 32),
-                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)in, 0));
-                  Cand& q = queue[qn + below];  // qn < 64, so qn + below < QCAP
-                  q.x = mx;
-                  q.y = my;
-                  q.z = mz;
-                  q.t = mt;
-                }
-                qn += __builtin_popcountll(in);
-                wave_sync();
-                if (qn >= 64) {
-                  batch(64);
-                  wave_sync();
-                  const int from = 64 + (lane < qn - 64 ? lane : 0);
-                  const double rx = queue[from].x, ry = queue[from].y, rz = queue[from].z;
-                  const uint64_t rt = queue[from].t;
-                  wave_sync();
-                  if (lane < qn - 64) {
-                    queue[lane].x = rx;
-                    queue[lane].y = ry;
-                    queue[lane].z = rz;
-                    queue[lane].t = rt;
-                  }
-                  qn -= 64;
-                  wave_sync();
-                }
-              }
-            }
-        if (qn > 0) batch(qn);
-        wave_sync();
+        nearm |= mine & ~left;
+        rem &= ~(mine & ~left);
       }
     }
-    if constexpr (!FILL) {
-      if (lane == 0) counts[e * NWAVE + w] = count;
+    if (nh + 64 > HITS) {
+      wave_sync();
+      flush();
     }
+    if ((nearm >> lane) & 1ULL) hits[nh + lanes_below(nearm)] = q.t;
+    nh += __builtin_popcountll(nearm);
+    wave_sync();
+  };
+
+  const uint64_t total = cell_before[MAX_CELLS];
+  int qn = 0;  // queued candidates (< 64 between batches)
+  for (uint64_t base = (uint64_t)w * 64; base < total; base += NL_WG) {
+    const uint64_t c = base + lane;
+    bool inside = false;
+    Cand v{0, 0, 0, 0};
+    if (c < total) {
+      int cell = 0;  // the cell of the c-th target: the last with cell_before <= c
+#pragma unroll
+      for (int step = MAX_CELLS / 2; step > 0; step >>= 1)
+        if (cell_before[cell + step] <= c) cell += step;
+      const int64_t i = cell_first[cell] + (int64_t)(c - cell_before[cell]);
+      v.x = xsorted[i * 3 + 0];
+      v.y = xsorted[i * 3 + 1];
+      v.z = xsorted[i * 3 + 2];
+      v.t = sidx[i];
+      inside = v.x >= glo[0] && v.x <= ghi[0] && v.y >= glo[1] && v.y <= ghi[1] && v.z >= glo[2] && v.z <= ghi[2];
+    }
+    const uint64_t in = __builtin_amdgcn_ballot_w64(inside);
+    if (inside) queue[qn + lanes_below(in)] = v;  // qn < 64, so the entry is below QCAP
+    qn += __builtin_popcountll(in);
+    wave_sync();
+    if (qn >= 64) {
+      batch(64);
+      const Cand rest = queue[64 + (lane < qn - 64 ? lane : 0)];
+      wave_sync();
+      if (lane < qn - 64) queue[lane] = rest;
+      qn -= 64;
+      wave_sync();
+    }
+  }
+  if (qn > 0) batch(qn);
+  // What is left of the four waves' hits goes out together.
+  if (lane == 0) nhits[w] = nh;
+  __syncthreads();
+  int before = 0, all = 0;
+#pragma unroll
+  for (int k = 0; k < NWAVE; k++) {
+    before += k < w ? nhits[k] : 0;
+    all += nhits[k];
+  }
+  if (threadIdx.x == 0 && all) out_base = atomicAdd(counter, (unsigned long long)all);
+  __syncthreads();
+  for (int i = lane; i < nh; i += 64) {
+    const int64_t pos = (int64_t)out_base + before + i;
+    if (pos < cap) out[pos] = ((Key)e << tbits) | (Key)hits[i];
   }
 }
 
 // near_elem_dsp[e] / near_elem_cnt[e]: the range of element e in the sorted
-// keys (e << 32 | t), found by binary search (dsp = the pairs of the
+// keys (e << tbits | t), found by binary search (dsp = the pairs of the
 // elements before e, also for an element without pairs).
+template <class Key>
 __global__ void __launch_bounds__(NL_WG)
-k_nl_elem_ranges(int64_t nelem, const uint64_t* __restrict__ keys, int64_t n, int64_t* __restrict__ ecnt_out,
+k_nl_elem_ranges(int64_t nelem, const Key* __restrict__ keys, int64_t n, int tbits, int64_t* __restrict__ ecnt_out,
                  int64_t* __restrict__ edsp_out) {
   const int64_t e = (int64_t)blockIdx.x * NL_WG + threadIdx.x;
   if (e >= nelem) return;
-  const int64_t lo = lower_bound_u64(keys, n, (uint64_t)e << 32);
-  const int64_t hi = lower_bound_u64(keys, n, (uint64_t)(e + 1) << 32);
-  ecnt_out[e] = hi - lo;
-  edsp_out[e] = lo;
-}
-
-// Elements ordered by node count, largest first (the order only schedules).
-__global__ void __launch_bounds__(NL_WG)
-k_nl_order_keys(int64_t nelem, const int64_t* __restrict__ ecnt, uint32_t* __restrict__ keys,
-                uint32_t* __restrict__ idx) {
-  const int64_t e = (int64_t)blockIdx.x * NL_WG + threadIdx.x;
-  if (e >= nelem) return;
-  const int64_t c = ecnt[e];
-  keys[e] = 0xffffffffu - (uint32_t)(c < 0 ? 0 : (c > 0xffffffffLL ? 0xffffffffLL : c));
-  idx[e] = (uint32_t)e;
+  int64_t at[2];
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    int64_t lo = 0, hi = n;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if ((int64_t)(keys[mid] >> tbits) < e + k) lo = mid + 1;
+      else hi = mid;
+    }
+    at[k] = lo;
+  }
+  ecnt_out[e] = at[1] - at[0];
+  edsp_out[e] = at[0];
 }
 
 __global__ void __launch_bounds__(NL_WG) k_nl_zero(int64_t* __restrict__ a, int64_t n) {
@@ -386,45 +434,71 @@ __global__ void __launch_bounds__(NL_WG) k_nl_zero(int64_t* __restrict__ a, int6
   if (i < n) a[i] = 0;
 }
 
-// Pair i (element-major): gather the target's coordinates / normal, count it
-// for its target, and form the (target, pair) key of the target-major sort.
+// The targets in the order of their keys.
+__global__ void __launch_bounds__(NL_WG) k_nl_gather(const double* __restrict__ xt, int64_t nt,
+                                                     const uint32_t* __restrict__ sidx, double* __restrict__ xsorted) {
+  const int64_t i = (int64_t)blockIdx.x * NL_WG + threadIdx.x;
+  if (i >= nt) return;
+  const int64_t t = sidx[i];
+#pragma unroll
+  for (int k = 0; k < 3; k++) xsorted[i * 3 + k] = xt[t * 3 + k];
+}
+
+// Pair i (element-major): gather the target's coordinates / normal, and its
+// key (the target) and value (the pair) for the target-major sort.
+template <class Key>
 __global__ void __launch_bounds__(NL_WG)
-k_nl_unpack(int64_t n, const uint64_t* __restrict__ pairs, const double* __restrict__ xt,
+k_nl_unpack(int64_t n, const Key* __restrict__ pairs, int tbits, const double* __restrict__ xt,
             const double* __restrict__ xn, double* __restrict__ xtn, double* __restrict__ xntn,
-            unsigned long long* __restrict__ tcnt, uint64_t* __restrict__ key2) {
+            uint32_t* __restrict__ trg, uint32_t* __restrict__ pair) {
   const int64_t i = (int64_t)blockIdx.x * NL_WG + threadIdx.x;
   if (i >= n) return;
-  const uint64_t t = pairs[i] & 0xffffffffULL;
+  const uint64_t t = (uint64_t)pairs[i] & ((1ULL << tbits) - 1);
 #pragma unroll
   for (int k = 0; k < 3; k++) xtn[i * 3 + k] = xt[t * 3 + k];
   if (xn) {
 #pragma unroll
     for (int k = 0; k < 3; k++) xntn[i * 3 + k] = xn[t * 3 + k];
   }
-  atomicAdd(&tcnt[t], 1ULL);
-  key2[i] = (t << 32) | (uint64_t)i;
+  trg[i] = (uint32_t)t;
+  pair[i] = (uint32_t)i;
 }
 
 // Target-major position q: scatter_index[q] = the pair; near_trg_dsp of a
-// target = its first position.
+// target = its first position, near_trg_cnt the length of its run (its end
+// minus its start, added to 0 by the run's two ends).
 __global__ void __launch_bounds__(NL_WG)
-k_nl_scatter(int64_t n, const uint64_t* __restrict__ key2s, int64_t* __restrict__ scatter, int64_t* __restrict__ tdsp) {
+k_nl_scatter(int64_t n, const uint32_t* __restrict__ trg, const uint32_t* __restrict__ pair,
+             int64_t* __restrict__ scatter, unsigned long long* __restrict__ tcnt, int64_t* __restrict__ tdsp) {
   const int64_t q = (int64_t)blockIdx.x * NL_WG + threadIdx.x;
   if (q >= n) return;
-  const uint64_t k = key2s[q];
-  scatter[q] = (int64_t)(k & 0xffffffffULL);
-  const uint64_t t = k >> 32;
-  if (q == 0 || (key2s[q - 1] >> 32) != t) tdsp[t] = q;
+  const uint32_t t = trg[q];
+  scatter[q] = (int64_t)pair[q];
+  if (q == 0 || trg[q - 1] != t) {
+    tdsp[t] = q;
+    if (q) atomicAdd(&tcnt[t], 0ULL - (unsigned long long)q);
+  }
+  if (q == n - 1 || trg[q + 1] != t) atomicAdd(&tcnt[t], (unsigned long long)(q + 1));
 }
 
-int grid_of(int64_t n) { return (int)((n + NL_WG - 1) / NL_WG); }
-
-template <class T> int dev_alloc(T** p, int64_t n) {
-  *p = nullptr;
-  if (n <= 0) return SCTL_AMD_SUCCESS;
-  SCTL_HIP_TRY(hipMalloc(p, sizeof(T) * n));
-  return SCTL_AMD_SUCCESS;
+// Up to seven arrays of 8-byte words copied by one launch.
+struct CopyList {
+  const uint64_t* src[7];
+  uint64_t* dst[7];
+  int64_t end[7];  // words of the arrays up to and including this one
+};
+__global__ void __launch_bounds__(NL_WG) k_nl_copy(CopyList c) {
+  for (int64_t i = (int64_t)blockIdx.x * NL_WG + threadIdx.x; i < c.end[6]; i += (int64_t)gridDim.x * NL_WG) {
+    int64_t begin = 0;
+#pragma unroll
+    for (int k = 0; k < 7; k++) {
+      if (i >= begin && i < c.end[k]) c.dst[k][i - begin] = c.src[k][i - begin];
+      begin = c.end[k];
+    }
+  }
 }
+
+unsigned grid_of(int64_t n) { return (unsigned)((n + NL_WG - 1) / NL_WG); }
 
 int bits_for(int64_t n) {
   int b = 0;
@@ -432,139 +506,124 @@ int bits_for(int64_t n) {
   return b;
 }
 
+// One pool allocation for a list of n pairs, its count and offset arrays zeroed.
+int list_alloc(sctl_amd_near_list_s* L, int64_t n, hipStream_t s) {
+  DeviceInfo dev;
+  SCTL_TRY(device_info(&dev));
+  Carve c;
+  const size_t xtn = c.take(sizeof(double) * 3 * n), xntn = c.take(L->has_normal ? sizeof(double) * 3 * n : 0),
+               scatter = c.take(sizeof(int64_t) * n), ecnt = c.take(sizeof(int64_t) * L->nelem),
+               edsp = c.take(sizeof(int64_t) * L->nelem), tcnt = c.take(sizeof(int64_t) * L->ntrg),
+               tdsp = c.take(sizeof(int64_t) * L->ntrg);
+  L->n_near = n;
+  if (!c.bytes) return SCTL_AMD_SUCCESS;
+  SCTL_HIP_TRY(hipMallocFromPoolAsync(reinterpret_cast<void**>(&L->buf), c.bytes, dev.pool, s));
+  L->d_xtn = reinterpret_cast<double*>(L->buf + xtn);
+  if (L->has_normal) L->d_xntn = reinterpret_cast<double*>(L->buf + xntn);
+  L->d_scatter = reinterpret_cast<int64_t*>(L->buf + scatter);
+  L->d_ecnt = reinterpret_cast<int64_t*>(L->buf + ecnt);
+  L->d_edsp = reinterpret_cast<int64_t*>(L->buf + edsp);
+  L->d_tcnt = reinterpret_cast<int64_t*>(L->buf + tcnt);
+  L->d_tdsp = reinterpret_cast<int64_t*>(L->buf + tdsp);
+  const int64_t words = (int64_t)(c.bytes - ecnt) / 8;
+  if (words > 0) {
+    hipLaunchKernelGGL(k_nl_zero, dim3(grid_of(words)), dim3(NL_WG), 0, s, L->d_ecnt, words);
+    SCTL_HIP_TRY(hipGetLastError());
+  }
+  return SCTL_AMD_SUCCESS;
+}
+
+// The near pairs' keys, sorted, and the arrays made from them.
+template <class Key>
+int build_pairs(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const double* xn, const double* xs, int64_t ns,
+                const double* rad, int64_t nelem, const int64_t* ecnt, const int64_t* edsp, const double* xsorted,
+                const uint64_t* keys, const uint32_t* idx, const double* cube, hipStream_t s) {
+  const int tbits = bits_for(nt);
+  // Room for 24 pairs per target at first; a longer list is filled again.
+  int64_t cap = (int64_t)std::min<double>((double)nt * (double)nelem, std::max(24.0 * (double)nt, 65536.0)), n = 0;
+  Scratch found;
+  for (int pass = 0; pass < 2; pass++) {
+    Carve c;
+    const size_t counter = c.take(sizeof(int64_t)), pairs_in = c.take(sizeof(Key) * cap);
+    SCTL_TRY(found.alloc(c.bytes, s));
+    int64_t* cnt = reinterpret_cast<int64_t*>(found.as<char>() + counter);
+    hipLaunchKernelGGL(k_nl_zero, dim3(1), dim3(NL_WG), 0, s, cnt, (int64_t)1);
+    hipLaunchKernelGGL((k_nl_elements<Key>), dim3((unsigned)nelem), dim3(NL_WG), 0, s, ecnt, edsp, ns, xs, rad, nt,
+                       xsorted, keys, idx, cube, tbits, reinterpret_cast<unsigned long long*>(cnt), cap,
+                       reinterpret_cast<Key*>(found.as<char>() + pairs_in));
+    SCTL_HIP_TRY(hipGetLastError());
+    SCTL_HIP_TRY(hipMemcpyAsync(&n, cnt, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    SCTL_HIP_TRY(hipStreamSynchronize(s));
+    if (n <= cap) break;
+    SCTL_CHECK_ARG(pass == 0, "near-pair count exceeds its bound (internal error)");
+    cap = n;
+  }
+  SCTL_CHECK_ARG(n < ((int64_t)1 << 32), "more than 2^32-1 near pairs");
+  SCTL_TRY(list_alloc(L, n, s));
+  if (n == 0) return SCTL_AMD_SUCCESS;
+
+  const Key* pairs_in = reinterpret_cast<const Key*>(found.as<char>() + 256);
+  size_t bytes1 = 0, bytes2 = 0;
+  const int bits = tbits + bits_for(nelem);
+  SCTL_HIP_TRY(rocprim::radix_sort_keys(nullptr, bytes1, (Key*)nullptr, (Key*)nullptr, (size_t)n, 0, bits, s));
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes2, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr,
+                                         (uint32_t*)nullptr, (size_t)n, 0, std::max(tbits, 1), s));
+  Carve c;
+  const size_t o_pairs = c.take(sizeof(Key) * n), o_trg = c.take(4 * n), o_pair = c.take(4 * n),
+               o_trg_s = c.take(4 * n), o_pair_s = c.take(4 * n), o_tmp = c.take(std::max(bytes1, bytes2));
+  Scratch work;
+  SCTL_TRY(work.alloc(c.bytes, s));
+  char* w = work.as<char>();
+  Key* pairs = reinterpret_cast<Key*>(w + o_pairs);
+  uint32_t *trg = reinterpret_cast<uint32_t*>(w + o_trg), *pair = reinterpret_cast<uint32_t*>(w + o_pair);
+  uint32_t *trg_s = reinterpret_cast<uint32_t*>(w + o_trg_s), *pair_s = reinterpret_cast<uint32_t*>(w + o_pair_s);
+  SCTL_HIP_TRY(rocprim::radix_sort_keys(w + o_tmp, bytes1, pairs_in, pairs, (size_t)n, 0, std::max(bits, 1), s));
+  hipLaunchKernelGGL((k_nl_elem_ranges<Key>), dim3(grid_of(nelem)), dim3(NL_WG), 0, s, nelem, pairs, n, tbits,
+                     L->d_ecnt, L->d_edsp);
+  SCTL_HIP_TRY(hipGetLastError());
+  hipLaunchKernelGGL((k_nl_unpack<Key>), dim3(grid_of(n)), dim3(NL_WG), 0, s, n, pairs, tbits, xt, xn, L->d_xtn,
+                     L->d_xntn, trg, pair);
+  SCTL_HIP_TRY(hipGetLastError());
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(w + o_tmp, bytes2, trg, trg_s, pair, pair_s, (size_t)n, 0,
+                                         std::max(tbits, 1), s));
+  hipLaunchKernelGGL(k_nl_scatter, dim3(grid_of(n)), dim3(NL_WG), 0, s, n, trg_s, pair_s, L->d_scatter,
+                     reinterpret_cast<unsigned long long*>(L->d_tcnt), L->d_tdsp);
+  SCTL_HIP_TRY(hipGetLastError());
+  return SCTL_AMD_SUCCESS;
+}
+
 // The build on device arrays.
 int build_list(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const double* xn, const double* xs, int64_t ns,
                const double* rad, int64_t nelem, const int64_t* ecnt, const int64_t* edsp, hipStream_t s) {
-  SCTL_TRY(dev_alloc(&L->d_ecnt, nelem));
-  SCTL_TRY(dev_alloc(&L->d_edsp, nelem));
-  SCTL_TRY(dev_alloc(&L->d_tcnt, nt));
-  SCTL_TRY(dev_alloc(&L->d_tdsp, nt));
-  if (nt > 0) {
-    hipLaunchKernelGGL(k_nl_zero, dim3(grid_of(nt)), dim3(NL_WG), 0, s, L->d_tcnt, nt);
-    hipLaunchKernelGGL(k_nl_zero, dim3(grid_of(nt)), dim3(NL_WG), 0, s, L->d_tdsp, nt);
-    SCTL_HIP_TRY(hipGetLastError());
-  }
-  if (nelem > 0) {
-    hipLaunchKernelGGL(k_nl_zero, dim3(grid_of(nelem)), dim3(NL_WG), 0, s, L->d_ecnt, nelem);
-    hipLaunchKernelGGL(k_nl_zero, dim3(grid_of(nelem)), dim3(NL_WG), 0, s, L->d_edsp, nelem);
-    SCTL_HIP_TRY(hipGetLastError());
-  }
-  if (nt == 0 || ns == 0 || nelem == 0) return SCTL_AMD_SUCCESS;
-
-  Scratch box, keys_in, keys, idx_in, idx, tmp;
-  SCTL_TRY(box.alloc(sizeof(double) * 6, s));
-  SCTL_TRY(bounding_box(xt, nt, xs, ns, box.as<double>(), s));
-  hipLaunchKernelGGL(k_nl_cube, dim3(1), dim3(64), 0, s, box.as<double>(), box.as<double>());
-  SCTL_HIP_TRY(hipGetLastError());
-  SCTL_TRY(keys_in.alloc(sizeof(uint64_t) * nt, s));
-  SCTL_TRY(keys.alloc(sizeof(uint64_t) * nt, s));
-  SCTL_TRY(idx_in.alloc(sizeof(uint32_t) * nt, s));
-  SCTL_TRY(idx.alloc(sizeof(uint32_t) * nt, s));
-  hipLaunchKernelGGL(k_nl_keys, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, box.as<double>(), keys_in.as<uint64_t>(),
-                     idx_in.as<uint32_t>());
-  SCTL_HIP_TRY(hipGetLastError());
-  size_t bytes = 0;
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, keys_in.as<uint64_t>(), keys.as<uint64_t>(),
-                                         idx_in.as<uint32_t>(), idx.as<uint32_t>(), (size_t)nt, 0, 63, s));
-  SCTL_TRY(tmp.alloc(bytes, s));
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(tmp.as<void>(), bytes, keys_in.as<uint64_t>(), keys.as<uint64_t>(),
-                                         idx_in.as<uint32_t>(), idx.as<uint32_t>(), (size_t)nt, 0, 63, s));
-  tmp.release();
-  keys_in.release();
-  idx_in.release();
-
-  // elements largest first (scheduling only)
-  Scratch okeys_in, okeys, oidx_in, oidx;
-  SCTL_TRY(okeys_in.alloc(sizeof(uint32_t) * nelem, s));
-  SCTL_TRY(okeys.alloc(sizeof(uint32_t) * nelem, s));
-  SCTL_TRY(oidx_in.alloc(sizeof(uint32_t) * nelem, s));
-  SCTL_TRY(oidx.alloc(sizeof(uint32_t) * nelem, s));
-  hipLaunchKernelGGL(k_nl_order_keys, dim3(grid_of(nelem)), dim3(NL_WG), 0, s, nelem, ecnt, okeys_in.as<uint32_t>(),
-                     oidx_in.as<uint32_t>());
-  SCTL_HIP_TRY(hipGetLastError());
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, okeys_in.as<uint32_t>(), okeys.as<uint32_t>(),
-                                         oidx_in.as<uint32_t>(), oidx.as<uint32_t>(), (size_t)nelem, 0, 32, s));
-  SCTL_TRY(tmp.alloc(bytes, s));
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(tmp.as<void>(), bytes, okeys_in.as<uint32_t>(), okeys.as<uint32_t>(),
-                                         oidx_in.as<uint32_t>(), oidx.as<uint32_t>(), (size_t)nelem, 0, 32, s));
-  tmp.release();
-
-  // Count pass: candidates inside the grown boxes, per (element, wave): an
-  // upper bound of the near pairs.
-  const int64_t nw = nelem * NWAVE;
-  Scratch cnt_w, dsp_w;
-  SCTL_TRY(cnt_w.alloc(sizeof(int64_t) * nw, s));
-  SCTL_TRY(dsp_w.alloc(sizeof(int64_t) * nw, s));
-  const dim3 egrid((unsigned)nelem);
-  hipLaunchKernelGGL(k_nl_elements<false>, egrid, dim3(NL_WG), 0, s, oidx.as<uint32_t>(), ecnt, edsp, ns, xs, rad,
-                     nt, xt, keys.as<uint64_t>(), idx.as<uint32_t>(), box.as<double>(), cnt_w.as<int64_t>(), nullptr,
-                     (int64_t)0, nullptr);
-  SCTL_HIP_TRY(hipGetLastError());
-  SCTL_HIP_TRY(rocprim::exclusive_scan(nullptr, bytes, cnt_w.as<int64_t>(), dsp_w.as<int64_t>(), (int64_t)0,
-                                       (size_t)nw, rocprim::plus<int64_t>(), s));
-  SCTL_TRY(tmp.alloc(bytes, s));
-  SCTL_HIP_TRY(rocprim::exclusive_scan(tmp.as<void>(), bytes, cnt_w.as<int64_t>(), dsp_w.as<int64_t>(), (int64_t)0,
-                                       (size_t)nw, rocprim::plus<int64_t>(), s));
-  tmp.release();
-  int64_t last[2] = {0, 0};
-  SCTL_HIP_TRY(hipMemcpyAsync(&last[0], cnt_w.as<int64_t>() + nw - 1, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  SCTL_HIP_TRY(hipMemcpyAsync(&last[1], dsp_w.as<int64_t>() + nw - 1, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  SCTL_HIP_TRY(hipStreamSynchronize(s));
-  cnt_w.release();
-  dsp_w.release();
-  const int64_t cap = last[0] + last[1];
-
-  // Fill pass: the node tests, near pairs appended in any order.
-  int64_t n = 0;
-  Scratch pairs_in, pairs, key2_in, key2, counter;
-  if (cap > 0) {
-    SCTL_TRY(pairs_in.alloc(sizeof(uint64_t) * cap, s));
-    SCTL_TRY(counter.alloc(sizeof(int64_t), s));
-    hipLaunchKernelGGL(k_nl_zero, dim3(1), dim3(NL_WG), 0, s, counter.as<int64_t>(), (int64_t)1);
-    hipLaunchKernelGGL(k_nl_elements<true>, egrid, dim3(NL_WG), 0, s, oidx.as<uint32_t>(), ecnt, edsp, ns, xs, rad,
-                       nt, xt, keys.as<uint64_t>(), idx.as<uint32_t>(), box.as<double>(), nullptr,
-                       reinterpret_cast<unsigned long long*>(counter.as<int64_t>()), cap, pairs_in.as<uint64_t>());
-    SCTL_HIP_TRY(hipGetLastError());
-    SCTL_HIP_TRY(hipMemcpyAsync(&n, counter.as<int64_t>(), sizeof(int64_t), hipMemcpyDeviceToHost, s));
+  SCTL_HIP_TRY(hipEventCreateWithFlags(&L->last, hipEventDisableTiming));
+  if (nt == 0 || ns == 0 || nelem == 0) {
+    SCTL_TRY(list_alloc(L, 0, s));
     SCTL_HIP_TRY(hipStreamSynchronize(s));
+    return SCTL_AMD_SUCCESS;
   }
-  SCTL_CHECK_ARG(n <= cap, "near-pair count exceeds its bound (internal error)");
-  keys.release();
-  idx.release();
-  L->n_near = n;
-  if (n == 0) return SCTL_AMD_SUCCESS;  // d_ecnt, d_edsp were zeroed
-  SCTL_CHECK_ARG(n < ((int64_t)1 << 32), "more than 2^32-1 near pairs");
-
-  SCTL_TRY(pairs.alloc(sizeof(uint64_t) * n, s));
-  const int ebits = 32 + bits_for(nelem);
-  SCTL_HIP_TRY(rocprim::radix_sort_keys(nullptr, bytes, pairs_in.as<uint64_t>(), pairs.as<uint64_t>(), (size_t)n, 0,
-                                        ebits, s));
-  SCTL_TRY(tmp.alloc(bytes, s));
-  SCTL_HIP_TRY(rocprim::radix_sort_keys(tmp.as<void>(), bytes, pairs_in.as<uint64_t>(), pairs.as<uint64_t>(),
-                                        (size_t)n, 0, ebits, s));
-  tmp.release();
-  pairs_in.release();
-  hipLaunchKernelGGL(k_nl_elem_ranges, dim3(grid_of(nelem)), dim3(NL_WG), 0, s, nelem, pairs.as<uint64_t>(), n,
-                     L->d_ecnt, L->d_edsp);
+  size_t bytes = 0;
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, (uint64_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr,
+                                         (uint32_t*)nullptr, (size_t)nt, 0, 63, s));
+  Carve c;
+  const size_t o_cube = c.take(sizeof(double) * 6), o_keys_in = c.take(8 * nt), o_keys = c.take(8 * nt),
+               o_idx_in = c.take(4 * nt), o_idx = c.take(4 * nt), o_x = c.take(24 * nt), o_tmp = c.take(bytes);
+  Scratch work;
+  SCTL_TRY(work.alloc(c.bytes, s));
+  char* w = work.as<char>();
+  double *cube = reinterpret_cast<double*>(w + o_cube), *xsorted = reinterpret_cast<double*>(w + o_x);
+  uint64_t *keys_in = reinterpret_cast<uint64_t*>(w + o_keys_in), *keys = reinterpret_cast<uint64_t*>(w + o_keys);
+  uint32_t *idx_in = reinterpret_cast<uint32_t*>(w + o_idx_in), *idx = reinterpret_cast<uint32_t*>(w + o_idx);
+  SCTL_TRY(bounding_box(xt, nt, xs, ns, cube, s));
+  hipLaunchKernelGGL(k_nl_cube, dim3(1), dim3(64), 0, s, cube, cube);
+  hipLaunchKernelGGL(k_nl_keys, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, cube, keys_in, idx_in);
   SCTL_HIP_TRY(hipGetLastError());
-
-  SCTL_TRY(dev_alloc(&L->d_xtn, n * 3));
-  if (xn) SCTL_TRY(dev_alloc(&L->d_xntn, n * 3));
-  SCTL_TRY(dev_alloc(&L->d_scatter, n));
-  SCTL_TRY(key2_in.alloc(sizeof(uint64_t) * n, s));
-  SCTL_TRY(key2.alloc(sizeof(uint64_t) * n, s));
-  hipLaunchKernelGGL(k_nl_unpack, dim3(grid_of(n)), dim3(NL_WG), 0, s, n, pairs.as<uint64_t>(), xt, xn, L->d_xtn,
-                     L->d_xntn, reinterpret_cast<unsigned long long*>(L->d_tcnt), key2_in.as<uint64_t>());
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(w + o_tmp, bytes, keys_in, keys, idx_in, idx, (size_t)nt, 0, 63, s));
+  hipLaunchKernelGGL(k_nl_gather, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, idx, xsorted);
   SCTL_HIP_TRY(hipGetLastError());
-  const int tbits = 32 + bits_for(nt);
-  SCTL_HIP_TRY(rocprim::radix_sort_keys(nullptr, bytes, key2_in.as<uint64_t>(), key2.as<uint64_t>(), (size_t)n, 0,
-                                        tbits, s));
-  SCTL_TRY(tmp.alloc(bytes, s));
-  SCTL_HIP_TRY(rocprim::radix_sort_keys(tmp.as<void>(), bytes, key2_in.as<uint64_t>(), key2.as<uint64_t>(),
-                                        (size_t)n, 0, tbits, s));
-  hipLaunchKernelGGL(k_nl_scatter, dim3(grid_of(n)), dim3(NL_WG), 0, s, n, key2.as<uint64_t>(), L->d_scatter,
-                     L->d_tdsp);
-  SCTL_HIP_TRY(hipGetLastError());
+  if (bits_for(nt) < 32 && bits_for(nt) + bits_for(nelem) <= 32)
+    SCTL_TRY(build_pairs<uint32_t>(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, xsorted, keys, idx, cube, s));
+  else
+    SCTL_TRY(build_pairs<uint64_t>(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, xsorted, keys, idx, cube, s));
   SCTL_HIP_TRY(hipStreamSynchronize(s));
   return SCTL_AMD_SUCCESS;
 }
@@ -645,20 +704,39 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
   SCTL_CHECK_ARG((flags & ~SCTL_AMD_HOST_PTRS) == 0, "unknown flag bits");
   SCTL_CHECK_ARG(!Xn_trg_near || list->has_normal || list->n_near == 0, "the list was built without target normals");
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : hipStreamPerThread;
-  const hipMemcpyKind kind = (flags & SCTL_AMD_HOST_PTRS) ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
-  auto cp = [&](void* dst, const void* src, size_t bytes) -> int {
-    if (!dst || !src || !bytes) return SCTL_AMD_SUCCESS;
-    SCTL_HIP_TRY(hipMemcpyAsync(dst, src, bytes, kind, s));
-    return SCTL_AMD_SUCCESS;
-  };
-  const int64_t n = list->n_near;
-  SCTL_TRY(cp(Xtrg_near, list->d_xtn, sizeof(double) * 3 * n));
-  SCTL_TRY(cp(Xn_trg_near, list->d_xntn, sizeof(double) * 3 * n));
-  SCTL_TRY(cp(near_elem_cnt, list->d_ecnt, sizeof(int64_t) * list->nelem));
-  SCTL_TRY(cp(near_elem_dsp, list->d_edsp, sizeof(int64_t) * list->nelem));
-  SCTL_TRY(cp(near_scatter_index, list->d_scatter, sizeof(int64_t) * n));
-  SCTL_TRY(cp(near_trg_cnt, list->d_tcnt, sizeof(int64_t) * list->ntrg));
-  SCTL_TRY(cp(near_trg_dsp, list->d_tdsp, sizeof(int64_t) * list->ntrg));
+  const int64_t n = list->n_near, ne = list->nelem, nt = list->ntrg;
+  const struct {
+    void* dst;
+    const void* src;
+    int64_t words;
+  } a[7] = {{Xtrg_near, list->d_xtn, 3 * n},          {Xn_trg_near, list->d_xntn, 3 * n},
+            {near_elem_cnt, list->d_ecnt, ne},        {near_elem_dsp, list->d_edsp, ne},
+            {near_scatter_index, list->d_scatter, n}, {near_trg_cnt, list->d_tcnt, nt},
+            {near_trg_dsp, list->d_tdsp, nt}};
+  // Reads of the results follow each other whatever their streams, so that the
+  // list can be destroyed after the last one (a captured read runs later: its
+  // graph needs the list to live, as any graph its buffers).
+  const bool capturing = stream_capturing(s);
+  if (!capturing) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->last, 0));
+  if (flags & SCTL_AMD_HOST_PTRS) {
+    for (const auto& x : a)
+      if (x.dst && x.src && x.words)
+        SCTL_HIP_TRY(hipMemcpyAsync(x.dst, x.src, 8 * (size_t)x.words, hipMemcpyDeviceToHost, s));
+  } else {
+    CopyList c;
+    int64_t words = 0;
+    for (int k = 0; k < 7; k++) {
+      words += a[k].dst && a[k].src ? a[k].words : 0;
+      c.src[k] = static_cast<const uint64_t*>(a[k].src);
+      c.dst[k] = static_cast<uint64_t*>(a[k].dst);
+      c.end[k] = words;
+    }
+    if (words) {
+      hipLaunchKernelGGL(k_nl_copy, dim3(std::min<unsigned>(grid_of(words), 4096)), dim3(NL_WG), 0, s, c);
+      SCTL_HIP_TRY(hipGetLastError());
+    }
+  }
+  if (!capturing) SCTL_HIP_TRY(hipEventRecord(list->last, s));
   if (flags & SCTL_AMD_HOST_PTRS) SCTL_HIP_TRY(hipStreamSynchronize(s));
   return SCTL_AMD_SUCCESS;
 }
