@@ -169,27 +169,91 @@ k_reduce_splits(const double* __restrict__ part, int64_t n, int nsplit, double* 
 
 // ------------------------------------------------------------- KernelMatrix
 // M[(s*K0+k0)*ld + t*K1+k1] = scale * u[k0][k1]; one lane per target, the
-// workgroup's gridDim.y slices stride over the sources.
+// workgroup's gridDim.y slices stride over the sources.  HBM-write bound: the
+// rows leave through LDS as consecutive words, so that a wave's store covers
+// four whole 128-byte lines where a lane's own K1 words would leave lines to
+// be merged.  A row starts anywhere within a line, so each workgroup writes the
+// whole lines that start within its columns, and computes HALO targets of its
+// predecessor's for the words of the first; only a row's first and last line
+// is shared with its neighbours.  Where a source gives one word per target,
+// four sources go under one barrier and the stores are nontemporal (wider rows
+// were 10-25 % slower with them).  Two words per target are one 16-byte store
+// and stay as they are.  MI355X, TB/s written, lane by lane / through LDS:
+//   Laplace FxU 10001 x 9000 3.0 / 5.4, 8192 x 8192 3.3 / 5.5
+//   Stokes FxU 2003 x 3001 4.5 / 5.3; Laplace FxdU 3658 x 1056 4.8 / 5.8
+//   Laplace Fxd2U 2001 x 2000 2.7 / 6.5; Stokes FxT 1000 x 1003 2.7 / 6.5
+// (a fill of 2 GiB: 6.8; Helmholtz FxU, left alone, 5.4-5.9).
+template <int K1> constexpr int kmat_halo() { return (15 + K1 - 1) / K1; }  // targets that cover 15 words
+template <int KER> constexpr int kmat_sources() { return Ker<KER>::K0 * Ker<KER>::K1 == 1 ? 4 : 1; }
+
 template <int KER, int NEWTON>
 __global__ void __launch_bounds__(WG)
 k_kernel_matrix(const double* __restrict__ xt, int64_t nt, const double* __restrict__ xs,
                 const double* __restrict__ xn, int64_t ns, double* __restrict__ M, double scale, double mu) {
   using K = Ker<KER>;
-  constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND;
-  const int64_t t = (int64_t)blockIdx.x * WG + threadIdx.x;
-  if (t >= nt) return;
-  const int64_t ld = nt * K1;
-  const double tx = xt[t * 3 + 0], ty = xt[t * 3 + 1], tz = xt[t * 3 + 2];
-  for (int64_t s = blockIdx.y; s < ns; s += gridDim.y) {
+  constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, SB = kmat_sources<KER>();
+  constexpr bool DIRECT = K1 == 2;
+  constexpr int HALO = DIRECT ? 0 : kmat_halo<K1>(), TB = WG - HALO;
+  const int tid = threadIdx.x;
+  const int64_t first = (int64_t)blockIdx.x * TB, t = first - HALO + tid, ld = nt * K1;
+  const int64_t tc = t < 0 ? 0 : (t < nt ? t : nt - 1);  // the targets past either end are not written
+  const double tx = xt[tc * 3 + 0], ty = xt[tc * 3 + 1], tz = xt[tc * 3 + 2];
+  auto values = [&](int64_t s, double(&u)[K0][K1]) {
     double n[3] = {0, 0, 0};
 #pragma unroll
     for (int k = 0; k < ND; k++) n[k] = xn[s * 3 + k];
-    double u[K0][K1];
     kmatrix<KER, NEWTON>(u, tx - xs[s * 3 + 0], ty - xs[s * 3 + 1], tz - xs[s * 3 + 2], n, mu);
+  };
+  if constexpr (DIRECT) {
+    for (int64_t s = blockIdx.y; s < ns; s += gridDim.y) {
+      double u[K0][K1];
+      values(s, u);
+      if (t < nt) {
 #pragma unroll
-    for (int k0 = 0; k0 < K0; k0++)
+        for (int k0 = 0; k0 < K0; k0++)
 #pragma unroll
-      for (int k1 = 0; k1 < K1; k1++) M[(s * K0 + k0) * ld + t * K1 + k1] = u[k0][k1] * scale;
+          for (int k1 = 0; k1 < K1; k1++) M[(s * K0 + k0) * ld + t * K1 + k1] = u[k0][k1] * scale;
+      }
+    }
+  } else {
+    __shared__ double rows[2][SB][WG * K1];
+    const int64_t base = (first - HALO) * K1, c_lo = first * K1, c_hi = (first + TB) * K1;
+    // Row r of M from a buffer.
+    auto write = [&](int64_t r, const double* row) {
+      double* Mr = M + r * ld;
+      const int64_t a = (int64_t)((reinterpret_cast<uintptr_t>(Mr) >> 3) & 15);
+      const int64_t c0 = blockIdx.x ? c_lo - ((c_lo + a) & 15) : 0;
+      const int64_t c1 = c_hi < ld ? c_hi - ((c_hi + a) & 15) : ld;
+#pragma unroll
+      for (int i = 0; i < K1 + 1; i++) {  // c1 - c0 <= TB * K1 + 15 <= (K1 + 1) * WG
+        const int64_t c = c0 + tid + (int64_t)i * WG;
+        if (c < c1) {
+          if constexpr (K1 == 1) __builtin_nontemporal_store(row[c - base], Mr + c);
+          else Mr[c] = row[c - base];
+        }
+      }
+    };
+    // Two buffers, one barrier each time one is filled: a thread fills a buffer
+    // again only after every thread has passed the other's barrier, and so has
+    // read this one.
+    int buf = 0;
+    for (int64_t s = (int64_t)blockIdx.y * SB; s < ns; s += (int64_t)gridDim.y * SB) {
+      double u[SB][K0][K1];
+#pragma unroll
+      for (int j = 0; j < SB; j++) values(s + j < ns ? s + j : ns - 1, u[j]);
+#pragma unroll
+      for (int k0 = 0; k0 < K0; k0++) {
+#pragma unroll
+        for (int j = 0; j < SB; j++)
+#pragma unroll
+          for (int k1 = 0; k1 < K1; k1++) rows[buf][j][tid * K1 + k1] = u[j][k0][k1] * scale;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SB; j++)
+          if (s + j < ns) write((s + j) * K0 + k0, rows[buf][j]);
+        buf ^= 1;
+      }
+    }
   }
 }
 
@@ -335,9 +399,19 @@ int launch_eval_f64(int ker, int newton, const double* r_trg, int64_t nt, const 
 int launch_kernel_matrix(int ker, int newton, const double* r_trg, int64_t nt, const double* r_src,
                          const double* n_src, int64_t ns, double* M, double ctx, hipStream_t stream) {
   if (nt <= 0 || ns <= 0) return SCTL_AMD_SUCCESS;
-  const int64_t tb = (nt + WG - 1) / WG;
+  DeviceInfo dev;
+  SCTL_TRY(device_info(&dev));
+  int K0, K1, ND;
+  kernel_dims(ker, &K0, &K1, &ND);
+  const int64_t per = K1 == 2 ? WG : WG - (15 + K1 - 1) / K1;  // targets per workgroup (kmat_halo)
+  const int64_t tb = (nt + per - 1) / per;
   SCTL_CHECK_ARG(tb <= 0x7fffffffLL, "too many targets for one launch");
-  const int64_t gy = std::min<int64_t>(ns, 8192);
+  // About 32 workgroups per CU, each with several rows to its targets (8 to 64
+  // are within 3 %); the 16-byte stores run best with a source to a workgroup
+  // (3501 x 3000: 5.9 against 5.3 TB/s).
+  const int64_t want = 32LL * std::max(dev.num_cus, 1);
+  const int64_t gy = K1 == 2 ? std::min<int64_t>(ns, 8192)
+                             : std::min<int64_t>(ns, std::min<int64_t>(65535, (want + tb - 1) / tb));
   const double scale = kernel_scale(ker);
   profile_count(ker, nt * ns);
   ProfileScope prof(stream);
