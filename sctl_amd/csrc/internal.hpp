@@ -146,6 +146,7 @@ int f64_apply(int ker, int newton, const double* r_trg, int64_t nt, const double
 bool mixed_runs_f64(int ker, int64_t nt, int64_t ns);
 struct MixedGeometry {
   int ti = 0, Q = 0;
+  bool mfma = false;  // the far form on the matrix cores
   int64_t tb = 0, ntiles = 0, nsplit = 1, tps = 0;
   int64_t group = 1;  // splits per launch (split_group)
   size_t packed_bytes = 0, meta_bytes = 0, part_bytes = 0;

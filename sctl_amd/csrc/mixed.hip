@@ -8,23 +8,23 @@
 // H^2 = max |s'|^2.  A target (held in FP64) forms t - c once per tile the same
 // way, t' + t''.
 //
-// Per (wave, tile) one of two loops runs:
-//   far  -- every target of the wave has |t'| >= 3H, so every pair has
-//           r >= 2H.  Laplace kernels use r^2 = |t'|^2 + |s'|^2 - 2 t'.s'
-//           (one add and three FMAs; the rounding error is at most a few ulp
-//           of r^2 because r^2 >= (|t'| - H)^2 is never small against the
-//           terms).  Stokes kernels use dx = t' - s'.
-//   near -- some target is within 3H of the tile centre: positions are
-//           differenced from both halves, dx = (t' - s') + (t'' - s''), which
-//           is accurate to about 2^-23 relative to dx however small r is, and
-//           r^2 == 0 is masked as in the reference (kernel_functions.hpp:45).
+// Per (wave, tile or 64-source sub-tile) one of three forms runs:
+//   far  -- pairs so far apart for the tile's size that the expanded r^2 =
+//           |t'|^2 + |s'|^2 - 2 t'.s' is accurate to a few ulp; formed on the
+//           matrix cores (k_eval_mixed_mfma; the kernels and sizes of
+//           far_mfma_at).
+//   mid  -- every pair has r >= H: dx = t' - s'.
+//   near -- positions are differenced from both halves, dx = (t' - s') +
+//           (t'' - s''), which is accurate to about 2^-23 relative to dx
+//           however small r is, and r^2 == 0 is masked as in the reference
+//           (kernel_functions.hpp:45).
 // Targets in Hilbert order keep a wave's targets together, so only tiles next
 // to the wave take the near loop.  The pairs of every 64 sources are summed
 // in FP32 and added into an FP64 sum of the tile, so that a tile's largest
 // term does not take up the rounding of 255 FP32 additions (this halved the
 // headline's error against FP64, 5.4e-7 -> 2.7e-7, at no cost in time).  A
-// far tile whose sum is not finite is redone by the near loop.  Each tile's
-// sum is added into the FP64 per-target sum with Kahan compensation.
+// tile whose sum is not finite is redone by the near loop.  The tiles' sums are
+// added up in FP64 per target.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -92,35 +92,20 @@ __device__ __forceinline__ void fill_record(float* r, const double* d, const dou
   r[LO + 2] = lo[2];
 }
 
-// Far-field interaction.  th: t' ; a: -2 t' ; T: |t'|^2 ; r: the record.
+// Mid-range pair (r >= H): one-part FP32 differences, accurate to a few ulp of
+// r there, and no mask.  th: t'; r: the record.
 template <int KER, int NEWTON>
-__device__ __forceinline__ void mix_far(float* p, const float* th, const float* a, float T, const float* r, float mu) {
-  if constexpr (KER == LAP_FXU) {
-    const float r2 = fmad(a[2], r[2], fmad(a[1], r[1], fmad(a[0], r[0], T + r[3])));
-    p[0] = fmad(rsq_deferred<NEWTON>(r2), r[4], p[0]);
-  } else if constexpr (KER == LAP_DXU) {
-    const float r2 = fmad(a[2], r[2], fmad(a[1], r[1], fmad(a[0], r[0], T + r[3])));
-    const float rnq = fmad(th[2], r[6], fmad(th[1], r[5], fmad(th[0], r[4], r[7])));
-    const float z = rsq_deferred<NEWTON>(r2);
-    p[0] = fmad(rnq, z * z * z, p[0]);
-  } else {
-    using L = MixLayout<KER>;
-    interact<KER, NEWTON, false>(p, th[0] - r[0], th[1] - r[1], th[2] - r[2], r + L::NOFF, r + L::FOFF, mu);
-  }
-}
-
-// Mid-range pair of the Laplace kernels (every target of the wave at least
-// 2H from the tile centre, so r >= H): one-part FP32 differences, accurate
-// to a few ulp of r there, and no mask.
-template <int KER, int NEWTON>
-__device__ __forceinline__ void mix_mid(float* p, const float* th, const float* r) {
+__device__ __forceinline__ void mix_mid(float* p, const float* th, const float* r, float mu) {
   const float dx = th[0] - r[0], dy = th[1] - r[1], dz = th[2] - r[2];
   if constexpr (KER == LAP_FXU) {
     const float f[1] = {r[4]};
     interact<LAP_FXU, NEWTON, false>(p, dx, dy, dz, f, f);
-  } else {
+  } else if constexpr (KER == LAP_DXU) {
     const float one[1] = {1.0f}, nq[3] = {r[4], r[5], r[6]};
     interact<LAP_DXU, NEWTON, false>(p, dx, dy, dz, nq, one);
+  } else {
+    using L = MixLayout<KER>;
+    interact<KER, NEWTON, false>(p, dx, dy, dz, r + L::NOFF, r + L::FOFF, mu);
   }
 }
 
@@ -284,31 +269,27 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
     const double4 m = meta[tile];
     __syncthreads();
 
-    // A wave whose targets are all |t'| >= 3H from the tile centre takes the
-    // far form over the whole tile (the expanded r^2 of the Laplace kernels,
-    // one-part differences for the others; the latter from |t'| >= 2H).
-    // Otherwise each 64-source sub-tile q (centre b_q, radius h_q about it)
-    // is classified on its own, with X = |t'| + H the scale of the rounding
-    // of t' and s' and r >= |t' - b_q| - h_q: far where that bound is >= X/2
-    // (relative error of the expanded r^2 <= 4 eps), mid (one-part
-    // differences, relative error <= 3 eps) where it is >= X/3, else near
-    // (two-part differences, masked).  A non-finite partial redoes the tile
-    // in the near form.
-    constexpr bool EXPANDED = KER == LAP_FXU || KER == LAP_DXU;
-    const float far_r2 = (EXPANDED ? 9.0f : 4.0f) * (float)m.w;
+    // A wave whose targets are all |t'| >= 2H from the tile centre (so r >= H)
+    // takes the mid form over the whole tile.  Otherwise each 64-source sub-tile
+    // q (centre b_q, radius h_q about it) is classified on its own, with X =
+    // |t'| + H the scale of the rounding of t' and s' and r >= |t' - b_q| - h_q:
+    // mid (relative error <= 3 eps) where that bound is >= X/3, else near
+    // (two-part differences, masked).  A non-finite partial redoes the tile in
+    // the near form.
+    const float mid_r2 = 4.0f * (float)m.w;
     // p: FP32 sums of at most 64 pairs, added into the FP64 tile sums pt
     // after every 64 sources (sub64), so that a tile's dominant term does
     // not absorb the rounding of 255 FP32 additions.
     float th[TPL][3], T[TPL], p[TPL][K1];
     double pt[TPL][K1];
-    bool notfar = false;
+    bool notmid = false;
 #pragma unroll
     for (int j = 0; j < TPL; j++) {
       th[j][0] = (float)(t64[j][0] - m.x);
       th[j][1] = (float)(t64[j][1] - m.y);
       th[j][2] = (float)(t64[j][2] - m.z);
       T[j] = fmad(th[j][2], th[j][2], fmad(th[j][1], th[j][1], th[j][0] * th[j][0]));
-      notfar |= T[j] < far_r2;
+      notmid |= T[j] < mid_r2;
 #pragma unroll
       for (int k = 0; k < K1; k++) {
         p[j][k] = 0.0f;
@@ -326,50 +307,21 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
     };
     const float* recs = reinterpret_cast<const float*>(lds);
     bool use_near = false;
-    // -2 t', formed where a far loop needs it (not held across the sub-tiles)
-    auto minus2 = [&](float(&a)[TPL][3]) {
-#pragma unroll
-      for (int j = 0; j < TPL; j++)
-#pragma unroll
-        for (int k = 0; k < 3; k++) a[j][k] = -2.0f * th[j][k];
-    };
     // At more than one target per lane a wave's targets span more space and
     // the sub-tile classes would raise the kernel's registers (two targets
-    // per lane: 70 -> 93 VGPRs); such shapes classify whole tiles only, with
-    // the mid class at |t'| >= 2H.
+    // per lane: 70 -> 93 VGPRs); such shapes classify whole tiles only.
     constexpr bool SUBTILES = TPL == 1;
-    bool tile_mid = false;
-    if constexpr (!SUBTILES) {
-      const float mid_r2 = 4.0f * (float)m.w;
-      bool near = false;
-#pragma unroll
-      for (int j = 0; j < TPL; j++) near |= T[j] < mid_r2;
-      use_near = __builtin_amdgcn_ballot_w64(near) != 0;
-      tile_mid = !use_near && EXPANDED && __builtin_amdgcn_ballot_w64(notfar) != 0;
-    }
+    const bool tile_mid = __builtin_amdgcn_ballot_w64(notmid) == 0;
+    use_near = !SUBTILES && !tile_mid;
     if (use_near) {
       // the near loop below
     } else if (tile_mid) {
-      if constexpr (EXPANDED) {
-        for (int i0 = 0; i0 < TILE; i0 += 64) {
-#pragma unroll 4
-          for (int i = i0; i < i0 + 64; i++) {
-            const float* rec = recs + i * R;
-#pragma unroll
-            for (int j = 0; j < TPL; j++) mix_mid<KER, NEWTON>(p[j], th[j], rec);
-          }
-          sub64();
-        }
-      }
-    } else if (!SUBTILES || __builtin_amdgcn_ballot_w64(notfar) == 0) {
-      float a[TPL][3];
-      minus2(a);
       for (int i0 = 0; i0 < TILE; i0 += 64) {
 #pragma unroll 4
         for (int i = i0; i < i0 + 64; i++) {
           const float* rec = recs + i * R;
 #pragma unroll
-          for (int j = 0; j < TPL; j++) mix_far<KER, NEWTON>(p[j], th[j], a[j], T[j], rec, mu);
+          for (int j = 0; j < TPL; j++) mix_mid<KER, NEWTON>(p[j], th[j], rec, mu);
         }
         sub64();
       }
@@ -379,14 +331,13 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
       for (int q = 0; q < WG / 64; q++) {
         const float4 b = sub[tile * (WG / 64) + q];
         const float h = sqrtf(b.w);
-        bool qnotfar = false, qnear = false;
+        bool qnear = false;
 #pragma unroll
         for (int j = 0; j < TPL; j++) {
           const float X = sqrtf(T[j]) + H;
           const float dx = th[j][0] - b.x, dy = th[j][1] - b.y, dz = th[j][2] - b.z;
           const float d2 = fmad(dz, dz, fmad(dy, dy, dx * dx));
-          const float ef = fmad(0.5f, X, h), em = fmad(1.0f / 3.0f, X, h);
-          qnotfar |= d2 < ef * ef;
+          const float em = fmad(1.0f / 3.0f, X, h);
           qnear |= d2 < em * em;
         }
         const float* qrec = recs + q * 64 * R;
@@ -403,21 +354,11 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
 #pragma unroll
             for (int j = 0; j < TPL; j++) mix_near<KER, NEWTON>(p[j], th[j], tl[j], qrec + i * R, mu);
           }
-        } else if (EXPANDED && __builtin_amdgcn_ballot_w64(qnotfar) != 0) {
-          if constexpr (EXPANDED) {
-#pragma unroll 4
-            for (int i = 0; i < 64; i++) {
-#pragma unroll
-              for (int j = 0; j < TPL; j++) mix_mid<KER, NEWTON>(p[j], th[j], qrec + i * R);
-            }
-          }
         } else {
-          float a[TPL][3];
-          minus2(a);
 #pragma unroll 4
           for (int i = 0; i < 64; i++) {
 #pragma unroll
-            for (int j = 0; j < TPL; j++) mix_far<KER, NEWTON>(p[j], th[j], a[j], T[j], qrec + i * R, mu);
+            for (int j = 0; j < TPL; j++) mix_mid<KER, NEWTON>(p[j], th[j], qrec + i * R, mu);
           }
         }
         sub64();
@@ -482,9 +423,10 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
   }
 }
 
-// ---- Laplace kernels: the far form on the matrix cores ---------------------
+// ---- The far form on the matrix cores --------------------------------------
 // The far form's r^2 = |t'|^2 + |s'|^2 - 2 t'.s' (and the double layer's
-// f n.r = t'.nq - s'.nq) is a contraction over the three axes.  FP32 values are
+// f n.r = t'.nq - s'.nq, Stokes' f.r and n.r) is a contraction over the three
+// axes.  FP32 values are
 // cut into three bf16 parts (8 of the 24 mantissa bits each, by truncation, so
 // the parts' sum is exact), and a product of two such values is the sum of
 // eight products of parts (all but the last parts' product, 2^-32 of it): the
@@ -497,8 +439,8 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
 // Cycles per 256 pairs of one SIMD on MI355X (8 waves, 2.4 GHz): 17 for the
 // instruction, 33 for four v_rsq_f32, 12 for four FMAs, 55 together; the
 // FP32 form needs 94.  Dense plan applies, 524288 x 524288 sphere and shell
-// (FP32 form -> this): Laplace FxU 46.5 -> 30.4 ms (9.0e12 pairs/s), DxU 70.7
-// -> 48.6 ms; 131072 x 131072 cube 3.36 -> 2.66 and 5.04 -> 3.98 ms.
+// (FP32 form -> this): Laplace FxU 46.5 -> 29.2 ms (9.4e12 pairs/s), DxU 70.7
+// -> 45.6 ms; 131072 x 131072 cube 3.36 -> 2.60 and 5.04 -> 3.84 ms.
 //
 // The matrix cores round sums toward minus infinity somewhere below 2^-29 of
 // their largest term: a bias of one sign, which 130 001 double layer terms of
@@ -514,7 +456,42 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
-template <int KER> constexpr bool far_mfma() { return KER == LAP_FXU || KER == LAP_DXU; }
+
+// A kernel's far form.  NV: dot products with t' - s' beside r^2 (DxU: nq;
+// Stokes: f, and n for the double layer).  GRAD: outputs along r = t' - s',
+// summed as t'_k (sum g) - (sum g s'_k).  NROW: FP32 words per source that the
+// pairs read besides (s' where GRAD, then the densities).
+template <int KER> struct FarForm {
+  static constexpr bool ON = false;
+  static constexpr int NV = 0, NROW = 0;
+  static constexpr bool GRAD = false;
+};
+template <> struct FarForm<LAP_FXU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 0, NROW = 1;
+  static constexpr bool GRAD = false;
+};
+template <> struct FarForm<LAP_DXU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 1, NROW = 0;
+  static constexpr bool GRAD = false;
+};
+template <> struct FarForm<LAP_FXDU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 0, NROW = 4;
+  static constexpr bool GRAD = true;
+};
+template <> struct FarForm<STK_FXU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 1, NROW = 6;
+  static constexpr bool GRAD = true;
+};
+template <> struct FarForm<STK_DXU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 2, NROW = 3;
+  static constexpr bool GRAD = true;
+};
+template <int KER> constexpr bool far_mfma() { return FarForm<KER>::ON; }
 // |t'|^2 below this takes the FP32 forms: the matrix cores may flush parts
 // below 2^-126, which are 2^-16 of |t'|^2.
 constexpr float MFMA_MIN_T = 0x1p-100f;
@@ -552,27 +529,63 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Mixed Eval of the Laplace kernels, 64 targets per wave.  Each tile's sources
+// One far pair: D = r^2, d = the NV dot products, row(k) = word k of the source.
+template <int KER, int NEWTON, class Row>
+__device__ __forceinline__ void far_pair(float* p, float& G, float r2, const float* d, Row&& row) {
+  float z = rsq_deferred<NEWTON>(r2);
+  if constexpr (Ker<KER>::POW == 0 && NEWTON > 0) z *= (float)newton_c2(NEWTON);
+  if constexpr (KER == LAP_FXU) {
+    p[0] = fmad(z, row(0), p[0]);
+  } else if constexpr (KER == LAP_DXU) {
+    p[0] = fmad(d[0] * z, z * z, p[0]);
+  } else if constexpr (KER == STK_FXU) {  // z (f + w r), w = (f.r) z^2
+    const float w = d[0] * (z * z);
+#pragma unroll
+    for (int k = 0; k < 3; k++) p[k] = fmad(z, fmad(-w, row(k), row(3 + k)), p[k]);
+    G = fmad(w, z, G);
+  } else {  // g r
+    const float z2 = z * z;
+    const float g = KER == LAP_FXDU ? row(3) * z * z2 : (d[0] * z2) * (d[1] * z2) * z;
+#pragma unroll
+    for (int k = 0; k < 3; k++) p[k] = fmad(-g, row(k), p[k]);
+    G += g;
+  }
+}
+
+// Mixed Eval with the far form above, 64 targets per wave.  Each tile's sources
 // are staged as k-slots; the classes are those of k_eval_mixed at one target
 // per lane (whole tile, else 64-source sub-tiles).  Far pairs are summed in the
 // matrix layout (at most 64 per FP32 sum), mid and near ones with one target
 // per lane from records that the wave stages for itself, NEAR_ST at a time.
 //
-// Four waves per SIMD are asked for: left alone the compiler takes 148
-// registers for the double layer (three waves), 58.6 instead of 48.6 ms at
-// 524288 x 524288; at six waves the single layer spills (32.1 against 30.4 ms).
+// Waves per SIMD asked for: left alone the compiler takes 148 registers for the
+// Laplace double layer (three waves), 58.6 instead of 45.6 ms at 524288 x
+// 524288; at six waves the single layer spills (32.1 against 30.4 ms then).
+// Three outputs hold 12 FP64 sums per lane more, and run three waves (128
+// registers spill: Stokes FxU 105 against 85 ms).
+template <int KER> constexpr int mfma_waves() { return Ker<KER>::K1 == 1 ? 4 : 3; }
+// Chunks and sources unrolled, from sweeps of 1, 2 and 4 resp. 2, 4 and 8.
+template <int KER> constexpr int far_unroll() { return Ker<KER>::K1 == 1 ? 4 : (KER == STK_FXU ? 2 : 1); }
+template <int KER> constexpr int lane_unroll() { return KER == STK_FXU || KER == STK_DXU ? 2 : 4; }
 template <int KER, int NEWTON>
-__global__ void __launch_bounds__(WG, 4)
+__global__ void __launch_bounds__(WG, (mfma_waves<KER>()))
 k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __restrict__ tperm,
                   const float4* __restrict__ packed, const double4* __restrict__ meta, const float4* __restrict__ sub,
                   int64_t ntiles, int64_t tiles_per_split, double* __restrict__ out, int direct, double scale,
                   double) {
-  constexpr int Q = MixLayout<KER>::Q, R = 4 * Q, NEAR_ST = 32, GROUPS = 4, CHUNKS = TILE / 16;
-  constexpr bool DXU = KER == LAP_DXU;
-  __shared__ u32x4 rs[TILE * 4];                  // -2 s' (group 3: ones against |t'|^2)
-  __shared__ u32x4 rn[DXU ? TILE * 4 : 1];        // nq (group 3: zeros)
-  __shared__ float sS[TILE], sq[DXU ? 1 : TILE];  // |s'|^2, density
-  __shared__ float sn[DXU ? TILE : 1];            // -s'.nq
+  using F = FarForm<KER>;
+  using L = MixLayout<KER>;
+  constexpr int K1 = Ker<KER>::K1, Q = L::Q, R = 4 * Q, NEAR_ST = 32, GROUPS = 4, CHUNKS = TILE / 16;
+  constexpr int NV = F::NV, NROW = F::NROW;
+  constexpr bool LAP = KER == LAP_FXU || KER == LAP_DXU;
+  // k-slots, 16 rows x 3 axes per chunk; the last entry is all of group 3's:
+  // ones against |t'|^2 in rs, zeros in rv.
+  constexpr int SLOTS = TILE * 3;
+  __shared__ u32x4 rs[SLOTS + 1];                    // -2 s'
+  __shared__ u32x4 rv[NV ? NV : 1][NV ? SLOTS + 1 : 1];  // the NV vectors v
+  __shared__ float sS[TILE];                        // |s'|^2
+  __shared__ float sv[NV ? NV : 1][NV ? TILE : 1];  // -s'.v
+  __shared__ float srow[NROW ? NROW : 1][NROW ? TILE : 1];
   __shared__ float4 near_all[(WG / 64) * NEAR_ST * Q];
 
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
@@ -583,25 +596,33 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
   const int64_t q0 = wg.block * WG + (tid & ~63);  // the wave's first target
 
   // t64: this lane's target (q0 + lane); tg: axis g of the targets q0 + 16 m + c16
-  double t64[3], tg[GROUPS], accn = 0.0, accf[GROUPS];
+  double t64[3], tg[GROUPS], accn[K1], accf[GROUPS][K1];
 #pragma unroll
   for (int k = 0; k < 3; k++) t64[k] = q0 + lane < nt ? xt[(q0 + lane) * 3 + k] : 0.0;
 #pragma unroll
   for (int m = 0; m < GROUPS; m++) {
     const int64_t q = q0 + 16 * m + c16;
     tg[m] = q < nt && g < 3 ? xt[q * 3 + g] : 0.0;
-    accf[m] = 0.0;
   }
-  // group 3's slots never change: this thread's row of chunk tid / 16
-  rs[(tid >> 4) * 64 + 48 + (tid & 15)] = u32x4{0x3f803f80u, 0x00003f80u, 0u, 0u};
-  if constexpr (DXU) rn[(tid >> 4) * 64 + 48 + (tid & 15)] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int k = 0; k < K1; k++) {
+    accn[k] = 0.0;
+#pragma unroll
+    for (int m = 0; m < GROUPS; m++) accf[m][k] = 0.0;
+  }
+  const int slot = (tid >> 4) * 48 + (tid & 15);  // this thread's row, written per tile
+  const int my_slot = g < 3 ? lane : SLOTS, my_step = g < 3 ? 48 : 0;  // read: this lane's in chunk 0, and per chunk
+  if (tid == 0) {
+    rs[SLOTS] = u32x4{0x3f803f80u, 0x00003f80u, 0u, 0u};
+#pragma unroll
+    for (int v = 0; v < NV; v++) rv[v][SLOTS] = u32x4{0u, 0u, 0u, 0u};
+  }
 
   for (int64_t tile = tile_begin; tile < tile_end; tile++) {
     const float4* src = packed + tile * (TILE * Q);
     float rec[R];
 #pragma unroll
-    for (int q = 0; q < Q; q++) {
-      if (DXU && q == 2) continue;  // the residuals: read only by near waves
+    for (int q = 0; q <= (L::LO - 1) / 4; q++) {  // the residuals only where they share a word with the rest
       const float4 v = src[tid * Q + q];
       rec[4 * q] = v.x;
       rec[4 * q + 1] = v.y;
@@ -612,14 +633,24 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
     const double cg = g == 0 ? m.x : (g == 1 ? m.y : m.z);
     __syncthreads();  // the previous tile's readers
 #pragma unroll
-    for (int k = 0; k < 3; k++) rs[(tid >> 4) * 64 + 16 * k + (tid & 15)] = row_slots(-2.0f * rec[k]);
-    sS[tid] = rec[3];
-    if constexpr (DXU) {
+    for (int k = 0; k < 3; k++) rs[slot + 16 * k] = row_slots(-2.0f * rec[k]);
+    if constexpr (LAP) sS[tid] = rec[3];
+    else sS[tid] = (float)((double)rec[0] * rec[0] + (double)rec[1] * rec[1] + (double)rec[2] * rec[2]);
 #pragma unroll
-      for (int k = 0; k < 3; k++) rn[(tid >> 4) * 64 + 16 * k + (tid & 15)] = row_slots(tid & 1 ? -rec[4 + k] : rec[4 + k]);
-      sn[tid] = tid & 1 ? -rec[7] : rec[7];
+    for (int v = 0; v < NV; v++) {
+      const float* x = rec + (KER == LAP_DXU ? 4 : 3 + 3 * v);
+      const float c = KER == LAP_DXU
+                          ? rec[7]
+                          : (float)-((double)rec[0] * x[0] + (double)rec[1] * x[1] + (double)rec[2] * x[2]);
+#pragma unroll
+      for (int k = 0; k < 3; k++) rv[v][slot + 16 * k] = row_slots(tid & 1 ? -x[k] : x[k]);
+      sv[v][tid] = tid & 1 ? -c : c;
+    }
+    if constexpr (KER == LAP_FXU) {
+      srow[0][tid] = rec[4];
     } else {
-      sq[tid] = rec[4];
+#pragma unroll
+      for (int k = 0; k < NROW; k++) srow[k][tid] = rec[k];  // s', then the densities from FOFF = 3
     }
     __syncthreads();
 
@@ -632,34 +663,45 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
       const float Tj = __shfl(T, 16 * j + c16, 64);
       col[j] = column_slots(g < 3 ? (float)(tg[j] - cg) : Tj);
     }
-    float pf[GROUPS], pn[1] = {0.0f};
-    double ptn = 0.0;
+    float pf[GROUPS][K1], pG[GROUPS], pn[K1];
+    double ptn[K1];
 #pragma unroll
-    for (int j = 0; j < GROUPS; j++) pf[j] = 0.0f;
+    for (int j = 0; j < GROUPS; j++) pG[j] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < K1; k++) {
+      pn[k] = 0.0f;
+      ptn[k] = 0.0;
+#pragma unroll
+      for (int j = 0; j < GROUPS; j++) pf[j][k] = 0.0f;
+    }
     auto far = [&](int ch0, auto count) {
-#pragma unroll 4
+#pragma unroll (far_unroll<KER>())
       for (int ch = ch0; ch < ch0 + decltype(count)::value; ch++) {
-        const u32x4 a = rs[ch * 64 + lane];
-        const f32x4 S4 = *reinterpret_cast<const f32x4*>(sS + ch * 16 + 4 * g);
-        if constexpr (DXU) {
-          const u32x4 an = rn[ch * 64 + lane];
-          const f32x4 n4 = *reinterpret_cast<const f32x4*>(sn + ch * 16 + 4 * g);
+        auto four = [&](const float* a) { return *reinterpret_cast<const f32x4*>(a + ch * 16 + 4 * g); };
+        const int at = my_slot + ch * my_step;
+        const u32x4 a = rs[at];
+        const f32x4 S4 = four(sS);
+        u32x4 av[NV ? NV : 1];
+        f32x4 v4[NV ? NV : 1], w4[NROW ? NROW : 1];
 #pragma unroll
-          for (int j = 0; j < GROUPS; j++) {
-            const f32x4 r2 = mfma16(a, col[j], S4), rnq = mfma16(an, col[j], n4);
+        for (int v = 0; v < NV; v++) {
+          av[v] = rv[v][at];
+          v4[v] = four(sv[v]);
+        }
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-              const float z = rsq_deferred<NEWTON>(r2[i]);
-              pf[j] = fmad((i & 1 ? -rnq[i] : rnq[i]) * z, z * z, pf[j]);
-            }
-          }
-        } else {
-          const f32x4 f4 = *reinterpret_cast<const f32x4*>(sq + ch * 16 + 4 * g);
+        for (int k = 0; k < NROW; k++) w4[k] = four(srow[k]);
 #pragma unroll
-          for (int j = 0; j < GROUPS; j++) {
-            const f32x4 r2 = mfma16(a, col[j], S4);
+        for (int j = 0; j < GROUPS; j++) {
+          const f32x4 r2 = mfma16(a, col[j], S4);
+          f32x4 dots[NV ? NV : 1];
 #pragma unroll
-            for (int i = 0; i < 4; i++) pf[j] = fmad(rsq_deferred<NEWTON>(r2[i]), f4[i], pf[j]);
+          for (int v = 0; v < NV; v++) dots[v] = mfma16(av[v], col[j], v4[v]);
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            float d[NV ? NV : 1];
+#pragma unroll
+            for (int v = 0; v < NV; v++) d[v] = i & 1 ? -dots[v][i] : dots[v][i];
+            far_pair<KER, NEWTON>(pf[j], pG[j], r2[i], d, [&](int k) { return w4[k][i]; });
           }
         }
       }
@@ -675,15 +717,18 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
         wave_sync();
         const float* recs = reinterpret_cast<const float*>(nst);
         if (near) {
-#pragma unroll 2
+#pragma unroll (lane_unroll<KER>())
           for (int i = 0; i < NEAR_ST; i++) mix_near<KER, NEWTON>(pn, th, tl, recs + i * R, 0.0f);
         } else {
-#pragma unroll 4
-          for (int i = 0; i < NEAR_ST; i++) mix_mid<KER, NEWTON>(pn, th, recs + i * R);
+#pragma unroll (lane_unroll<KER>())
+          for (int i = 0; i < NEAR_ST; i++) mix_mid<KER, NEWTON>(pn, th, recs + i * R, 0.0f);
         }
       }
-      ptn += (double)pn[0];
-      pn[0] = 0.0f;
+#pragma unroll
+      for (int k = 0; k < K1; k++) {
+        ptn[k] += (double)pn[k];
+        pn[k] = 0.0f;
+      }
     };
     const bool tiny = __builtin_amdgcn_ballot_w64(T < MFMA_MIN_T) != 0;
     if (__builtin_amdgcn_ballot_w64(T < 9.0f * H2) == 0 && !tiny) {
@@ -702,33 +747,58 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
         else by_lane(q * 64, __builtin_amdgcn_ballot_w64(d2 < em * em) != 0);
       }
     }
-    bool bad = !__builtin_isfinite(ptn);
+    bool bad = false;
 #pragma unroll
-    for (int j = 0; j < GROUPS; j++) bad |= !__builtin_isfinite(pf[j]);
+    for (int k = 0; k < K1; k++) {
+      bad |= !__builtin_isfinite(ptn[k]);
+#pragma unroll
+      for (int j = 0; j < GROUPS; j++) bad |= !__builtin_isfinite(pf[j][k]);
+    }
+    if constexpr (F::GRAD) {
+#pragma unroll
+      for (int j = 0; j < GROUPS; j++) bad |= !__builtin_isfinite(pG[j]);
+    }
     if (__builtin_amdgcn_ballot_w64(bad) != 0) {  // the whole tile in the near form
 #pragma unroll
-      for (int j = 0; j < GROUPS; j++) pf[j] = 0.0f;
-      ptn = 0.0;
+      for (int k = 0; k < K1; k++) {
+        ptn[k] = 0.0;
+        pn[k] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < GROUPS; j++) pf[j][k] = 0.0f;
+      }
+#pragma unroll
+      for (int j = 0; j < GROUPS; j++) pG[j] = 0.0f;
       for (int q = 0; q < TILE / 64; q++) by_lane(q * 64, true);
     }
-    accn += ptn;
 #pragma unroll
-    for (int j = 0; j < GROUPS; j++) accf[j] += (double)pf[j];
+    for (int k = 0; k < K1; k++) {
+      accn[k] += ptn[k];
+#pragma unroll
+      for (int j = 0; j < GROUPS; j++) {
+        if constexpr (F::GRAD)
+          accf[j][k] += fmad((double)__shfl(th[k], 16 * j + c16, 64), (double)pG[j], (double)pf[j][k]);
+        else accf[j][k] += (double)pf[j][k];
+      }
+    }
   }
 
   // Target 16 j + c16's far sums: over the four lane groups, to the lane of that target.
-  double v = accn;
-#pragma unroll
-  for (int j = 0; j < GROUPS; j++) {
-    double f = accf[j];
-    f += __shfl_xor(f, 16, 64);
-    f += __shfl_xor(f, 32, 64);
-    if (g == j) v += f;
-  }
   const int64_t q = q0 + lane;
-  if (q < nt) {
-    if (direct) out[tperm[q]] += v * scale;
-    else out[wg.split * nt + q] = v;
+  const int64_t t = direct && q < nt ? (int64_t)tperm[q] : 0;
+#pragma unroll
+  for (int k = 0; k < K1; k++) {
+    double v = accn[k];
+#pragma unroll
+    for (int j = 0; j < GROUPS; j++) {
+      double f = accf[j][k];
+      f += __shfl_xor(f, 16, 64);
+      f += __shfl_xor(f, 32, 64);
+      if (g == j) v += f;
+    }
+    if (q < nt) {
+      if (direct) out[t * K1 + k] += v * scale;
+      else out[wg.split * nt * K1 + q * K1 + k] = v;
+    }
   }
 }
 
@@ -753,20 +823,24 @@ using PackFn = void (*)(const double*, const double*, const double*, int64_t, co
 constexpr int TPLS[3] = {1, 2, 4};
 int tpl_index(int tpl) { return tpl >= 4 ? 2 : (tpl >= 2 ? 1 : 0); }
 
-// Targets per lane of the mixed kernels (the matrix-core ones have one form).
-template <int KER> constexpr int mixed_max_tpl() { return far_mfma<KER>() ? 1 : max_tpl<KER>(); }
-
-template <int KER, int NEWTON> EvalMixFn mix_fn(int ti) {
-  if constexpr (far_mfma<KER>()) return k_eval_mixed_mfma<KER, NEWTON>;
-  constexpr int MT = max_tpl<KER>();
-  if (ti >= 2 && MT >= 4) return k_eval_mixed<KER, (MT >= 4 ? 4 : 1), NEWTON>;
-  if (ti >= 1 && MT >= 2) return k_eval_mixed<KER, (MT >= 2 ? 2 : 1), NEWTON>;
-  return k_eval_mixed<KER, 1, NEWTON>;
+// ti: targets per lane (the matrix-core kernels have one form; the Laplace
+// single and double layer have no other).
+template <int KER, int NEWTON> EvalMixFn mix_fn(int ti, bool mfma) {
+  if constexpr (far_mfma<KER>()) {
+    if (mfma || KER == LAP_FXU || KER == LAP_DXU) return k_eval_mixed_mfma<KER, NEWTON>;
+  }
+  if constexpr (KER != LAP_FXU && KER != LAP_DXU) {
+    constexpr int MT = max_tpl<KER>();
+    if (ti >= 2 && MT >= 4) return k_eval_mixed<KER, (MT >= 4 ? 4 : 1), NEWTON>;
+    if (ti >= 1 && MT >= 2) return k_eval_mixed<KER, (MT >= 2 ? 2 : 1), NEWTON>;
+    return k_eval_mixed<KER, 1, NEWTON>;
+  }
+  return nullptr;  // not reached
 }
-EvalMixFn mix_fn(int ker, int newton, int ti) {
+EvalMixFn mix_fn(int ker, int newton, int ti, bool mfma) {
   return with_kernel(ker, [&](auto kc) -> EvalMixFn {
     constexpr int K = decltype(kc)::value;
-    return newton ? mix_fn<K, 1>(ti) : mix_fn<K, 0>(ti);
+    return newton ? mix_fn<K, 1>(ti, mfma) : mix_fn<K, 0>(ti, mfma);
   });
 }
 PackFn pack_fn(int ker) {
@@ -776,7 +850,7 @@ int layout_q(int ker) {
   return with_kernel(ker, [](auto kc) { return MixLayout<decltype(kc)::value>::Q; });
 }
 int max_tpl_index(int ker) {
-  return with_kernel(ker, [](auto kc) { return tpl_index(mixed_max_tpl<decltype(kc)::value>()); });
+  return with_kernel(ker, [](auto kc) { return tpl_index(max_tpl<decltype(kc)::value>()); });
 }
 
 }  // namespace
@@ -801,6 +875,27 @@ bool mixed_runs_f64(int ker, int64_t nt, int64_t ns) {
   return pairs <= (needs_ctx(ker) ? 6e7 : (K1 > 4 ? 2e7 : 4.2e7));
 }
 
+// Whether a mixed Eval of this size takes the matrix-core kernel.  The Laplace
+// single and double layer always do.  The kernels with three outputs run three
+// waves per SIMD in it, which their near pairs pay for: a gain only where far
+// tiles prevail.  Dense plan applies, FP32 form / matrix cores, us:
+//                    20000^2 cube   50000^2 cube  90000^2 cube  131072 x 150001  262144^2
+//                                                               clusters         sphere
+//   Stokes FxU       194 / 224      992 / 1039    3025 / 3050   7210 / 6698      24922 / 22008
+//   Stokes DxU       216 / 237      1131 / 1101   3512 / 3238   8521 / 7092      29523 / 23279
+//   Laplace FxdU     149 / 171      741 / 783     2261 / 2239   5367 / 4784      18542 / 15704
+bool far_mfma_at(int ker, int64_t nt, int64_t ns) {
+  const double pairs = (double)nt * (double)ns;
+  switch (ker) {
+    case LAP_FXU:
+    case LAP_DXU: return true;
+    case STK_DXU: return pairs >= 3e9;
+    case STK_FXU: return pairs >= 1e10;
+    case LAP_FXDU: return pairs >= 8e9;
+    default: return false;
+  }
+}
+
 // Launch geometry of one mixed Eval: target blocks and the source splits.
 // Split the sources over gridDim.y when the target blocks cannot fill the
 // device (>= 8 workgroups per CU, each split >= 4 tiles), and so that no
@@ -813,7 +908,8 @@ int mixed_geometry(int ker, int64_t nt, int64_t ns, const DenseShape& shape, Mix
   DeviceInfo dev;
   SCTL_TRY(device_info(&dev));
   SCTL_CHECK_ARG(ns <= 0xffffffffLL && nt <= 0xffffffffLL, "mixed precision supports at most 2^32-1 points");
-  g->ti = std::min(tpl_index(shape.tpl), max_tpl_index(ker));
+  g->mfma = far_mfma_at(ker, nt, ns);
+  g->ti = g->mfma ? 0 : std::min(tpl_index(shape.tpl), max_tpl_index(ker));
   const int tpl = TPLS[g->ti];
   g->tb = (nt + (int64_t)WG * tpl - 1) / ((int64_t)WG * tpl);
   SCTL_CHECK_ARG(g->tb <= 0x7fffffffLL, "too many targets for one launch");
@@ -869,7 +965,7 @@ int mixed_apply(int ker, int newton, const MixedGeometry& g, const DenseShape& s
                      v_src, ns, sperm, packed, meta, sub, g.ntiles, r_trg, nt, tperm, xt_sorted);
   SCTL_HIP_TRY(hipGetLastError());
   const double scale = (double)(kernel_scale(ker) * fold_factor(ker, newton ? 1 : 0));
-  const EvalMixFn fn = mix_fn(ker, newton, g.ti);
+  const EvalMixFn fn = mix_fn(ker, newton, g.ti, g.mfma);
   size_t dyn = 0;
   SCTL_TRY(occupancy_lds((const void*)fn, shape.occ, sizeof(float4) * TILE * g.Q, &dyn));
   if (!stream_capturing(stream)) profile_count(ker, nt * ns);

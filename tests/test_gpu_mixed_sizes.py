@@ -71,3 +71,29 @@ def test_both_sides(gpu, k, shape, where):
         gpu.synchronize()
         # the split partial sums may come in other groups: FP64 rounding of the groups' sums
         assert np.abs(o.download() - out).max() <= 1e-12 * max(np.abs(out).max(), magnitude(k, *a))
+
+
+@pytest.mark.parametrize("shape", [(100003, 100001), (5003, 2000003), (1500001, 7001)],
+                         ids=["square", "few-targets", "few-sources"])
+@pytest.mark.parametrize("k", [2, 3, 4])
+def test_large_three_outputs(gpu, k, shape):
+    """The sizes from which the Stokes layers and the Laplace gradient form their far pairs on the matrix cores:
+    against the FP64 Eval (held to the oracle elsewhere), clustered points with coincident ones, with and without
+    the FP32 Newton step.  1e-6 normwise, the mixed bar."""
+    nt, ns = shape
+    rng = np.random.default_rng(nt + k)
+    _, K0, K1, _, _ = oracle.dims(k)
+    c = rng.random((64, 3))
+    xs, xt = (c[rng.integers(0, 64, m)] + 0.05 * rng.standard_normal((m, 3)) for m in (ns, nt))
+    xt[:37] = xs[ns - 37:]
+    n, v = rng.standard_normal(3 * ns), rng.uniform(-1, 1, K0 * ns)
+    d = [gpu.DeviceArray.from_host(a.ravel()) for a in (xt, xs, n, v)]
+    res = []
+    for prec, flags in ((gpu.FP64, 0), (gpu.MIXED, 0), (gpu.MIXED, gpu.MIXED_NEWTON)):
+        o = gpu.DeviceArray.from_host(np.zeros(nt * K1))
+        gpu.eval(k, d[0], d[1], d[2], d[3], o, precision=prec, flags=flags)
+        gpu.synchronize()
+        res.append(o.download())
+    for out in res[1:]:
+        assert np.isfinite(out).all()
+        assert np.abs(out - res[0]).max() <= 1e-6 * np.abs(res[0]).max()
