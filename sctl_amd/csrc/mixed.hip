@@ -16,15 +16,17 @@
 //   mid  -- every pair has r >= H: dx = t' - s'.
 //   near -- positions are differenced from both halves, dx = (t' - s') +
 //           (t'' - s''), which is accurate to about 2^-23 relative to dx
-//           however small r is, and r^2 == 0 is masked as in the reference
-//           (kernel_functions.hpp:45).
+//           however small r is.  A pair with r^2 == 0 makes the tile's sum
+//           non-finite, and the tile is redone with r^2 == 0 masked as in the
+//           reference (kernel_functions.hpp:45): the mask on every near pair
+//           took 3 % of a 20 000 x 20 000 cube's apply (115.7 -> 112.4 us).
 // Targets in Hilbert order keep a wave's targets together, so only tiles next
 // to the wave take the near loop.  The pairs of every 64 sources are summed
 // in FP32 and added into an FP64 sum of the tile, so that a tile's largest
 // term does not take up the rounding of 255 FP32 additions (this halved the
 // headline's error against FP64, 5.4e-7 -> 2.7e-7, at no cost in time).  A
-// tile whose sum is not finite is redone by the near loop.  The tiles' sums are
-// added up in FP64 per target.
+// tile whose sum is not finite is redone by the masked near loop.  The tiles'
+// sums are added up in FP64 per target.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -109,8 +111,9 @@ __device__ __forceinline__ void mix_mid(float* p, const float* th, const float* 
   }
 }
 
-// Near-field interaction: two-part differencing, r^2 == 0 masked.
-template <int KER, int NEWTON>
+// Near-field interaction: two-part differencing.  MASK: r^2 == 0 contributes 0;
+// without it such a pair makes the sum non-finite, and its tile is redone.
+template <int KER, int NEWTON, bool MASK>
 __device__ __forceinline__ void mix_near(float* p, const float* th, const float* tl, const float* r, float mu) {
   constexpr int LO = MixLayout<KER>::LO;
   const float dx = (th[0] - r[0]) + (tl[0] - r[LO + 0]);
@@ -118,13 +121,13 @@ __device__ __forceinline__ void mix_near(float* p, const float* th, const float*
   const float dz = (th[2] - r[2]) + (tl[2] - r[LO + 2]);
   if constexpr (KER == LAP_FXU) {
     const float f[1] = {r[4]};
-    interact<LAP_FXU, NEWTON, true>(p, dx, dy, dz, f, f);
+    interact<LAP_FXU, NEWTON, MASK>(p, dx, dy, dz, f, f);
   } else if constexpr (KER == LAP_DXU) {
     const float one[1] = {1.0f}, nq[3] = {r[4], r[5], r[6]};
-    interact<LAP_DXU, NEWTON, true>(p, dx, dy, dz, nq, one);
+    interact<LAP_DXU, NEWTON, MASK>(p, dx, dy, dz, nq, one);
   } else {
     using L = MixLayout<KER>;
-    interact<KER, NEWTON, true>(p, dx, dy, dz, r + L::NOFF, r + L::FOFF, mu);
+    interact<KER, NEWTON, MASK>(p, dx, dy, dz, r + L::NOFF, r + L::FOFF, mu);
   }
 }
 
@@ -352,7 +355,7 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
 #pragma unroll 2
           for (int i = 0; i < 64; i++) {
 #pragma unroll
-            for (int j = 0; j < TPL; j++) mix_near<KER, NEWTON>(p[j], th[j], tl[j], qrec + i * R, mu);
+            for (int j = 0; j < TPL; j++) mix_near<KER, NEWTON, false>(p[j], th[j], tl[j], qrec + i * R, mu);
           }
         } else {
 #pragma unroll 4
@@ -390,7 +393,7 @@ k_eval_mixed(const double* __restrict__ xt, int64_t nt, const uint32_t* __restri
         for (int i = i0; i < i0 + 64; i++) {
           const float* rec = recs + i * R;
 #pragma unroll
-          for (int j = 0; j < TPL; j++) mix_near<KER, NEWTON>(p[j], th[j], tl[j], rec, mu);
+          for (int j = 0; j < TPL; j++) mix_near<KER, NEWTON, true>(p[j], th[j], tl[j], rec, mu);
         }
         sub64();
       }
@@ -566,7 +569,7 @@ __device__ __forceinline__ void far_pair(float* p, float& G, float r2, const flo
 template <int KER> constexpr int mfma_waves() { return Ker<KER>::K1 == 1 ? 4 : 3; }
 // Chunks and sources unrolled, from sweeps of 1, 2 and 4 resp. 2, 4 and 8.
 template <int KER> constexpr int far_unroll() { return Ker<KER>::K1 == 1 ? 4 : (KER == STK_FXU ? 2 : 1); }
-template <int KER> constexpr int lane_unroll() { return KER == STK_FXU || KER == STK_DXU ? 2 : 4; }
+template <int KER> constexpr int lane_unroll() { return KER == LAP_FXU || KER == LAP_FXDU ? 4 : 2; }
 template <int KER, int NEWTON>
 __global__ void __launch_bounds__(WG, (mfma_waves<KER>()))
 k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __restrict__ tperm,
@@ -707,7 +710,8 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
       }
     };
     // Sub-tile sq0 / 64 with one target per lane: the mid form, or the near form.
-    auto by_lane = [&](int sq0, bool near) {
+    // (near: 0 mid, 1 near, 2 near with r^2 == 0 masked)
+    auto by_lane = [&](int sq0, int near) {
       const float tl[3] = {(float)((t64[0] - m.x) - (double)th[0]), (float)((t64[1] - m.y) - (double)th[1]),
                            (float)((t64[2] - m.z) - (double)th[2])};
 #pragma unroll 1
@@ -716,9 +720,12 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
         for (int i = lane; i < NEAR_ST * Q; i += 64) nst[i] = src[s0 * Q + i];
         wave_sync();
         const float* recs = reinterpret_cast<const float*>(nst);
-        if (near) {
+        if (near == 2) {
+#pragma unroll 1
+          for (int i = 0; i < NEAR_ST; i++) mix_near<KER, NEWTON, true>(pn, th, tl, recs + i * R, 0.0f);
+        } else if (near) {
 #pragma unroll (lane_unroll<KER>())
-          for (int i = 0; i < NEAR_ST; i++) mix_near<KER, NEWTON>(pn, th, tl, recs + i * R, 0.0f);
+          for (int i = 0; i < NEAR_ST; i++) mix_near<KER, NEWTON, false>(pn, th, tl, recs + i * R, 0.0f);
         } else {
 #pragma unroll (lane_unroll<KER>())
           for (int i = 0; i < NEAR_ST; i++) mix_mid<KER, NEWTON>(pn, th, recs + i * R, 0.0f);
@@ -744,7 +751,7 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
         const float ef = fmad(0.5f, X, h), em = fmad(1.0f / 3.0f, X, h);
         if (__builtin_amdgcn_ballot_w64(d2 < ef * ef) == 0 && !tiny)
           far(q * (CHUNKS / 4), std::integral_constant<int, CHUNKS / 4>());
-        else by_lane(q * 64, __builtin_amdgcn_ballot_w64(d2 < em * em) != 0);
+        else by_lane(q * 64, __builtin_amdgcn_ballot_w64(d2 < em * em) != 0 ? 1 : 0);
       }
     }
     bool bad = false;
@@ -768,7 +775,7 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
       }
 #pragma unroll
       for (int j = 0; j < GROUPS; j++) pG[j] = 0.0f;
-      for (int q = 0; q < TILE / 64; q++) by_lane(q * 64, true);
+      for (int q = 0; q < TILE / 64; q++) by_lane(q * 64, 2);
     }
 #pragma unroll
     for (int k = 0; k < K1; k++) {
