@@ -52,8 +52,7 @@ namespace {
 
 constexpr int NWG = 256;        // 4 independent waves per workgroup
 constexpr int MAT_ST = 16;      // targets per near-matrix stripe (one wave)
-constexpr int GEMV_ROWS = 16;   // rows per GEMV wave tile
-constexpr int GEMV_GR = 8;      // GEMV rows walked together
+constexpr int GEMV_GR = 8;      // rows per GEMV wave tile, walked together
 constexpr int NEAR_NEWTON = 2;  // KernelMatrix at digits -1 (boundary_integral.txx:1197,1211)
 
 __device__ __forceinline__ void wave_sync() {
@@ -96,17 +95,17 @@ struct Row {
   int a;
 };
 
-// Row k of target t (dof rows per target) of a stripe of nts targets; the
-// rows of targets past the stripe get extent 0.
-__device__ __forceinline__ Row row_of(double* Ks, int t, int nts, int64_t ld, int dof = 1, int k = 0) {
+// Row k of target t (dof rows per target) of a stripe of nts targets, `len`
+// entries of it from Ks on; the rows of targets past the stripe get extent 0.
+__device__ __forceinline__ Row row_of(double* Ks, int t, int nts, int64_t ld, int len, int dof = 1, int k = 0) {
   // Built where it is used: kept opaque so that the resources of all rows
   // are not hoisted out of the caller's loop (64 scalar registers).
   uint64_t base = reinterpret_cast<uint64_t>(Ks);
-  asm volatile("" : "+s"(base), "+s"(ld), "+s"(nts));
+  asm volatile("" : "+s"(base), "+s"(ld), "+s"(nts), "+s"(len));
   double* p = reinterpret_cast<double*>(base) + ((int64_t)min(t, nts - 1) * dof + k) * ld;
   Row R;
   R.a = (int)((reinterpret_cast<uintptr_t>(p) >> 3) & 15);
-  R.rsrc = __builtin_amdgcn_make_buffer_rsrc(p, 0, t < nts ? (int)(ld * 8) : 0, 0x00020000);
+  R.rsrc = __builtin_amdgcn_make_buffer_rsrc(p, 0, t < nts ? len * 8 : 0, 0x00020000);
   return R;
 }
 
@@ -122,8 +121,8 @@ __device__ __forceinline__ double buffer_load_d(__amdgpu_buffer_rsrc_t r, int of
 
 // KNearSubtract / store of one layout's blocks.  NDOT: contract the KDIM1
 // outputs with the target normal (KDIM1 == 3 -> one row per target).
-// A wave owns one stripe (MAT_ST targets x all sources of a block), a
-// contiguous range of K_near: lanes 0..MAT_ST-1 hold the stripe's targets,
+// A wave owns one stripe (MAT_ST targets x the block's sources, or a piece of
+// them where one stripe would outlast the others' work: near_tiles): lanes 0..MAT_ST-1 hold the stripe's targets,
 // the wave walks the sources 64 at a time (one per lane) and, per chunk,
 // writes every target row's 64*KDIM0 entries.
 //
@@ -152,7 +151,8 @@ __device__ __forceinline__ double buffer_load_d(__amdgpu_buffer_rsrc_t r, int of
 // store before each load.
 template <int KER, bool NDOT, bool SUB>
 __global__ void __launch_bounds__(NWG)
-k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ tile_dsp, int64_t ntiles,
+k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ tile_dsp,
+              const int32_t* __restrict__ tile_piece, int64_t ntiles,
               const int64_t* __restrict__ trg_dsp, const int32_t* __restrict__ trg_cnt,
               const int64_t* __restrict__ src_dsp, const int32_t* __restrict__ src_cnt,
               const int64_t* __restrict__ mat_off, const double* __restrict__ xt, const double* __restrict__ n_trg,
@@ -177,8 +177,11 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
   const int64_t first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (NWG / 64) + (threadIdx.x >> 6)));
   for (int64_t tile = first; tile < ntiles; tile += nwaves) {
     const int b = __builtin_amdgcn_readfirstlane(tile_blk[tile]);
-    const int t0 = (int)(tile - tile_dsp[b]) * MAT_ST;
-    const int sc = src_cnt[b];
+    // Piece pc of the stripe's columns: sources [s_first, s_first + sc), a
+    // matrix of its own with the block's row stride.
+    const int all = src_cnt[b], piece = tile_piece[b], npc = (all + piece - 1) / piece;
+    const int local = (int)(tile - tile_dsp[b]), stripe = local / npc, s_first = (local - stripe * npc) * piece;
+    const int t0 = stripe * MAT_ST, sc = min(piece, all - s_first);
     const int nts = min(MAT_ST, trg_cnt[b] - t0);
     // The stripe's targets (and normals) in the wave's LDS slot, read back per
     // row by broadcast (one address for the whole wave): no VALU work per row
@@ -195,9 +198,10 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
     }
     wave_sync();
     const double* tx = tslot;
-    const int64_t ld = (int64_t)sc * K0;
-    double* Ks = uniform_ptr(K + mat_off[b] + (int64_t)t0 * DOF * ld);
-    const int64_t sb = src_dsp[b];
+    const int64_t ld = (int64_t)all * K0;
+    const int len = sc * K0;  // entries of a row in this piece
+    double* Ks = uniform_ptr(K + mat_off[b] + (int64_t)t0 * DOF * ld + (int64_t)s_first * K0);
+    const int64_t sb = src_dsp[b] + s_first;
     // This lane's source record of the chunk at s0: position, normal, weight
     // (the column clamped to the block's last source).
     auto load = [&](int s0, double(&r)[7]) {
@@ -292,7 +296,7 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
         if constexpr (SUB) {
 #pragma unroll
           for (int t = 0; t < MAT_ST; t++) {
-            const Row R = row_of(Ks, t, nts, ld);
+            const Row R = row_of(Ks, t, nts, ld, len);
             old[t] = buffer_load_d(R.rsrc, (s0 - R.a + lane) * 8);
           }
         }
@@ -301,7 +305,7 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
           // per-row values derived here, not kept across the chunk loop
           int nr = nts;
           asm volatile("" : "+s"(nr));
-          const Row R = row_of(Ks, t, nr, ld);
+          const Row R = row_of(Ks, t, nr, ld, len);
           const double v = tail ? 0.0 : value1(min(t, nr - 1), cur, ws);
           const double rot = bpermute_d(v, ((lane - R.a) & 63) << 2);
           const double prev = cs[t * 16 + (lane & 15)];
@@ -366,7 +370,7 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
           }
 #pragma unroll
           for (int k1 = 0; k1 < DOF; k1++) {
-            const Row R = row_of(Ks, t, nr, ld, DOF, k1);
+            const Row R = row_of(Ks, t, nr, ld, len, DOF, k1);
             double* cr = cw + (t * DOF + k1) * 16;
 #pragma unroll
             for (int k0 = 0; k0 < K0; k0++) stg[lane * K0 + k0] = e[k1][k0];
@@ -416,9 +420,9 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
 
 // U_near[block rows] = K_near_ * F_element.  Blocks without a matrix
 // (offset < 0) or without sources get zero rows, as the reference's GEMV loop
-// writes them (boundary_integral.txx:1329-1332).  A wave owns GEMV_ROWS
-// consecutive rows (a contiguous range of K_near) and walks them GEMV_GR at a
-// time with its 64 lanes along the rows: every load is 64 consecutive
+// writes them (boundary_integral.txx:1329-1332).  A wave owns GEMV_GR
+// consecutive rows, or a piece of their columns (near_tiles), with its 64
+// lanes along the rows: every load is 64 consecutive
 // entries of one row, each lane's F entries serve all GEMV_GR rows, and two
 // column chunks per step keep 2*GEMV_GR loads in flight.  Rows past the
 // block's last (a tail tile) re-read its last row and columns past the row
@@ -426,68 +430,85 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
 // the block and no load is predicated.  The GEMV_GR row sums are reduced
 // across the wave by a halving butterfly: each exchange hands half of the
 // rows still held to the partner lane (4 + 2 + 1 + 3 exchanges for 8 rows).
+// Rows whose columns are cut leave partial sums for k_near_gemv_sum.
 __global__ void __launch_bounds__(NWG)
-k_near_gemv(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ tile_dsp, int64_t ntiles,
+k_near_gemv(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ tile_dsp,
+            const int32_t* __restrict__ tile_piece, int64_t ntiles,
             const int64_t* __restrict__ trg_dsp, const int32_t* __restrict__ trg_cnt,
             const int64_t* __restrict__ src_dsp, const int32_t* __restrict__ src_cnt,
             const int64_t* __restrict__ mat_off, int K0, int dof, const double* __restrict__ K,
-            const double* __restrict__ F, double* __restrict__ U) {
-  static_assert(GEMV_GR == 8 && GEMV_ROWS % GEMV_GR == 0, "the butterfly below reduces 8 rows");
+            const double* __restrict__ F, double* __restrict__ U, const int64_t* __restrict__ part_dsp,
+            double* __restrict__ part) {
+  static_assert(GEMV_GR == 8, "the butterfly below reduces 8 rows");
   const int lane = threadIdx.x & 63;
   const int64_t nwaves = (int64_t)gridDim.x * (NWG / 64);
   const int64_t first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (NWG / 64) + (threadIdx.x >> 6)));
   for (int64_t tile = first; tile < ntiles; tile += nwaves) {
     const int b = __builtin_amdgcn_readfirstlane(tile_blk[tile]);
-    const int64_t local = tile - tile_dsp[b];
     const int64_t rows = (int64_t)trg_cnt[b] * dof;
     const int64_t ld = (int64_t)src_cnt[b] * K0;
     const int64_t off = mat_off[b];
+    const int piece = tile_piece[b];
+    const int npc = (int)max((int64_t)1, (ld + piece - 1) / piece);
+    const int64_t local = tile - tile_dsp[b];
+    const int64_t row0 = local / npc * GEMV_GR, c0 = (local - local / npc * npc) * piece;
+    const int64_t c1 = min(c0 + piece, ld);
     const double* Fb = F + src_dsp[b] * K0;
-    double* Ub = U + trg_dsp[b] * dof;
-    for (int rr = 0; rr < GEMV_ROWS; rr += GEMV_GR) {
-      const int64_t row0 = local * GEMV_ROWS + rr;
-      if (row0 >= rows) break;
-      const int64_t nr = min((int64_t)GEMV_GR, rows - row0);
-      double acc[GEMV_GR];
+    const int64_t nr = min((int64_t)GEMV_GR, rows - row0);
+    double acc[GEMV_GR];
 #pragma unroll
-      for (int r = 0; r < GEMV_GR; r++) acc[r] = 0.0;
-      if (off >= 0) {
-        const double* Kr = K + off + row0 * ld;
-        for (int64_t j0 = 0; j0 < ld; j0 += 128) {
-          const int64_t ja = j0 + lane, jb = ja + 64;
-          const int64_t ca = min(ja, ld - 1), cb = min(jb, ld - 1);
-          const double fa = ja < ld ? Fb[ca] : 0.0, fb = jb < ld ? Fb[cb] : 0.0;
-          double ka[GEMV_GR], kb[GEMV_GR];
+    for (int r = 0; r < GEMV_GR; r++) acc[r] = 0.0;
+    if (off >= 0) {
+      const double* Kr = K + off + row0 * ld;
+      for (int64_t j0 = c0; j0 < c1; j0 += 128) {
+        const int64_t ja = j0 + lane, jb = ja + 64;
+        const int64_t ca = min(ja, c1 - 1), cb = min(jb, c1 - 1);
+        const double fa = ja < c1 ? Fb[ca] : 0.0, fb = jb < c1 ? Fb[cb] : 0.0;
+        double ka[GEMV_GR], kb[GEMV_GR];
 #pragma unroll
-          for (int r = 0; r < GEMV_GR; r++) {
-            const double* Kq = Kr + min((int64_t)r, nr - 1) * ld;
-            ka[r] = Kq[ca];
-            kb[r] = Kq[cb];
-          }
+        for (int r = 0; r < GEMV_GR; r++) {
+          const double* Kq = Kr + min((int64_t)r, nr - 1) * ld;
+          ka[r] = Kq[ca];
+          kb[r] = Kq[cb];
+        }
 #pragma unroll
-          for (int r = 0; r < GEMV_GR; r++) {
-            ka[r] = ja < ld ? ka[r] : 0.0;
-            kb[r] = jb < ld ? kb[r] : 0.0;
-            acc[r] = fmad(kb[r], fb, fmad(ka[r], fa, acc[r]));
-          }
+        for (int r = 0; r < GEMV_GR; r++) {
+          ka[r] = ja < c1 ? ka[r] : 0.0;
+          kb[r] = jb < c1 ? kb[r] : 0.0;
+          acc[r] = fmad(kb[r], fb, fmad(ka[r], fa, acc[r]));
         }
       }
+    }
 #pragma unroll
-      for (int h = GEMV_GR / 2, m = 32; h >= 1; h >>= 1, m >>= 1) {
-        const bool up = lane & m;
+    for (int h = GEMV_GR / 2, m = 32; h >= 1; h >>= 1, m >>= 1) {
+      const bool up = lane & m;
 #pragma unroll
-        for (int i = 0; i < h; i++) {
-          const double send = up ? acc[i] : acc[i + h];
-          const double keep = up ? acc[i + h] : acc[i];
-          acc[i] = keep + __shfl_xor(send, m, 64);
-        }
+      for (int i = 0; i < h; i++) {
+        const double send = up ? acc[i] : acc[i + h];
+        const double keep = up ? acc[i + h] : acc[i];
+        acc[i] = keep + __shfl_xor(send, m, 64);
       }
+    }
 #pragma unroll
-      for (int m = 4; m >= 1; m >>= 1) acc[0] += __shfl_xor(acc[0], m, 64);
-      const int rl = lane >> 3;  // row of this lane's sum: bits 5, 4, 3 of the lane
-      if ((lane & 7) == 0 && rl < nr) Ub[row0 + rl] = acc[0];
+    for (int m = 4; m >= 1; m >>= 1) acc[0] += __shfl_xor(acc[0], m, 64);
+    const int rl = lane >> 3;  // row of this lane's sum: bits 5, 4, 3 of the lane
+    if ((lane & 7) == 0 && rl < nr) {
+      if (npc == 1) U[trg_dsp[b] * dof + row0 + rl] = acc[0];
+      else part[part_dsp[b] + (row0 + rl) * npc + c0 / piece] = acc[0];
     }
   }
+}
+
+// One workgroup per group of up to NWG cut rows: the pieces' sums in order.
+__global__ void __launch_bounds__(NWG)
+k_near_gemv_sum(const SplitRows* __restrict__ groups, const double* __restrict__ part, double* __restrict__ U) {
+  const SplitRows G = groups[blockIdx.x];
+  const int i = threadIdx.x;
+  if (i >= G.rows) return;
+  const double* p = part + G.p + (int64_t)i * G.pieces;
+  double s = 0.0;
+  for (int k = 0; k < G.pieces; k++) s += p[k];
+  U[G.u + i] = s;
 }
 
 // ScatterForward + per-target accumulation: for every target i and every
@@ -517,7 +538,7 @@ k_near_accumulate(int64_t ntrg, const int64_t* __restrict__ cnt, const int64_t* 
   for (int k = 0; k < DOF; k++) U[i * DOF + k] = acc[k];
 }
 
-using NearMatFn = void (*)(const int32_t*, const int64_t*, int64_t, const int64_t*, const int32_t*, const int64_t*,
+using NearMatFn = void (*)(const int32_t*, const int64_t*, const int32_t*, int64_t, const int64_t*, const int32_t*, const int64_t*,
                            const int32_t*, const int64_t*, const double*, const double*, const double*,
                            const double*, const double*, double*, double, double);
 
@@ -534,10 +555,36 @@ NearMatFn near_mat_fn(int ker, bool ndot, bool sub) {
   });
 }
 
+// Columns per piece of each block for a kernel whose wave tiles take row_words
+// = rows x words per column.  A tile holds at most 1/share of what one of 8
+// waves per CU has to move on average, and at least `least` columns, rounded up
+// to whole 64-column chunks: with all of a block's columns in one tile a few
+// long ones outlasted the rest by far, and few blocks left the GPU idle.  The
+// matrix kernel pays for each cut with a pass of part-filled lines per row, so
+// its share is the smallest that the sweeps of 1 to 6 bear; the GEMV's is 4.
+// MI355X, us before / after:
+//   KNearSubtract  Laplace DxU 16 blocks 221 / 20, 64 277 / 54, 300 450 / 412, 512 793 / 795
+//                  Stokes DxU 16 1112 / 83, 60 2257 / 820, 200 3290 / 2366
+//   GEMV           Laplace DxU 16 29 / 9, 64 60 / 24, 300 177 / 159, 512 314 / 309
+//                  Stokes DxU 16 136 / 32, 60 375 / 270, 200 859 / 845
+std::vector<int32_t> near_pieces(const std::vector<int64_t>& cols, const std::vector<int64_t>& groups,
+                                 int64_t row_words, int64_t least, int64_t share, int num_cus) {
+  int64_t total = 0;
+  for (size_t b = 0; b < cols.size(); b++) total += cols[b] * groups[b] * row_words;
+  const int64_t most = std::max<int64_t>(least, total / (8 * num_cus * share) / std::max<int64_t>(1, row_words));
+  std::vector<int32_t> piece(cols.size());
+  for (size_t b = 0; b < cols.size(); b++) {
+    const int64_t n = std::max<int64_t>(1, (cols[b] + most - 1) / most);
+    piece[b] = (int32_t)std::max<int64_t>(64, ((cols[b] + n - 1) / n + 63) / 64 * 64);
+  }
+  return piece;
+}
+
 // Flattens per-block tile counts into a device tile list, blocks in
 // decreasing order of cost per tile (longest-processing-time first; a
 // block's tiles stay consecutive).
-int build_tiles(const std::vector<int64_t>& per_block, const std::vector<int64_t>& cost, TileList* out) {
+int build_tiles(const std::vector<int64_t>& per_block, const std::vector<int64_t>& cost,
+                const std::vector<int32_t>& piece, TileList* out) {
   const size_t nb = per_block.size();
   std::vector<size_t> order(nb);
   std::iota(order.begin(), order.end(), 0);
@@ -555,6 +602,7 @@ int build_tiles(const std::vector<int64_t>& per_block, const std::vector<int64_t
   out->ntiles = total;
   SCTL_TRY(dev_upload(&out->d_tile_blk, blk));
   SCTL_TRY(dev_upload(&out->d_tile_dsp, dsp));
+  SCTL_TRY(dev_upload(&out->d_piece, piece));
   return SCTL_AMD_SUCCESS;
 }
 
@@ -577,7 +625,7 @@ int near_matrix_launch(sctl_amd_plan_s* p, bool sub, const double* wts, const do
   }
   ProfileScope prof(s);
   hipLaunchKernelGGL(near_mat_fn(p->kernel, p->near_ndot, sub), dim3(tile_grid(p->mat_tiles.ntiles)), dim3(NWG), 0,
-                     s, p->mat_tiles.d_tile_blk, p->mat_tiles.d_tile_dsp, p->mat_tiles.ntiles, p->d_trg_dsp,
+                     s, p->mat_tiles.d_tile_blk, p->mat_tiles.d_tile_dsp, p->mat_tiles.d_piece, p->mat_tiles.ntiles, p->d_trg_dsp,
                      p->d_trg_cnt, p->d_src_dsp, p->d_src_cnt, p->d_near_off, p->d_xt, n_trg, p->d_xs, p->d_xn, wts,
                      K, kernel_scale(p->kernel), p->ctx);
   SCTL_HIP_TRY(hipGetLastError());
@@ -588,9 +636,14 @@ int near_gemv_launch(sctl_amd_plan_s* p, const double* K, const double* F, doubl
   if (p->gemv_tiles.ntiles == 0) return SCTL_AMD_SUCCESS;
   ProfileScope prof(s);
   hipLaunchKernelGGL(k_near_gemv, dim3(tile_grid(p->gemv_tiles.ntiles)), dim3(NWG), 0, s, p->gemv_tiles.d_tile_blk,
-                     p->gemv_tiles.d_tile_dsp, p->gemv_tiles.ntiles, p->d_trg_dsp, p->d_trg_cnt, p->d_src_dsp,
-                     p->d_src_cnt, p->d_near_off, p->K0, p->near_dof, K, F, U);
+                     p->gemv_tiles.d_tile_dsp, p->gemv_tiles.d_piece, p->gemv_tiles.ntiles, p->d_trg_dsp, p->d_trg_cnt,
+                     p->d_src_dsp, p->d_src_cnt, p->d_near_off, p->K0, p->near_dof, K, F, U, p->d_gemv_part_dsp,
+                     p->d_gemv_part);
   SCTL_HIP_TRY(hipGetLastError());
+  if (p->gemv_nsplit) {
+    hipLaunchKernelGGL(k_near_gemv_sum, dim3(p->gemv_nsplit), dim3(NWG), 0, s, p->d_gemv_split, p->d_gemv_part, U);
+    SCTL_HIP_TRY(hipGetLastError());
+  }
   return SCTL_AMD_SUCCESS;
 }
 
@@ -684,21 +737,54 @@ int sctl_amd_plan_near_layout(sctl_amd_plan p, const int64_t* blk_off, int trg_n
                      "block matrices overlap (blocks " + std::to_string(order[i - 1]) + " and " +
                          std::to_string(order[i]) + ")");
   }
-  std::vector<int64_t> mat(nb), gemv(nb), cost(nb);
+  DeviceInfo dev;
+  SCTL_TRY(device_info(&dev));
+  const int cus = std::max(dev.num_cus, 1);
+  std::vector<int64_t> mat(nb), gemv(nb), src(nb), cols(nb), cost_m(nb), cost_g(nb), part_dsp(nb, -1);
   for (int64_t b = 0; b < nb; b++) {
     const int64_t tc = p->trg_cnt[b], sc = p->src_cnt[b];
     mat[b] = (off[b] >= 0 && tc > 0 && sc > 0) ? (tc + MAT_ST - 1) / MAT_ST : 0;
-    gemv[b] = tc > 0 ? (tc * dof + GEMV_ROWS - 1) / GEMV_ROWS : 0;
-    cost[b] = off[b] >= 0 ? sc : 0;
+    gemv[b] = tc > 0 ? (tc * dof + GEMV_GR - 1) / GEMV_GR : 0;
+    src[b] = off[b] >= 0 ? sc : 0;
+    cols[b] = src[b] * p->K0;
   }
+  const std::vector<int32_t> mat_piece = near_pieces(src, mat, (int64_t)MAT_ST * dof * p->K0, 128,
+                                                       dof * p->K0 == 1 ? 1 : 2, cus);
+  std::vector<int32_t> gemv_piece = near_pieces(cols, gemv, GEMV_GR, 512, 4, cus);
+  std::vector<SplitRows> split;
+  int64_t part_words = 0;
+  for (int64_t b = 0; b < nb; b++) {
+    mat[b] *= std::max<int64_t>(1, (src[b] + mat_piece[b] - 1) / mat_piece[b]);
+    cost_m[b] = std::min<int64_t>(src[b], mat_piece[b]);
+    if (off[b] < 0) gemv_piece[b] = 0x7fffffff;  // zero rows, in one piece
+    const int64_t n = std::max<int64_t>(1, (cols[b] + gemv_piece[b] - 1) / gemv_piece[b]);
+    cost_g[b] = std::min<int64_t>(cols[b], gemv_piece[b]);
+    gemv[b] *= n;
+    if (n > 1) {
+      part_dsp[b] = part_words;
+      const int64_t rows = p->trg_cnt[b] * dof;
+      for (int64_t r = 0; r < rows; r += NWG)
+        split.push_back(SplitRows{p->trg_dsp[b] * dof + r, part_words + r * n, (int32_t)std::min<int64_t>(NWG, rows - r),
+                                  (int32_t)n});
+      part_words += rows * n;
+    }
+  }
+  SCTL_CHECK_ARG(split.size() < 0x7fffffffULL, "near-field layout has too many rows");
   p->free_near();
   int rc = dev_upload(&p->d_near_off, off);
-  if (!rc) rc = build_tiles(mat, cost, &p->mat_tiles);
-  if (!rc) rc = build_tiles(gemv, cost, &p->gemv_tiles);
+  if (!rc) rc = build_tiles(mat, cost_m, mat_piece, &p->mat_tiles);
+  if (!rc) rc = build_tiles(gemv, cost_g, gemv_piece, &p->gemv_tiles);
+  if (!rc) rc = dev_upload(&p->d_gemv_part_dsp, part_dsp);
+  if (!rc) rc = dev_upload(&p->d_gemv_split, split);
+  if (!rc && part_words && hipMalloc(&p->d_gemv_part, sizeof(double) * part_words) != hipSuccess) {
+    set_error("hipMalloc of the near-field partial sums failed");
+    rc = SCTL_AMD_ERROR_OUT_OF_MEMORY;
+  }
   if (rc) {
     p->free_near();
     return rc;
   }
+  p->gemv_nsplit = (int)split.size();
   p->near_off = off;
   p->near_dof = dof;
   p->near_ndot = trg_normal_dot != 0;
