@@ -158,10 +158,11 @@ int stage_in(Scratch& buf, const double* host, int64_t n, hipStream_t s, const d
 
 // Pinned host staging for large device-to-host results (a host KernelMatrix):
 // chunks of PIN_CHUNK bytes taken from a process-wide pool of page-locked
-// buffers (allocated with hipHostMalloc on first use, reused, never returned
-// to the driver), two per call so that the copy of one chunk into the
-// caller's memory overlaps the DMA of the next.
-constexpr size_t PIN_CHUNK = (size_t)8 << 20;
+// buffers (allocated with hipHostMalloc on first use and reused; PIN_KEEP free
+// ones are kept, more go back to the driver), two per call so that the copy of
+// one chunk into the caller's memory overlaps the DMA of the next.  A host Eval
+// that fits one chunk goes through one (eval_host_small).
+constexpr size_t PIN_CHUNK = (size_t)8 << 20, PIN_KEEP = 32;
 std::mutex g_pin_mutex;
 std::vector<void*> g_pin_free;
 
@@ -179,8 +180,14 @@ int pin_take(void** p) {
 }
 void pin_give(void* p) {
   if (!p) return;
-  std::lock_guard<std::mutex> lock(g_pin_mutex);
-  g_pin_free.push_back(p);
+  {
+    std::lock_guard<std::mutex> lock(g_pin_mutex);
+    if (g_pin_free.size() < PIN_KEEP) {
+      g_pin_free.push_back(p);
+      return;
+    }
+  }
+  (void)hipHostFree(p);
 }
 
 // host[0, bytes) = dev[0, bytes), through two pinned chunks on stream s
@@ -270,6 +277,76 @@ int eval_args(int kernel, const double* ctx, int* precision, int digits, const d
 
 double eval_ctx_value(int kernel, const double* ctx) { return ctx_value(kernel, ctx); }
 
+namespace {
+
+// The Eval on device arrays, arguments checked and precision resolved.
+int eval_device(int kernel, const double* ctx, int precision, int digits, const double* r_trg, int64_t nt,
+                const double* r_src, const double* n_src, const double* v_src, int64_t ns, double* v_trg,
+                uint32_t flags, hipStream_t s) {
+  const int newton = precision == SCTL_AMD_FP64 ? newton_steps_f64(digits) : ((flags & SCTL_AMD_MIXED_NEWTON) ? 1 : 0);
+  const DenseShape shape = pick_dense_shape(kernel, precision, newton, nt, ns);
+  const double mu = ctx_value(kernel, ctx);
+  if (precision == SCTL_AMD_FP64)
+    return launch_eval_f64(kernel, newton, r_trg, nt, r_src, n_src, v_src, ns, v_trg, shape, mu, s);
+  return launch_eval_mixed(kernel, newton, r_trg, nt, r_src, n_src, v_src, ns, v_trg, shape, mu, s);
+}
+
+// A host Eval whose arrays fit one pinned chunk: they go over in one copy from
+// there and the result comes back in one.  With a copy from each of the
+// caller's pageable arrays to an allocation of its own, a numpy caller's Eval
+// took, us before / after: Laplace FxU 200 x 200 112 / 47 (both with the device
+// work of their time), 2000 x 3000 172 / 66, 20 000 x 20 000 394 / 288; Stokes DxU
+// 2000 x 3000 243 / 76.
+int eval_host_small(int kernel, const double* ctx, int precision, int digits, const double* r_trg, int64_t nt,
+                    const double* r_src, const double* n_src, const double* v_src, int64_t ns, double* v_trg,
+                    uint32_t flags, hipStream_t s, bool* done) {
+  const KernelMeta& m = META[kernel];
+  // Each count is bounded first: the sum of their products cannot wrap.
+  constexpr int64_t MOST = (int64_t)(PIN_CHUNK / sizeof(double));
+  if (nt > MOST || ns > MOST) return SCTL_AMD_SUCCESS;
+  Carve c;
+  const size_t o_vt = c.take(sizeof(double) * nt * m.K1), o_rt = c.take(sizeof(double) * nt * 3),
+               o_rs = c.take(sizeof(double) * ns * 3), o_n = c.take(sizeof(double) * ns * m.ND),
+               o_vs = c.take(sizeof(double) * ns * m.K0);
+  if (c.bytes > PIN_CHUNK) return SCTL_AMD_SUCCESS;
+  Scratch buf;
+  SCTL_TRY(buf.alloc(c.bytes, s));
+  void* pin = nullptr;
+  if (pin_take(&pin) != SCTL_AMD_SUCCESS) {  // no pinned memory: the copies from pageable arrays
+    (void)hipGetLastError();
+    return SCTL_AMD_SUCCESS;
+  }
+  char *p = static_cast<char*>(pin), *d = buf.as<char>();
+  auto at = [](char* base, size_t off) { return reinterpret_cast<double*>(base + off); };
+  std::memcpy(p + o_vt, v_trg, sizeof(double) * nt * m.K1);
+  std::memcpy(p + o_rt, r_trg, sizeof(double) * nt * 3);
+  std::memcpy(p + o_rs, r_src, sizeof(double) * ns * 3);
+  if (m.ND) std::memcpy(p + o_n, n_src, sizeof(double) * ns * m.ND);
+  std::memcpy(p + o_vs, v_src, sizeof(double) * ns * m.K0);
+  auto run = [&]() -> int {
+    SCTL_HIP_TRY(hipMemcpyAsync(d, p, c.bytes, hipMemcpyHostToDevice, s));
+    SCTL_TRY(eval_device(kernel, ctx, precision, digits, at(d, o_rt), nt, at(d, o_rs), m.ND ? at(d, o_n) : nullptr,
+                         at(d, o_vs), ns, at(d, o_vt), flags, s));
+    SCTL_HIP_TRY(hipMemcpyAsync(p + o_vt, d + o_vt, sizeof(double) * nt * m.K1, hipMemcpyDeviceToHost, s));
+    return SCTL_AMD_SUCCESS;
+  };
+  int rc = run();
+  buf.release();
+  const hipError_t e = hipStreamSynchronize(s);  // also after a failure: copies may be in flight
+  if (rc == SCTL_AMD_SUCCESS && e != hipSuccess) {
+    set_error(std::string("hipStreamSynchronize failed: ") + hipGetErrorString(e));
+    rc = SCTL_AMD_ERROR_HIP;
+  }
+  if (rc == SCTL_AMD_SUCCESS) {
+    std::memcpy(v_trg, p + o_vt, sizeof(double) * nt * m.K1);
+    *done = true;
+  }
+  pin_give(pin);
+  return rc;
+}
+
+}  // namespace
+
 }  // namespace sctl_amd
 
 using namespace sctl_amd;
@@ -328,6 +405,11 @@ int sctl_amd_eval_ctx(int kernel, const double* ctx, int precision, int digits, 
   const KernelMeta& m = META[kernel];
   hipStream_t s = as_stream(stream);
   const bool host = flags & SCTL_AMD_HOST_PTRS;
+  if (host) {
+    bool done = false;
+    SCTL_TRY(eval_host_small(kernel, ctx, precision, digits, r_trg, nt, r_src, n_src, v_src, ns, v_trg, flags, s, &done));
+    if (done) return SCTL_AMD_SUCCESS;
+  }
   Scratch b_rt, b_rs, b_ns, b_vs, b_vt;
   const double *rt = r_trg, *rs = r_src, *nsrc = m.ND ? n_src : nullptr, *vs = v_src;
   double* vt = v_trg;
@@ -340,13 +422,7 @@ int sctl_amd_eval_ctx(int kernel, const double* ctx, int precision, int digits, 
     SCTL_TRY(stage_in(b_vt, v_trg, nt * m.K1, s, &vt_c));
     vt = b_vt.as<double>();
   }
-  const int newton = precision == SCTL_AMD_FP64 ? newton_steps_f64(digits) : ((flags & SCTL_AMD_MIXED_NEWTON) ? 1 : 0);
-  const DenseShape shape = pick_dense_shape(kernel, precision, newton, nt, ns);
-  if (precision == SCTL_AMD_FP64) {
-    SCTL_TRY(launch_eval_f64(kernel, newton, rt, nt, rs, nsrc, vs, ns, vt, shape, ctx_value(kernel, ctx), s));
-  } else {
-    SCTL_TRY(launch_eval_mixed(kernel, newton, rt, nt, rs, nsrc, vs, ns, vt, shape, ctx_value(kernel, ctx), s));
-  }
+  SCTL_TRY(eval_device(kernel, ctx, precision, digits, rt, nt, rs, nsrc, vs, ns, vt, flags, s));
   if (host) {
     SCTL_HIP_TRY(hipMemcpyAsync(v_trg, vt, sizeof(double) * nt * m.K1, hipMemcpyDeviceToHost, s));
     b_rt.release(); b_rs.release(); b_ns.release(); b_vs.release(); b_vt.release();
