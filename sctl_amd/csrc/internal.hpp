@@ -180,8 +180,11 @@ size_t hilbert_order_bytes(int64_t na, int64_t nb);
 int hilbert_order(const double* a, int64_t na, uint32_t* perm_a, const double* b, int64_t nb, uint32_t* perm_b,
                  void* work, hipStream_t stream);
 // Axis-aligned bounding box of two point sets (either may be empty):
-// box6 (device) = {min x, min y, min z, max x, max y, max z}.  sort.hip.
-int bounding_box(const double* a, int64_t na, const double* b, int64_t nb, double* box6, hipStream_t stream);
+// box6 (device) = {min x, min y, min z, max x, max y, max z}; `work` (device)
+// holds bounding_box_bytes(na, nb) bytes.  sort.hip.
+size_t bounding_box_bytes(int64_t na, int64_t nb);
+int bounding_box(const double* a, int64_t na, const double* b, int64_t nb, double* box6, void* work,
+                 hipStream_t stream);
 
 // Shape defaults and tuning-database lookup (tune.cpp).  `newton` is the
 // Newton count of the path (part of the tuning key).

@@ -36,40 +36,157 @@
 // target keys), so the list is exact.
 //
 // Build, get and destroy for 2048 elements (0.9 M nodes) and 500 009 targets on
-// MI355X: 5.76 -> 1.59 ms; the passes over the elements, two of them before
-// (candidates counted, then tested), 1.78 -> 0.36 ms, the sorts of the pairs 0.38
-// -> 0.19.  All results live in one buffer of the library's pool: seven
-// hipMalloc and hipFree each, and their waits, were half of the time.
+// MI355X: 5.53 -> 0.87 ms; the passes over the elements, two of them before
+// (candidates counted, then tested), 1.78 -> 0.35 ms, the sorts of the pairs 0.38
+// -> 0.19.  Scratch and results are one block each of memory kept between
+// builds (block_take): seven hipMalloc and hipFree each for the results, and
+// their waits, were half of the time.
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include <algorithm>
+#include <mutex>
 #include <string>
+#include <vector>
 
 #include "internal.hpp"
 #include "wave.hpp"
+
+namespace sctl_amd {
+namespace {
+
+// Device memory of near lists (a build's scratch, a list's results) kept for
+// the next build: up to KEEP_BLOCKS blocks and KEEP_BYTES per device, the
+// oldest given back beyond that.  A block carries an event recorded after its
+// last use; whoever takes it makes its stream wait for that event, so threads
+// and streams share the blocks freely.  (The stream-ordered pool, asked for
+// such buffers again while the last read of the previous ones was under way,
+// mapped new memory instead, and past its threshold did so on every call: 5.4
+// instead of 1.3 ms, or 1.3, from one run to the next.)
+struct Block {
+  char* p = nullptr;
+  size_t bytes = 0;
+  int device = 0;
+  hipEvent_t used = nullptr;
+};
+constexpr size_t KEEP_BYTES = (size_t)2 << 30;
+constexpr int KEEP_BLOCKS = 8;
+std::mutex g_blocks_mutex;
+std::vector<Block>& free_blocks() {  // oldest first; never destroyed (the runtime may be gone by then)
+  static auto* v = new std::vector<Block>();
+  return *v;
+}
+
+void block_drop(Block b) {  // hipFree waits for the device
+  int cur = -1;
+  (void)hipGetDevice(&cur);
+  if (cur != b.device) (void)hipSetDevice(b.device);
+  if (b.p) (void)hipFree(b.p);
+  if (b.used) (void)hipEventDestroy(b.used);
+  if (cur >= 0 && cur != b.device) (void)hipSetDevice(cur);
+}
+
+// A block of at least `bytes` on the current device, usable on stream s.
+int block_take(size_t bytes, hipStream_t s, Block* out) {
+  DeviceInfo dev;
+  SCTL_TRY(device_info(&dev));
+  {
+    std::lock_guard<std::mutex> lock(g_blocks_mutex);
+    auto& v = free_blocks();
+    size_t best = v.size();
+    for (size_t i = 0; i < v.size(); i++)
+      if (v[i].device == dev.device && v[i].bytes >= bytes && v[i].bytes / 4 <= bytes + ((size_t)16 << 20) &&
+          (best == v.size() || v[i].bytes < v[best].bytes))
+        best = i;
+    if (best < v.size()) {
+      *out = v[best];
+      v.erase(v.begin() + best);
+    }
+  }
+  if (out->p) {
+    SCTL_HIP_TRY(hipStreamWaitEvent(s, out->used, 0));
+    return SCTL_AMD_SUCCESS;
+  }
+  size_t step = (size_t)1 << 16;  // an eighth of the size's power of two, so that sizes that differ a little reuse
+  while (step * 16 <= bytes) step *= 2;
+  out->device = dev.device;
+  out->bytes = (bytes + step - 1) / step * step;
+  if (hipMalloc(reinterpret_cast<void**>(&out->p), out->bytes) != hipSuccess) {
+    (void)hipGetLastError();  // give back what is kept and try once more
+    std::vector<Block> all;
+    {
+      std::lock_guard<std::mutex> lock(g_blocks_mutex);
+      all.swap(free_blocks());
+    }
+    for (Block& b : all) block_drop(b);
+    out->p = nullptr;
+    SCTL_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&out->p), out->bytes));
+  }
+  SCTL_HIP_TRY(hipEventCreateWithFlags(&out->used, hipEventDisableTiming));
+  return SCTL_AMD_SUCCESS;
+}
+
+// Returns a block whose `used` event has been recorded after its last use.
+void block_give(Block b) {
+  if (!b.p || !b.used) {
+    block_drop(b);
+    return;
+  }
+  std::vector<Block> drop;
+  {
+    std::lock_guard<std::mutex> lock(g_blocks_mutex);
+    auto& v = free_blocks();
+    v.push_back(b);
+    size_t bytes = 0, count = 0;
+    for (const Block& x : v)
+      if (x.device == b.device) {
+        bytes += x.bytes;
+        count++;
+      }
+    for (size_t i = 0; i < v.size() && (bytes > KEEP_BYTES || count > KEEP_BLOCKS);) {
+      if (v[i].device != b.device) {
+        i++;
+        continue;
+      }
+      bytes -= v[i].bytes;
+      count--;
+      drop.push_back(v[i]);
+      v.erase(v.begin() + i);
+    }
+  }
+  for (Block& x : drop) block_drop(x);
+}
+
+// A build's scratch: given back in stream order when it goes out of scope.
+struct BlockScratch {
+  Block b;
+  hipStream_t s = nullptr;
+  int alloc(size_t bytes, hipStream_t stream) {
+    s = stream;
+    return block_take(bytes, s, &b);
+  }
+  ~BlockScratch() {
+    if (!b.p) return;
+    if (hipEventRecord(b.used, s) != hipSuccess) {  // no order known: free it, which waits
+      (void)hipGetLastError();
+      block_drop(b);
+      return;
+    }
+    block_give(b);
+  }
+};
+
+}  // namespace
+}  // namespace sctl_amd
 
 struct sctl_amd_near_list_s {
   int device = 0;
   int64_t ntrg = 0, nelem = 0, n_near = 0;
   bool has_normal = false;
-  char* buf = nullptr;         // all results, from the library's pool
-  size_t counts = 0, counts_bytes = 0;  // the four count and offset arrays within buf, adjacent
+  sctl_amd::Block buf;  // all results; its event: the latest read of them, on whichever stream
   double *d_xtn = nullptr, *d_xntn = nullptr;
   int64_t *d_ecnt = nullptr, *d_edsp = nullptr, *d_scatter = nullptr, *d_tcnt = nullptr, *d_tdsp = nullptr;
-  hipEvent_t last = nullptr;  // the latest read of the results, on whichever stream
-  ~sctl_amd_near_list_s() {
-    int cur = -1;
-    (void)hipGetDevice(&cur);
-    if (cur != device) (void)hipSetDevice(device);
-    if (buf) {
-      // Freed in this thread's stream after the last read.
-      if (last) (void)hipStreamWaitEvent(hipStreamPerThread, last, 0);
-      (void)hipFreeAsync(buf, hipStreamPerThread);
-    }
-    if (last) (void)hipEventDestroy(last);
-    if (cur >= 0 && cur != device) (void)hipSetDevice(cur);
-  }
+  ~sctl_amd_near_list_s() { sctl_amd::block_give(buf); }
 };
 
 namespace sctl_amd {
@@ -506,10 +623,8 @@ int bits_for(int64_t n) {
   return b;
 }
 
-// One pool allocation for a list of n pairs, its count and offset arrays zeroed.
+// The buffer of a list of n pairs, its count and offset arrays zeroed.
 int list_alloc(sctl_amd_near_list_s* L, int64_t n, hipStream_t s) {
-  DeviceInfo dev;
-  SCTL_TRY(device_info(&dev));
   Carve c;
   const size_t xtn = c.take(sizeof(double) * 3 * n), xntn = c.take(L->has_normal ? sizeof(double) * 3 * n : 0),
                scatter = c.take(sizeof(int64_t) * n), ecnt = c.take(sizeof(int64_t) * L->nelem),
@@ -517,115 +632,139 @@ int list_alloc(sctl_amd_near_list_s* L, int64_t n, hipStream_t s) {
                tdsp = c.take(sizeof(int64_t) * L->ntrg);
   L->n_near = n;
   if (!c.bytes) return SCTL_AMD_SUCCESS;
-  SCTL_HIP_TRY(hipMallocFromPoolAsync(reinterpret_cast<void**>(&L->buf), c.bytes, dev.pool, s));
-  L->d_xtn = reinterpret_cast<double*>(L->buf + xtn);
-  if (L->has_normal) L->d_xntn = reinterpret_cast<double*>(L->buf + xntn);
-  L->d_scatter = reinterpret_cast<int64_t*>(L->buf + scatter);
-  L->d_ecnt = reinterpret_cast<int64_t*>(L->buf + ecnt);
-  L->d_edsp = reinterpret_cast<int64_t*>(L->buf + edsp);
-  L->d_tcnt = reinterpret_cast<int64_t*>(L->buf + tcnt);
-  L->d_tdsp = reinterpret_cast<int64_t*>(L->buf + tdsp);
+  SCTL_TRY(block_take(c.bytes, s, &L->buf));
+  L->d_xtn = reinterpret_cast<double*>(L->buf.p + xtn);
+  if (L->has_normal) L->d_xntn = reinterpret_cast<double*>(L->buf.p + xntn);
+  L->d_scatter = reinterpret_cast<int64_t*>(L->buf.p + scatter);
+  L->d_ecnt = reinterpret_cast<int64_t*>(L->buf.p + ecnt);
+  L->d_edsp = reinterpret_cast<int64_t*>(L->buf.p + edsp);
+  L->d_tcnt = reinterpret_cast<int64_t*>(L->buf.p + tcnt);
+  L->d_tdsp = reinterpret_cast<int64_t*>(L->buf.p + tdsp);
   const int64_t words = (int64_t)(c.bytes - ecnt) / 8;
   if (words > 0) {
     hipLaunchKernelGGL(k_nl_zero, dim3(grid_of(words)), dim3(NL_WG), 0, s, L->d_ecnt, words);
     SCTL_HIP_TRY(hipGetLastError());
   }
+  // Until a read is recorded: a failed build destroys its list here.
+  SCTL_HIP_TRY(hipEventRecord(L->buf.used, s));
   return SCTL_AMD_SUCCESS;
 }
 
-// The near pairs' keys, sorted, and the arrays made from them.
+// Scratch of the steps that follow once the number of pairs n is known.
+template <class Key> struct PairScratch {
+  size_t pairs, trg, pair, trg_s, pair_s, tmp, tmp1 = 0, tmp2 = 0, bytes;
+  int tbits, bits;
+};
+template <class Key> int pair_scratch(int64_t nt, int64_t nelem, int64_t n, PairScratch<Key>* p) {
+  p->tbits = bits_for(nt);
+  p->bits = p->tbits + bits_for(nelem);
+  SCTL_HIP_TRY(rocprim::radix_sort_keys(nullptr, p->tmp1, (Key*)nullptr, (Key*)nullptr, (size_t)n, 0,
+                                        std::max(p->bits, 1), nullptr));
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, p->tmp2, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr,
+                                         (uint32_t*)nullptr, (size_t)n, 0, std::max(p->tbits, 1), nullptr));
+  Carve c;
+  p->pairs = c.take(sizeof(Key) * n);
+  p->trg = c.take(4 * n);
+  p->pair = c.take(4 * n);
+  p->trg_s = c.take(4 * n);
+  p->pair_s = c.take(4 * n);
+  p->tmp = c.take(std::max(p->tmp1, p->tmp2));
+  p->bytes = c.bytes;
+  return SCTL_AMD_SUCCESS;
+}
+
+// The build on device arrays of at least one target, node and element.  One
+// scratch allocation as long as the pairs are at most USUAL per target, which
+// the later steps' share of it is sized for: each stream-ordered free costs
+// the host some hundred microseconds here.
 template <class Key>
 int build_pairs(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const double* xn, const double* xs, int64_t ns,
-                const double* rad, int64_t nelem, const int64_t* ecnt, const int64_t* edsp, const double* xsorted,
-                const uint64_t* keys, const uint32_t* idx, const double* cube, hipStream_t s) {
-  const int tbits = bits_for(nt);
-  // Room for 24 pairs per target at first; a longer list is filled again.
-  int64_t cap = (int64_t)std::min<double>((double)nt * (double)nelem, std::max(24.0 * (double)nt, 65536.0)), n = 0;
-  Scratch found;
+                const double* rad, int64_t nelem, const int64_t* ecnt, const int64_t* edsp, hipStream_t s) {
+  constexpr double ROOM = 24, USUAL = 8;  // pairs per target
+  auto at_most = [&](double per_target) {
+    return (int64_t)std::min<double>((double)nt * (double)nelem, std::max(per_target * (double)nt, 65536.0));
+  };
+  int64_t cap = at_most(ROOM), n = 0;
+  const int64_t usual = at_most(USUAL);
+  size_t sort_bytes = 0;
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, sort_bytes, (uint64_t*)nullptr, (uint64_t*)nullptr,
+                                         (uint32_t*)nullptr, (uint32_t*)nullptr, (size_t)nt, 0, 63, s));
+  PairScratch<Key> ps;
+  SCTL_TRY(pair_scratch(nt, nelem, usual, &ps));
+  Carve c;
+  const size_t o_cube = c.take(sizeof(double) * 6), o_part = c.take(bounding_box_bytes(nt, ns)),
+               o_counter = c.take(sizeof(int64_t)), o_keys_in = c.take(8 * nt), o_keys = c.take(8 * nt),
+               o_idx_in = c.take(4 * nt), o_idx = c.take(4 * nt), o_x = c.take(24 * nt), o_tmp = c.take(sort_bytes),
+               o_found = c.take(sizeof(Key) * cap), o_later = c.take(ps.bytes);
+  BlockScratch work, more, later;
+  SCTL_TRY(work.alloc(c.bytes, s));
+  char* w = work.b.p;
+  double *cube = reinterpret_cast<double*>(w + o_cube), *xsorted = reinterpret_cast<double*>(w + o_x);
+  uint64_t *keys_in = reinterpret_cast<uint64_t*>(w + o_keys_in), *keys = reinterpret_cast<uint64_t*>(w + o_keys);
+  uint32_t *idx_in = reinterpret_cast<uint32_t*>(w + o_idx_in), *idx = reinterpret_cast<uint32_t*>(w + o_idx);
+  int64_t* counter = reinterpret_cast<int64_t*>(w + o_counter);
+  Key* found = reinterpret_cast<Key*>(w + o_found);
+  SCTL_TRY(bounding_box(xt, nt, xs, ns, cube, w + o_part, s));
+  hipLaunchKernelGGL(k_nl_cube, dim3(1), dim3(64), 0, s, cube, cube);
+  hipLaunchKernelGGL(k_nl_keys, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, cube, keys_in, idx_in);
+  SCTL_HIP_TRY(hipGetLastError());
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(w + o_tmp, sort_bytes, keys_in, keys, idx_in, idx, (size_t)nt, 0, 63, s));
+  hipLaunchKernelGGL(k_nl_gather, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, idx, xsorted);
+  SCTL_HIP_TRY(hipGetLastError());
   for (int pass = 0; pass < 2; pass++) {
-    Carve c;
-    const size_t counter = c.take(sizeof(int64_t)), pairs_in = c.take(sizeof(Key) * cap);
-    SCTL_TRY(found.alloc(c.bytes, s));
-    int64_t* cnt = reinterpret_cast<int64_t*>(found.as<char>() + counter);
-    hipLaunchKernelGGL(k_nl_zero, dim3(1), dim3(NL_WG), 0, s, cnt, (int64_t)1);
+    hipLaunchKernelGGL(k_nl_zero, dim3(1), dim3(NL_WG), 0, s, counter, (int64_t)1);
     hipLaunchKernelGGL((k_nl_elements<Key>), dim3((unsigned)nelem), dim3(NL_WG), 0, s, ecnt, edsp, ns, xs, rad, nt,
-                       xsorted, keys, idx, cube, tbits, reinterpret_cast<unsigned long long*>(cnt), cap,
-                       reinterpret_cast<Key*>(found.as<char>() + pairs_in));
+                       xsorted, keys, idx, cube, ps.tbits, reinterpret_cast<unsigned long long*>(counter), cap, found);
     SCTL_HIP_TRY(hipGetLastError());
-    SCTL_HIP_TRY(hipMemcpyAsync(&n, cnt, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    SCTL_HIP_TRY(hipMemcpyAsync(&n, counter, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     SCTL_HIP_TRY(hipStreamSynchronize(s));
     if (n <= cap) break;
     SCTL_CHECK_ARG(pass == 0, "near-pair count exceeds its bound (internal error)");
     cap = n;
+    SCTL_TRY(more.alloc(sizeof(Key) * cap, s));
+    found = reinterpret_cast<Key*>(more.b.p);
   }
   SCTL_CHECK_ARG(n < ((int64_t)1 << 32), "more than 2^32-1 near pairs");
   SCTL_TRY(list_alloc(L, n, s));
-  if (n == 0) return SCTL_AMD_SUCCESS;
-
-  const Key* pairs_in = reinterpret_cast<const Key*>(found.as<char>() + 256);
-  size_t bytes1 = 0, bytes2 = 0;
-  const int bits = tbits + bits_for(nelem);
-  SCTL_HIP_TRY(rocprim::radix_sort_keys(nullptr, bytes1, (Key*)nullptr, (Key*)nullptr, (size_t)n, 0, bits, s));
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes2, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr,
-                                         (uint32_t*)nullptr, (size_t)n, 0, std::max(tbits, 1), s));
-  Carve c;
-  const size_t o_pairs = c.take(sizeof(Key) * n), o_trg = c.take(4 * n), o_pair = c.take(4 * n),
-               o_trg_s = c.take(4 * n), o_pair_s = c.take(4 * n), o_tmp = c.take(std::max(bytes1, bytes2));
-  Scratch work;
-  SCTL_TRY(work.alloc(c.bytes, s));
-  char* w = work.as<char>();
-  Key* pairs = reinterpret_cast<Key*>(w + o_pairs);
-  uint32_t *trg = reinterpret_cast<uint32_t*>(w + o_trg), *pair = reinterpret_cast<uint32_t*>(w + o_pair);
-  uint32_t *trg_s = reinterpret_cast<uint32_t*>(w + o_trg_s), *pair_s = reinterpret_cast<uint32_t*>(w + o_pair_s);
-  SCTL_HIP_TRY(rocprim::radix_sort_keys(w + o_tmp, bytes1, pairs_in, pairs, (size_t)n, 0, std::max(bits, 1), s));
-  hipLaunchKernelGGL((k_nl_elem_ranges<Key>), dim3(grid_of(nelem)), dim3(NL_WG), 0, s, nelem, pairs, n, tbits,
+  if (n == 0) {
+    SCTL_HIP_TRY(hipStreamSynchronize(s));
+    return SCTL_AMD_SUCCESS;
+  }
+  char* l = w + o_later;
+  SCTL_TRY(pair_scratch(nt, nelem, n, &ps));
+  if (n > usual) {
+    SCTL_TRY(later.alloc(ps.bytes, s));
+    l = later.b.p;
+  }
+  Key* pairs = reinterpret_cast<Key*>(l + ps.pairs);
+  uint32_t *trg = reinterpret_cast<uint32_t*>(l + ps.trg), *pair = reinterpret_cast<uint32_t*>(l + ps.pair);
+  uint32_t *trg_s = reinterpret_cast<uint32_t*>(l + ps.trg_s), *pair_s = reinterpret_cast<uint32_t*>(l + ps.pair_s);
+  SCTL_HIP_TRY(rocprim::radix_sort_keys(l + ps.tmp, ps.tmp1, found, pairs, (size_t)n, 0, std::max(ps.bits, 1), s));
+  hipLaunchKernelGGL((k_nl_elem_ranges<Key>), dim3(grid_of(nelem)), dim3(NL_WG), 0, s, nelem, pairs, n, ps.tbits,
                      L->d_ecnt, L->d_edsp);
   SCTL_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL((k_nl_unpack<Key>), dim3(grid_of(n)), dim3(NL_WG), 0, s, n, pairs, tbits, xt, xn, L->d_xtn,
+  hipLaunchKernelGGL((k_nl_unpack<Key>), dim3(grid_of(n)), dim3(NL_WG), 0, s, n, pairs, ps.tbits, xt, xn, L->d_xtn,
                      L->d_xntn, trg, pair);
   SCTL_HIP_TRY(hipGetLastError());
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(w + o_tmp, bytes2, trg, trg_s, pair, pair_s, (size_t)n, 0,
-                                         std::max(tbits, 1), s));
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(l + ps.tmp, ps.tmp2, trg, trg_s, pair, pair_s, (size_t)n, 0,
+                                         std::max(ps.tbits, 1), s));
   hipLaunchKernelGGL(k_nl_scatter, dim3(grid_of(n)), dim3(NL_WG), 0, s, n, trg_s, pair_s, L->d_scatter,
                      reinterpret_cast<unsigned long long*>(L->d_tcnt), L->d_tdsp);
   SCTL_HIP_TRY(hipGetLastError());
+  SCTL_HIP_TRY(hipStreamSynchronize(s));
   return SCTL_AMD_SUCCESS;
 }
 
-// The build on device arrays.
 int build_list(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const double* xn, const double* xs, int64_t ns,
                const double* rad, int64_t nelem, const int64_t* ecnt, const int64_t* edsp, hipStream_t s) {
-  SCTL_HIP_TRY(hipEventCreateWithFlags(&L->last, hipEventDisableTiming));
   if (nt == 0 || ns == 0 || nelem == 0) {
     SCTL_TRY(list_alloc(L, 0, s));
     SCTL_HIP_TRY(hipStreamSynchronize(s));
     return SCTL_AMD_SUCCESS;
   }
-  size_t bytes = 0;
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, (uint64_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr,
-                                         (uint32_t*)nullptr, (size_t)nt, 0, 63, s));
-  Carve c;
-  const size_t o_cube = c.take(sizeof(double) * 6), o_keys_in = c.take(8 * nt), o_keys = c.take(8 * nt),
-               o_idx_in = c.take(4 * nt), o_idx = c.take(4 * nt), o_x = c.take(24 * nt), o_tmp = c.take(bytes);
-  Scratch work;
-  SCTL_TRY(work.alloc(c.bytes, s));
-  char* w = work.as<char>();
-  double *cube = reinterpret_cast<double*>(w + o_cube), *xsorted = reinterpret_cast<double*>(w + o_x);
-  uint64_t *keys_in = reinterpret_cast<uint64_t*>(w + o_keys_in), *keys = reinterpret_cast<uint64_t*>(w + o_keys);
-  uint32_t *idx_in = reinterpret_cast<uint32_t*>(w + o_idx_in), *idx = reinterpret_cast<uint32_t*>(w + o_idx);
-  SCTL_TRY(bounding_box(xt, nt, xs, ns, cube, s));
-  hipLaunchKernelGGL(k_nl_cube, dim3(1), dim3(64), 0, s, cube, cube);
-  hipLaunchKernelGGL(k_nl_keys, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, cube, keys_in, idx_in);
-  SCTL_HIP_TRY(hipGetLastError());
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(w + o_tmp, bytes, keys_in, keys, idx_in, idx, (size_t)nt, 0, 63, s));
-  hipLaunchKernelGGL(k_nl_gather, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, idx, xsorted);
-  SCTL_HIP_TRY(hipGetLastError());
   if (bits_for(nt) < 32 && bits_for(nt) + bits_for(nelem) <= 32)
-    SCTL_TRY(build_pairs<uint32_t>(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, xsorted, keys, idx, cube, s));
-  else
-    SCTL_TRY(build_pairs<uint64_t>(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, xsorted, keys, idx, cube, s));
-  SCTL_HIP_TRY(hipStreamSynchronize(s));
-  return SCTL_AMD_SUCCESS;
+    return build_pairs<uint32_t>(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, s);
+  return build_pairs<uint64_t>(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, s);
 }
 
 }  // namespace
@@ -717,7 +856,7 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
   // list can be destroyed after the last one (a captured read runs later: its
   // graph needs the list to live, as any graph its buffers).
   const bool capturing = stream_capturing(s);
-  if (!capturing) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->last, 0));
+  if (!capturing && list->buf.used) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->buf.used, 0));
   if (flags & SCTL_AMD_HOST_PTRS) {
     for (const auto& x : a)
       if (x.dst && x.src && x.words)
@@ -736,7 +875,7 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
       SCTL_HIP_TRY(hipGetLastError());
     }
   }
-  if (!capturing) SCTL_HIP_TRY(hipEventRecord(list->last, s));
+  if (!capturing && list->buf.used) SCTL_HIP_TRY(hipEventRecord(list->buf.used, s));
   if (flags & SCTL_AMD_HOST_PTRS) SCTL_HIP_TRY(hipStreamSynchronize(s));
   return SCTL_AMD_SUCCESS;
 }

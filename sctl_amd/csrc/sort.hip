@@ -421,16 +421,19 @@ __global__ void __launch_bounds__(RX_WG) k_rx_scatter_high(const uint32_t* __res
 
 }  // namespace
 
-int bounding_box(const double* a, int64_t na, const double* b, int64_t nb, double* box6, hipStream_t stream) {
+size_t bounding_box_bytes(int64_t na, int64_t nb) {
+  return sizeof(double) * 6 * ((na + BB_PER_BLK - 1) / BB_PER_BLK + (nb + BB_PER_BLK - 1) / BB_PER_BLK);
+}
+
+int bounding_box(const double* a, int64_t na, const double* b, int64_t nb, double* box6, void* work,
+                 hipStream_t stream) {
   const int64_t per_blk = BB_PER_BLK;
   const int blk_a = (int)((na + per_blk - 1) / per_blk), blk_b = (int)((nb + per_blk - 1) / per_blk);
   SCTL_CHECK_ARG(blk_a + blk_b > 0, "bounding box of no points");
-  Scratch part;
-  SCTL_TRY(part.alloc(sizeof(double) * 6 * (blk_a + blk_b), stream));
-  hipLaunchKernelGGL(k_bbox_partial, dim3(blk_a + blk_b), dim3(BB_WG), 0, stream, a, na, b, nb, blk_a,
-                     part.as<double>());
+  double* part = static_cast<double*>(work);
+  hipLaunchKernelGGL(k_bbox_partial, dim3(blk_a + blk_b), dim3(BB_WG), 0, stream, a, na, b, nb, blk_a, part);
   SCTL_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(BB_WG), 0, stream, part.as<double>(), blk_a + blk_b, 0, box6);
+  hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(BB_WG), 0, stream, part, blk_a + blk_b, 0, box6);
   SCTL_HIP_TRY(hipGetLastError());
   return SCTL_AMD_SUCCESS;
 }
