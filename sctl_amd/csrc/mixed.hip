@@ -924,9 +924,13 @@ int mixed_geometry(int ker, int64_t nt, int64_t ns, const DenseShape& shape, Mix
   SCTL_CHECK_ARG(g->ntiles <= 0x7fffffffLL, "too many sources for one launch");
   g->Q = layout_q(ker);
   // Enough workgroups for 32 per CU (one tile per split at the least): a
-  // small problem (a few hundred tiles) still fills the GPU.
+  // small problem (a few hundred tiles) still fills the GPU.  The matrix-core
+  // kernel's, shorter and four or three to a CU, take 96, so that the last ones
+  // to run leave fewer CUs idle: Laplace FxU 50000^2 461 -> 448 us, 131072 x
+  // 150001 2452 -> 2408, 524288^2 28.96 -> 28.41 ms; Stokes FxU 131072 x 150001
+  // 6885 -> 6784 us.
   constexpr int64_t SPLIT_TILES = 256;
-  const int64_t want = 32LL * std::max(dev.num_cus, 1);
+  const int64_t want = (g->mfma ? 96LL : 32LL) * std::max(dev.num_cus, 1);
   int64_t nsplit = g->tb < want ? (want + g->tb - 1) / g->tb : 1;
   nsplit = std::min<int64_t>(std::min<int64_t>(nsplit, g->ntiles), 65535);
   nsplit = std::min<int64_t>(std::max<int64_t>(nsplit, (g->ntiles + SPLIT_TILES - 1) / SPLIT_TILES), 65535);
