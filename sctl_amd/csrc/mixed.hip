@@ -25,8 +25,8 @@
 // in FP32 and added into an FP64 sum of the tile, so that a tile's largest
 // term does not take up the rounding of 255 FP32 additions (this halved the
 // headline's error against FP64, 5.4e-7 -> 2.7e-7, at no cost in time).  A
-// tile whose sum is not finite is redone by the masked near loop.  The tiles'
-// sums are added up in FP64 per target.
+// tile whose sum is not finite is redone by the masked near loop.  Each tile's
+// sum is added into the FP64 per-target sum with Kahan compensation.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -532,6 +532,40 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// a and b hold a value per row of 16 lanes.  swap32: a's rows 2, 3 against b's
+// rows 0, 1; swap16: a's rows 1, 3 against b's rows 0, 2.
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(double& a, double& b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  a = __hiloint2double(hi[0], lo[0]);
+  b = __hiloint2double(hi[1], lo[1]);
+}
+// v[j] of row g -> v[g] of row j.
+__device__ __forceinline__ void transpose4(float* v) {
+  swap32(v[0], v[2]);
+  swap32(v[1], v[3]);
+  swap16(v[0], v[1]);
+  swap16(v[2], v[3]);
+}
+// In row j, the FP64 sum of v[j] over the four rows.
+__device__ __forceinline__ double sum_rows(float a, float b, float c, float d) {
+  swap32(a, c);
+  swap32(b, d);
+  double x = (double)a + (double)c, y = (double)b + (double)d;
+  swap16(x, y);
+  return x + y;
+}
+
 // One far pair: D = r^2, d = the NV dot products, row(k) = word k of the source.
 template <int KER, int NEWTON, class Row>
 __device__ __forceinline__ void far_pair(float* p, float& G, float r2, const float* d, Row&& row) {
@@ -561,17 +595,28 @@ __device__ __forceinline__ void far_pair(float* p, float& G, float r2, const flo
 // matrix layout (at most 64 per FP32 sum), mid and near ones with one target
 // per lane from records that the wave stages for itself, NEAR_ST at a time.
 //
-// Waves per SIMD asked for: left alone the compiler takes 148 registers for the
+// A tile's far sums go to the lane of their target (sum_rows), and the targets'
+// columns come from those lanes (transpose4), both by row swaps: a lane holds
+// one compensated sum per output of its own target.  With a sum per target
+// group and output, and the four groups' coordinates in FP64, the single layer
+// took 119 registers, not 95 (20000^2 cube 112.4 -> 108.1 us, 50000^2 445 ->
+// 424), and Stokes 20 words of scratch more (DxU 131072 x 150001 6993 -> 6671
+// us, FxU 6590 -> 6449).
+//
+// Waves per SIMD asked for: left alone the compiler took 148 registers for the
 // Laplace double layer (three waves), 58.6 instead of 45.6 ms at 524288 x
-// 524288; at six waves the single layer spills (32.1 against 30.4 ms then).
-// Three outputs hold 12 FP64 sums per lane more, and run three waves (128
-// registers spill: Stokes FxU 105 against 85 ms).
+// 524288; at six waves the single layer is no faster (28.6 and 28.3 ms).  Three
+// outputs run three waves (128 registers spill: Stokes FxU 131072 x 150001 6.9
+// against 6.4 ms), and no more are offered: else the scheduler saves registers
+// by using each product right after its instruction (Laplace FxdU 524288 x
+// 524288 65.2 against 59.8 ms).
 template <int KER> constexpr int mfma_waves() { return Ker<KER>::K1 == 1 ? 4 : 3; }
 // Chunks and sources unrolled, from sweeps of 1, 2 and 4 resp. 2, 4 and 8.
 template <int KER> constexpr int far_unroll() { return Ker<KER>::K1 == 1 ? 4 : (KER == STK_FXU ? 2 : 1); }
 template <int KER> constexpr int lane_unroll() { return KER == LAP_FXU || KER == LAP_FXDU ? 4 : 2; }
 template <int KER, int NEWTON>
-__global__ void __launch_bounds__(WG, (mfma_waves<KER>()))
+__global__ void __launch_bounds__(WG)
+__attribute__((amdgpu_waves_per_eu((mfma_waves<KER>()), (Ker<KER>::K1 == 1 ? 8 : 3))))
 k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __restrict__ tperm,
                   const float4* __restrict__ packed, const double4* __restrict__ meta, const float4* __restrict__ sub,
                   int64_t ntiles, int64_t tiles_per_split, double* __restrict__ out, int direct, double scale,
@@ -591,28 +636,18 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
   __shared__ float srow[NROW ? NROW : 1][NROW ? TILE : 1];
   __shared__ float4 near_all[(WG / 64) * NEAR_ST * Q];
 
-  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4;
   float4* nst = near_all + (tid >> 6) * (NEAR_ST * Q);
   const SplitCoord wg = split_coord((nt + WG - 1) / WG);
   const int64_t tile_begin = wg.split * tiles_per_split;
   const int64_t tile_end = tile_begin + tiles_per_split < ntiles ? tile_begin + tiles_per_split : ntiles;
   const int64_t q0 = wg.block * WG + (tid & ~63);  // the wave's first target
 
-  // t64: this lane's target (q0 + lane); tg: axis g of the targets q0 + 16 m + c16
-  double t64[3], tg[GROUPS], accn[K1], accf[GROUPS][K1];
+  double t64[3], acc[K1], comp[K1];  // of this lane's target, q0 + lane
 #pragma unroll
   for (int k = 0; k < 3; k++) t64[k] = q0 + lane < nt ? xt[(q0 + lane) * 3 + k] : 0.0;
 #pragma unroll
-  for (int m = 0; m < GROUPS; m++) {
-    const int64_t q = q0 + 16 * m + c16;
-    tg[m] = q < nt && g < 3 ? xt[q * 3 + g] : 0.0;
-  }
-#pragma unroll
-  for (int k = 0; k < K1; k++) {
-    accn[k] = 0.0;
-#pragma unroll
-    for (int m = 0; m < GROUPS; m++) accf[m][k] = 0.0;
-  }
+  for (int k = 0; k < K1; k++) acc[k] = comp[k] = 0.0;
   const int slot = (tid >> 4) * 48 + (tid & 15);  // this thread's row, written per tile
   const int my_slot = g < 3 ? lane : SLOTS, my_step = g < 3 ? 48 : 0;  // read: this lane's in chunk 0, and per chunk
   if (tid == 0) {
@@ -633,7 +668,6 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
       rec[4 * q + 3] = v.w;
     }
     const double4 m = meta[tile];
-    const double cg = g == 0 ? m.x : (g == 1 ? m.y : m.z);
     __syncthreads();  // the previous tile's readers
 #pragma unroll
     for (int k = 0; k < 3; k++) rs[slot + 16 * k] = row_slots(-2.0f * rec[k]);
@@ -660,12 +694,11 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
     const float th[3] = {(float)(t64[0] - m.x), (float)(t64[1] - m.y), (float)(t64[2] - m.z)};
     const float T = fmad(th[2], th[2], fmad(th[1], th[1], th[0] * th[0]));
     const float H2 = (float)m.w;
-    u32x4 col[GROUPS];
+    u32x4 col[GROUPS];  // lane group g: axis g (3: |t'|^2) of the targets q0 + 16 j + (lane & 15)
+    float cx[GROUPS] = {th[0], th[1], th[2], T};
+    transpose4(cx);
 #pragma unroll
-    for (int j = 0; j < GROUPS; j++) {
-      const float Tj = __shfl(T, 16 * j + c16, 64);
-      col[j] = column_slots(g < 3 ? (float)(tg[j] - cg) : Tj);
-    }
+    for (int j = 0; j < GROUPS; j++) col[j] = column_slots(cx[j]);
     float pf[GROUPS][K1], pG[GROUPS], pn[K1];
     double ptn[K1];
 #pragma unroll
@@ -777,35 +810,31 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
       for (int j = 0; j < GROUPS; j++) pG[j] = 0.0f;
       for (int q = 0; q < TILE / 64; q++) by_lane(q * 64, 2);
     }
+    double Gt = 0.0;
+    if constexpr (F::GRAD) Gt = sum_rows(pG[0], pG[1], pG[2], pG[3]);
 #pragma unroll
     for (int k = 0; k < K1; k++) {
-      accn[k] += ptn[k];
-#pragma unroll
-      for (int j = 0; j < GROUPS; j++) {
-        if constexpr (F::GRAD)
-          accf[j][k] += fmad((double)__shfl(th[k], 16 * j + c16, 64), (double)pG[j], (double)pf[j][k]);
-        else accf[j][k] += (double)pf[j][k];
+      ptn[k] += sum_rows(pf[0][k], pf[1][k], pf[2][k], pf[3][k]);
+      if constexpr (F::GRAD) {
+        float x = th[k];
+        asm volatile("" : "+v"(x));  // or the conversion is done in each pass of the far loop
+        ptn[k] = fmad((double)x, Gt, ptn[k]);
       }
+      const double y = ptn[k] - comp[k];  // Kahan: acc += ptn
+      const double sum = acc[k] + y;
+      comp[k] = (sum - acc[k]) - y;
+      acc[k] = sum;
     }
   }
 
-  // Target 16 j + c16's far sums: over the four lane groups, to the lane of that target.
   const int64_t q = q0 + lane;
-  const int64_t t = direct && q < nt ? (int64_t)tperm[q] : 0;
+  if (q >= nt) return;
+  const int64_t t = direct ? (int64_t)tperm[q] : 0;
 #pragma unroll
   for (int k = 0; k < K1; k++) {
-    double v = accn[k];
-#pragma unroll
-    for (int j = 0; j < GROUPS; j++) {
-      double f = accf[j][k];
-      f += __shfl_xor(f, 16, 64);
-      f += __shfl_xor(f, 32, 64);
-      if (g == j) v += f;
-    }
-    if (q < nt) {
-      if (direct) out[t * K1 + k] += v * scale;
-      else out[wg.split * nt * K1 + q * K1 + k] = v;
-    }
+    const double v = acc[k] - comp[k];
+    if (direct) out[t * K1 + k] += v * scale;
+    else out[wg.split * nt * K1 + q * K1 + k] = v;
   }
 }
 
@@ -888,25 +917,29 @@ bool mixed_runs_f64(int ker, int64_t nt, int64_t ns) {
 // tiles prevail.  Dense plan applies, FP32 form / matrix cores, us:
 //                    20000^2 cube   50000^2 cube  90000^2 cube  131072 x 150001  262144^2
 //                                                               clusters         sphere
-//   Stokes FxU       194 / 224      992 / 1039    3025 / 3050   7210 / 6698      24922 / 22008
-//   Stokes DxU       216 / 237      1131 / 1101   3512 / 3238   8521 / 7092      29523 / 23279
-//   Laplace FxdU     149 / 171      741 / 783     2261 / 2239   5367 / 4784      18542 / 15704
+//   Stokes FxU       195 / 203      1013 / 979    3124 / 2911   7682 / 6612      26421 / 22086
+//   Stokes DxU       219 / 216      1170 / 1038   3650 / 3043   8828 / 6840      30768 / 22346
+//   Laplace FxdU     151 / 157      757 / 730     2302 / 2129   5505 / 4696      19090 / 15338
+// Few sources make large tiles, near to more targets: cubes of 400003 x 5000
+// 906 / 1000, 1027 / 1076 and 697 / 763; x 20003 3195 / 3183, 3675 / 3392 and
+// 2353 / 2348; 1500001 x 7001 4991 / 4750, 5411 / 5189 and 4090 / 3559; the
+// other way round, 5000 x 400003, 843 / 789, 978 / 832 and 625 / 590.
 bool far_mfma_at(int ker, int64_t nt, int64_t ns) {
   const double pairs = (double)nt * (double)ns;
   switch (ker) {
     case LAP_FXU:
     case LAP_DXU: return true;
-    case STK_DXU: return pairs >= 3e9;
-    case STK_FXU: return pairs >= 1e10;
-    case LAP_FXDU: return pairs >= 8e9;
+    case STK_DXU: return pairs >= 1e10 || (ns >= 20000 && pairs >= 1e9);
+    case STK_FXU:
+    case LAP_FXDU: return pairs >= 1e10 || (ns >= 20000 && pairs >= 2e9);
     default: return false;
   }
 }
 
 // Launch geometry of one mixed Eval: target blocks and the source splits.
 // Split the sources over gridDim.y when the target blocks cannot fill the
-// device (>= 8 workgroups per CU, each split >= 4 tiles), and so that no
-// split exceeds SPLIT_TILES tiles: workgroups are dispatched in order of
+// device (each split one tile at the least), and so that no split exceeds
+// SPLIT_TILES tiles: workgroups are dispatched in order of
 // their linear index (blockIdx.x fastest), so the ones resident at a time
 // share one split's records (2 MiB for Laplace FxU) in their XCD's 4 MiB L2
 // instead of drifting apart over the whole source array.  The splits' partial
