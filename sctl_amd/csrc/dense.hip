@@ -7,12 +7,13 @@
 // there are too few target blocks to fill the 256 CUs, the source range is
 // split over the grid, down to a fraction of a tile per workgroup
 // (split_sources), and the per-split sums are reduced in split order by a
-// second kernel.  No MFMA: a pairwise sum is not a contraction.
+// second kernel.  No matrix cores: their FP64 rate is the vector rate.
 //
 // FP64 path: each tile is summed over its sources in index order, and the
 // tiles' sums in order (shorter sums than one running accumulator's, so less
-// rounding: Laplace DxU 100003 x 130001, error against 64 bits 2.9e-15 -> 1.0e-15).  A tile whose sum is not finite (some r2 == 0 in that
-// tile) is redone with the r2 > 0 mask.
+// rounding: Laplace DxU 100003 x 130001, error against 64 bits 2.9e-15 ->
+// 1.0e-15).  A tile whose sum is not finite (some r2 == 0 in that tile) is
+// redone with the r2 > 0 mask.
 //
 // The mixed-precision Eval is in mixed.hip.
 #include <hip/hip_runtime.h>
@@ -42,6 +43,9 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
            double scale, double mu) {
   using K = Ker<KER>;
   constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, R = rec_f64<KER>();
+  // Sources per tile.  The Helmholtz kernels' loop runs whole tiles (below), so
+  // theirs are as long as the shortest split.
+  constexpr int TS = needs_ctx(KER) ? 64 : TILE;
   __shared__ double lds[TILE * R];
 
   const int tid = threadIdx.x;
@@ -62,10 +66,10 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
     for (int k = 0; k < K1; k++) tot[j][k] = 0.0;
   }
 
-  for (int64_t sb = s_begin; sb < s_end; sb += TILE) {
-    const int len = (int)(s_end - sb < TILE ? s_end - sb : TILE);
+  for (int64_t sb = s_begin; sb < s_end; sb += TS) {
+    const int len = (int)(s_end - sb < TS ? s_end - sb : TS);
     __syncthreads();
-    for (int i = tid; i < TILE; i += WG) {
+    for (int i = tid; i < TS; i += WG) {
       double* rec = lds + i * R;
       if (i < len) {
         const int64_t s = sb + i;
@@ -120,11 +124,30 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
         else interact<KER, NEWTON, MASK>(acc[j], tx[j] - sx, ty[j] - sy, tz[j] - sz, n, f, mu);
       }
     };
-    // up to the first multiple of UNROLL at or past the tile's last source
-    // (the staged padding covers the rest)
-    for (int i = 0; i < len; i += UNROLL) {
+    if constexpr (needs_ctx(KER)) {
+      // The whole tile, written out: from a loop of variable length, or through
+      // the lambda, the compiler does not keep the sine's and cosine's constants
+      // in registers (Helmholtz FxU 70 -> 83 instructions per pair, 32768^2 2.04
+      // -> 2.28 ms).
+#pragma unroll 2
+      for (int i = 0; i < TS; i++) {
+        const double* rec = lds + i * R;
+        double n[3] = {0, 0, 0}, f[K0];
 #pragma unroll
-      for (int u = 0; u < UNROLL; u++) source(i + u, std::false_type());
+        for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
+#pragma unroll
+        for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
+#pragma unroll
+        for (int j = 0; j < TPL; j++)
+          interact<KER, NEWTON, false>(acc[j], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], n, f, mu);
+      }
+    } else {
+      // up to the first multiple of UNROLL at or past the tile's last source
+      // (the staged padding covers the rest)
+      for (int i = 0; i < len; i += UNROLL) {
+#pragma unroll
+        for (int u = 0; u < UNROLL; u++) source(i + u, std::false_type());
+      }
     }
 
     bool bad = false;
