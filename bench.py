@@ -5,13 +5,15 @@ Workload (one step): GenericKernel<Laplace3D_FxU>::Eval of 1,048,576 sources
 uniform by area on the unit sphere onto 1,048,576 targets uniform in the shell
 1.05 < r < 2, densities N(0,1), seed 0 -- 1.0995e12 interactions -- with the
 inputs already resident in HBM.  The headline value is the mixed-precision
-path (FP64 tile-centred differencing, FP32 pairwise, Kahan FP64 accumulation)
-in G interactions/s; the plain FP64 path is timed on the same inputs and the
-mixed result is checked against it (normwise max and RMS relative error).
+path (FP64 tile-centred differencing, r^2 of far pairs on the matrix cores, FP32
+pairwise, Kahan FP64 accumulation) in G interactions/s; the plain FP64 path is
+timed on the same inputs and the mixed result is checked against it (normwise
+max and RMS relative error).
 A step includes everything Eval does on the device (Hilbert ordering, tile
 packing, the summation kernel).
 
-roofline: the dominant kernel (the pairwise summation) is VALU-bound;
+roofline: the dominant kernel (the pairwise summation) is bound by the issue
+of v_rsq_f32 and of the density FMAs next to the matrix instructions;
 achieved = 11 flop/interaction (3 sub + 5 for r^2 + 1 rsqrt + 2 for the
 density FMA) x interactions per launch / mean launch time, the launch time
 taken from HIP events recorded around that kernel on its own stream.
@@ -46,7 +48,7 @@ PEAK_FP64_TFLOPS = 78.6   # MI355X published FP64 vector peak
 FLOP_PER_INT = {0: 11, 1: 19, 2: 29, 3: 30}  # algorithmic flop per interaction
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_k_eval_mixed_laplace_fxu_sphere_1M.json")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_k_eval_mixed_mfma_laplace_fxu_sphere_1M.json")
 
 
 def measured_traffic(n):
@@ -739,8 +741,7 @@ def main():
                                        stream=stream)
             tuned[name] = {"targets_per_lane": tpl, "wg_per_cu_cap": cap, "ms": round(ms, 3)}
         out.upload(np.zeros(N))
-    hs = S.dense_shape(K, N, N, precision=S.MIXED)
-    headline_kernel = "k_eval_mixed<Laplace3D_FxU, TPL %d>" % hs[0]
+    headline_kernel = "k_eval_mixed_mfma<Laplace3D_FxU>"
     log("mixed precision: %d warmup + %d timed steps (%s)" % (args.warmup, args.steps, headline_kernel))
     hp = S.FP64 if (args.headline_only and args.headline_precision == "fp64") else S.MIXED
     mx = timed_evals(K, dev, out, hp, -1, args.steps, args.warmup, stream)

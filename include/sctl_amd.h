@@ -43,7 +43,7 @@ typedef enum {
   SCTL_AMD_ERROR_NO_DEVICE = 4,      /* no HIP device visible */
   SCTL_AMD_ERROR_OUT_OF_MEMORY = 5,  /* device allocation failed */
   SCTL_AMD_ERROR_HIP = 6,            /* a HIP runtime call failed */
-  SCTL_AMD_ERROR_QUEUE = 7           /* batched work queue did not drain as planned */
+  SCTL_AMD_ERROR_QUEUE = 7           /* no longer returned: batched items are not queued */
 } sctl_amd_status;
 
 /* Micro-kernel ids: the aliases of kernel_functions.hpp:669-684.  r = x_t - x_s;
@@ -74,7 +74,8 @@ enum {
 /* Arithmetic of an evaluation. */
 enum {
   SCTL_AMD_FP64 = 0,  /* FP64 throughout; digits selects the Newton steps after v_rsq_f64 */
-  SCTL_AMD_MIXED = 1, /* FP64 tile-centred differencing, FP32 pairwise, Kahan FP64 accumulation */
+  SCTL_AMD_MIXED = 1, /* FP64 tile-centred differencing, FP32 pairwise, Kahan FP64 accumulation;
+                       * small problems: FP64 at the hardware's rsqrt estimate */
   SCTL_AMD_AUTO = 2   /* MIXED when 0 <= digits <= 7, else FP64 */
 };
 
@@ -230,9 +231,9 @@ int sctl_amd_plan_destroy(sctl_amd_plan plan);
  * (64 * sources_per_lane), targets per lane (1 or 2; kernels with more than
  * 4 outputs per target always run with 1), and a cap on resident workgroups
  * of 4 waves per CU (0 = no cap).  Chosen at creation from the tuning
- * database, else defaults (256-source stages, 2 targets per lane, cap 2 for
- * mixed precision with one output per target, else 4); sctl_amd_plan_tune
- * searches them. */
+ * database, else defaults (128-source stages, 64 for mixed precision with one
+ * output per target; 2 targets per lane; no cap); sctl_amd_plan_tune searches
+ * them. */
 int sctl_amd_plan_get_shape(sctl_amd_plan plan, int* sources_per_lane, int* targets_per_lane, int* wg_per_cu_cap);
 int sctl_amd_plan_set_shape(sctl_amd_plan plan, int sources_per_lane, int targets_per_lane, int wg_per_cu_cap);
 

@@ -30,9 +30,10 @@
 //                source per lane, 64 at a time, the target loop
 //                wave-uniform (targets broadcast from lanes 0..15), so every
 //                row segment written is 64*KDIM0 consecutive doubles;
-//   GEMV         16 rows, 8 at a time, the 64 lanes along the rows (64
-//                consecutive entries of a row per load), the 8 row sums
-//                reduced across the wave by a halving butterfly.
+//   GEMV         8 rows, the 64 lanes along the rows (64 consecutive entries
+//                of a row per load), the 8 row sums reduced across the wave
+//                by a halving butterfly.
+// Where these are too few for the GPU, columns are cut into pieces (near_pieces).
 // Nothing here allocates or issues a memset with device pointers, so the
 // calls can be captured in a hipGraph.
 #include <hip/hip_runtime.h>
