@@ -123,7 +123,7 @@ __device__ __forceinline__ double buffer_load_d(__amdgpu_buffer_rsrc_t r, int of
 // KNearSubtract / store of one layout's blocks.  NDOT: contract the KDIM1
 // outputs with the target normal (KDIM1 == 3 -> one row per target).
 // A wave owns one stripe (MAT_ST targets x the block's sources, or a piece of
-// them where one stripe would outlast the others' work: near_tiles): lanes 0..MAT_ST-1 hold the stripe's targets,
+// them where one stripe would outlast the others' work: near_pieces): lanes 0..MAT_ST-1 hold the stripe's targets,
 // the wave walks the sources 64 at a time (one per lane) and, per chunk,
 // writes every target row's 64*KDIM0 entries.
 //
@@ -422,8 +422,8 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
 // U_near[block rows] = K_near_ * F_element.  Blocks without a matrix
 // (offset < 0) or without sources get zero rows, as the reference's GEMV loop
 // writes them (boundary_integral.txx:1329-1332).  A wave owns GEMV_GR
-// consecutive rows, or a piece of their columns (near_tiles), with its 64
-// lanes along the rows: every load is 64 consecutive
+// consecutive rows, or a piece of their columns, with its 64 lanes along the
+// rows: every load is 64 consecutive
 // entries of one row, each lane's F entries serve all GEMV_GR rows, and two
 // column chunks per step keep 2*GEMV_GR loads in flight.  Rows past the
 // block's last (a tail tile) re-read its last row and columns past the row
@@ -431,85 +431,94 @@ k_near_matrix(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ 
 // the block and no load is predicated.  The GEMV_GR row sums are reduced
 // across the wave by a halving butterfly: each exchange hands half of the
 // rows still held to the partner lane (4 + 2 + 1 + 3 exchanges for 8 rows).
-// Rows whose columns are cut leave partial sums for k_near_gemv_sum.
-__global__ void __launch_bounds__(NWG)
+// The pieces of a row group (1, 2, 4, ... of them, gemv_tiles) are waves of one
+// workgroup and their sums meet in LDS, in piece order: the call has no
+// scratch, so calls on one plan may run side by side on several streams or in
+// graphs.  CUT: some row group has more than one piece.
+template <int WAVES, bool CUT>
+__global__ void __launch_bounds__(64 * WAVES)
 k_near_gemv(const int32_t* __restrict__ tile_blk, const int64_t* __restrict__ tile_dsp,
             const int32_t* __restrict__ tile_piece, int64_t ntiles,
             const int64_t* __restrict__ trg_dsp, const int32_t* __restrict__ trg_cnt,
             const int64_t* __restrict__ src_dsp, const int32_t* __restrict__ src_cnt,
             const int64_t* __restrict__ mat_off, int K0, int dof, const double* __restrict__ K,
-            const double* __restrict__ F, double* __restrict__ U, const int64_t* __restrict__ part_dsp,
-            double* __restrict__ part) {
+            const double* __restrict__ F, double* __restrict__ U) {
   static_assert(GEMV_GR == 8, "the butterfly below reduces 8 rows");
-  const int lane = threadIdx.x & 63;
-  const int64_t nwaves = (int64_t)gridDim.x * (NWG / 64);
-  const int64_t first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (NWG / 64) + (threadIdx.x >> 6)));
-  for (int64_t tile = first; tile < ntiles; tile += nwaves) {
-    const int b = __builtin_amdgcn_readfirstlane(tile_blk[tile]);
-    const int64_t rows = (int64_t)trg_cnt[b] * dof;
-    const int64_t ld = (int64_t)src_cnt[b] * K0;
-    const int64_t off = mat_off[b];
-    const int piece = tile_piece[b];
-    const int npc = (int)max((int64_t)1, (ld + piece - 1) / piece);
-    const int64_t local = tile - tile_dsp[b];
-    const int64_t row0 = local / npc * GEMV_GR, c0 = (local - local / npc * npc) * piece;
-    const int64_t c1 = min(c0 + piece, ld);
-    const double* Fb = F + src_dsp[b] * K0;
-    const int64_t nr = min((int64_t)GEMV_GR, rows - row0);
+  __shared__ double sums[CUT ? WAVES : 1][GEMV_GR];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t nwaves = (int64_t)gridDim.x * WAVES;
+  const int64_t first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * WAVES + wv));
+  // every wave of a workgroup makes the same number of passes
+  for (int64_t tile = first; tile - wv < ntiles; tile += nwaves) {
+    const int b = tile < ntiles ? __builtin_amdgcn_readfirstlane(tile_blk[tile]) : -1;
+    if (!CUT && b < 0) continue;
+    int lg = 0, pc = 0;
+    int64_t nr = 0, row_u = 0;
     double acc[GEMV_GR];
 #pragma unroll
     for (int r = 0; r < GEMV_GR; r++) acc[r] = 0.0;
-    if (off >= 0) {
-      const double* Kr = K + off + row0 * ld;
-      for (int64_t j0 = c0; j0 < c1; j0 += 128) {
-        const int64_t ja = j0 + lane, jb = ja + 64;
-        const int64_t ca = min(ja, c1 - 1), cb = min(jb, c1 - 1);
-        const double fa = ja < c1 ? Fb[ca] : 0.0, fb = jb < c1 ? Fb[cb] : 0.0;
-        double ka[GEMV_GR], kb[GEMV_GR];
+    if (b >= 0) {
+      const int64_t rows = (int64_t)trg_cnt[b] * dof;
+      const int64_t ld = (int64_t)src_cnt[b] * K0;
+      const int64_t off = mat_off[b];
+      const int64_t local = tile - tile_dsp[b];
+      const int piece = tile_piece[b] & ~63;  // columns per piece; log2 of the pieces below
+      lg = CUT ? tile_piece[b] & 63 : 0;
+      pc = (int)(local & ((1 << lg) - 1));
+      const int64_t row0 = (local >> lg) * GEMV_GR, c0 = (int64_t)pc * piece;
+      const int64_t c1 = min(c0 + piece, ld);
+      const double* Fb = F + src_dsp[b] * K0;
+      nr = min((int64_t)GEMV_GR, rows - row0);
+      row_u = trg_dsp[b] * dof + row0;
+      if (off >= 0) {
+        const double* Kr = K + off + row0 * ld;
+        for (int64_t j0 = c0; j0 < c1; j0 += 128) {
+          const int64_t ja = j0 + lane, jb = ja + 64;
+          const int64_t ca = min(ja, c1 - 1), cb = min(jb, c1 - 1);
+          const double fa = ja < c1 ? Fb[ca] : 0.0, fb = jb < c1 ? Fb[cb] : 0.0;
+          double ka[GEMV_GR], kb[GEMV_GR];
 #pragma unroll
-        for (int r = 0; r < GEMV_GR; r++) {
-          const double* Kq = Kr + min((int64_t)r, nr - 1) * ld;
-          ka[r] = Kq[ca];
-          kb[r] = Kq[cb];
-        }
+          for (int r = 0; r < GEMV_GR; r++) {
+            const double* Kq = Kr + min((int64_t)r, nr - 1) * ld;
+            ka[r] = Kq[ca];
+            kb[r] = Kq[cb];
+          }
 #pragma unroll
-        for (int r = 0; r < GEMV_GR; r++) {
-          ka[r] = ja < c1 ? ka[r] : 0.0;
-          kb[r] = jb < c1 ? kb[r] : 0.0;
-          acc[r] = fmad(kb[r], fb, fmad(ka[r], fa, acc[r]));
+          for (int r = 0; r < GEMV_GR; r++) {
+            ka[r] = ja < c1 ? ka[r] : 0.0;
+            kb[r] = jb < c1 ? kb[r] : 0.0;
+            acc[r] = fmad(kb[r], fb, fmad(ka[r], fa, acc[r]));
+          }
         }
       }
-    }
 #pragma unroll
-    for (int h = GEMV_GR / 2, m = 32; h >= 1; h >>= 1, m >>= 1) {
-      const bool up = lane & m;
+      for (int h = GEMV_GR / 2, m = 32; h >= 1; h >>= 1, m >>= 1) {
+        const bool up = lane & m;
 #pragma unroll
-      for (int i = 0; i < h; i++) {
-        const double send = up ? acc[i] : acc[i + h];
-        const double keep = up ? acc[i + h] : acc[i];
-        acc[i] = keep + __shfl_xor(send, m, 64);
+        for (int i = 0; i < h; i++) {
+          const double send = up ? acc[i] : acc[i + h];
+          const double keep = up ? acc[i + h] : acc[i];
+          acc[i] = keep + __shfl_xor(send, m, 64);
+        }
       }
-    }
 #pragma unroll
-    for (int m = 4; m >= 1; m >>= 1) acc[0] += __shfl_xor(acc[0], m, 64);
+      for (int m = 4; m >= 1; m >>= 1) acc[0] += __shfl_xor(acc[0], m, 64);
+    }
     const int rl = lane >> 3;  // row of this lane's sum: bits 5, 4, 3 of the lane
-    if ((lane & 7) == 0 && rl < nr) {
-      if (npc == 1) U[trg_dsp[b] * dof + row0 + rl] = acc[0];
-      else part[part_dsp[b] + (row0 + rl) * npc + c0 / piece] = acc[0];
+    const bool mine = (lane & 7) == 0 && rl < nr;
+    if constexpr (CUT) {
+      if ((lane & 7) == 0) sums[wv][rl] = acc[0];
+      __syncthreads();
+      if (mine && pc == 0) {
+        double s = acc[0];
+        for (int k = 1; k < 1 << lg; k++) s += sums[wv + k][rl];
+        U[row_u + rl] = s;
+      }
+      __syncthreads();  // before the next pass writes
+    } else if (mine) {
+      U[row_u + rl] = acc[0];
     }
   }
-}
-
-// One workgroup per group of up to NWG cut rows: the pieces' sums in order.
-__global__ void __launch_bounds__(NWG)
-k_near_gemv_sum(const SplitRows* __restrict__ groups, const double* __restrict__ part, double* __restrict__ U) {
-  const SplitRows G = groups[blockIdx.x];
-  const int i = threadIdx.x;
-  if (i >= G.rows) return;
-  const double* p = part + G.p + (int64_t)i * G.pieces;
-  double s = 0.0;
-  for (int k = 0; k < G.pieces; k++) s += p[k];
-  U[G.u + i] = s;
 }
 
 // ScatterForward + per-target accumulation: for every target i and every
@@ -562,12 +571,13 @@ NearMatFn near_mat_fn(int ker, bool ndot, bool sub) {
 // to whole 64-column chunks: with all of a block's columns in one tile a few
 // long ones outlasted the rest by far, and few blocks left the GPU idle.  The
 // matrix kernel pays for each cut with a pass of part-filled lines per row, so
-// its share is the smallest that the sweeps of 1 to 6 bear; the GEMV's is 4.
-// MI355X, us before / after:
+// its share is the smallest that the sweeps of 1 to 6 bear; the GEMV's is 4, and
+// its pieces are made powers of two (gemv_tiles).  MI355X, us before / after:
 //   KNearSubtract  Laplace DxU 16 blocks 221 / 20, 64 277 / 54, 300 450 / 412, 512 793 / 795
 //                  Stokes DxU 16 1112 / 83, 60 2257 / 820, 200 3290 / 2366
-//   GEMV           Laplace DxU 16 29 / 9, 64 60 / 24, 300 177 / 159, 512 314 / 309
-//                  Stokes DxU 16 136 / 32, 60 375 / 270, 200 859 / 845
+//   GEMV           Laplace DxU 16 29 / 10, 64 59 / 24, 300 177 / 150, 512 316 / 305
+//                  Stokes DxU 16 136 / 32, 60 375 / 266, 200 857 / 838
+//                  one block of 64 rows of 2^18 columns 3392 / 260
 std::vector<int32_t> near_pieces(const std::vector<int64_t>& cols, const std::vector<int64_t>& groups,
                                  int64_t row_words, int64_t least, int64_t share, int num_cus) {
   int64_t total = 0;
@@ -583,9 +593,10 @@ std::vector<int32_t> near_pieces(const std::vector<int64_t>& cols, const std::ve
 
 // Flattens per-block tile counts into a device tile list, blocks in
 // decreasing order of cost per tile (longest-processing-time first; a
-// block's tiles stay consecutive).
+// block's tiles stay consecutive).  A block's first tile is a multiple of
+// align[b] (where given); the tiles skipped for that belong to block -1.
 int build_tiles(const std::vector<int64_t>& per_block, const std::vector<int64_t>& cost,
-                const std::vector<int32_t>& piece, TileList* out) {
+                const std::vector<int32_t>& piece, TileList* out, const std::vector<int64_t>* align = nullptr) {
   const size_t nb = per_block.size();
   std::vector<size_t> order(nb);
   std::iota(order.begin(), order.end(), 0);
@@ -593,11 +604,12 @@ int build_tiles(const std::vector<int64_t>& per_block, const std::vector<int64_t
   std::vector<int64_t> dsp(nb);
   int64_t total = 0;
   for (size_t b : order) {
-    dsp[b] = total;
-    total += per_block[b];
+    const int64_t a = align && per_block[b] ? (*align)[b] : 1;
+    dsp[b] = (total + a - 1) / a * a;
+    total = dsp[b] + per_block[b];
   }
   SCTL_CHECK_ARG(total < (int64_t)1 << 34, "near-field layout has too many tiles");
-  std::vector<int32_t> blk((size_t)total);
+  std::vector<int32_t> blk((size_t)total, -1);
   for (size_t b = 0; b < nb; b++)
     for (int64_t i = 0; i < per_block[b]; i++) blk[(size_t)(dsp[b] + i)] = (int32_t)b;
   out->ntiles = total;
@@ -607,13 +619,40 @@ int build_tiles(const std::vector<int64_t>& per_block, const std::vector<int64_t
   return SCTL_AMD_SUCCESS;
 }
 
-int tile_grid(int64_t ntiles) {
-  DeviceInfo dev;
-  if (device_info(&dev) != SCTL_AMD_SUCCESS) return 1;
-  const int64_t want = (ntiles + NWG / 64 - 1) / (NWG / 64);
-  return (int)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)dev.num_cus * 64));
+// The GEMV's pieces, n[b] wanted, in waves of one workgroup: the power of two at
+// or above n[b], at most the waves of a workgroup.  Workgroups of four waves, or
+// of sixteen where a row group is wanted in more than four pieces.
+constexpr int GEMV_WAVES = 4, GEMV_WAVES_MAX = 16;
+struct GemvPieces {
+  int waves = GEMV_WAVES;
+  bool cut = false;
+  std::vector<int64_t> count;
+  std::vector<int32_t> code;  // columns per piece (a multiple of 64), log2 of the count in the low bits
+};
+GemvPieces gemv_tiles(const std::vector<int64_t>& cols, const std::vector<int32_t>& piece) {
+  GemvPieces g;
+  const size_t nb = cols.size();
+  g.count.resize(nb);
+  g.code.resize(nb);
+  for (size_t b = 0; b < nb; b++)
+    if (cols[b] > (int64_t)GEMV_WAVES * piece[b]) g.waves = GEMV_WAVES_MAX;
+  for (size_t b = 0; b < nb; b++) {
+    int lg = 0;
+    while ((1 << lg) < g.waves && cols[b] > ((int64_t)piece[b] << lg)) lg++;
+    g.count[b] = (int64_t)1 << lg;
+    g.cut |= lg > 0;
+    const int64_t len = std::max<int64_t>(64, (((cols[b] + g.count[b] - 1) >> lg) + 63) / 64 * 64);
+    g.code[b] = (int32_t)len | lg;
+  }
+  return g;
 }
 
+int tile_grid(int64_t ntiles, int waves = NWG / 64) {
+  DeviceInfo dev;
+  if (device_info(&dev) != SCTL_AMD_SUCCESS) return 1;
+  const int64_t want = (ntiles + waves - 1) / waves;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)dev.num_cus * 256 / waves));
+}
 
 int near_matrix_launch(sctl_amd_plan_s* p, bool sub, const double* wts, const double* n_trg, double* K,
                        hipStream_t s) {
@@ -636,15 +675,13 @@ int near_matrix_launch(sctl_amd_plan_s* p, bool sub, const double* wts, const do
 int near_gemv_launch(sctl_amd_plan_s* p, const double* K, const double* F, double* U, hipStream_t s) {
   if (p->gemv_tiles.ntiles == 0) return SCTL_AMD_SUCCESS;
   ProfileScope prof(s);
-  hipLaunchKernelGGL(k_near_gemv, dim3(tile_grid(p->gemv_tiles.ntiles)), dim3(NWG), 0, s, p->gemv_tiles.d_tile_blk,
-                     p->gemv_tiles.d_tile_dsp, p->gemv_tiles.d_piece, p->gemv_tiles.ntiles, p->d_trg_dsp, p->d_trg_cnt,
-                     p->d_src_dsp, p->d_src_cnt, p->d_near_off, p->K0, p->near_dof, K, F, U, p->d_gemv_part_dsp,
-                     p->d_gemv_part);
+  const auto fn = !p->gemv_cut ? k_near_gemv<GEMV_WAVES, false>
+                               : (p->gemv_waves == GEMV_WAVES ? k_near_gemv<GEMV_WAVES, true>
+                                                              : k_near_gemv<GEMV_WAVES_MAX, true>);
+  hipLaunchKernelGGL(fn, dim3(tile_grid(p->gemv_tiles.ntiles, p->gemv_waves)), dim3(64 * p->gemv_waves), 0, s,
+                     p->gemv_tiles.d_tile_blk, p->gemv_tiles.d_tile_dsp, p->gemv_tiles.d_piece, p->gemv_tiles.ntiles,
+                     p->d_trg_dsp, p->d_trg_cnt, p->d_src_dsp, p->d_src_cnt, p->d_near_off, p->K0, p->near_dof, K, F, U);
   SCTL_HIP_TRY(hipGetLastError());
-  if (p->gemv_nsplit) {
-    hipLaunchKernelGGL(k_near_gemv_sum, dim3(p->gemv_nsplit), dim3(NWG), 0, s, p->d_gemv_split, p->d_gemv_part, U);
-    SCTL_HIP_TRY(hipGetLastError());
-  }
   return SCTL_AMD_SUCCESS;
 }
 
@@ -741,51 +778,33 @@ int sctl_amd_plan_near_layout(sctl_amd_plan p, const int64_t* blk_off, int trg_n
   DeviceInfo dev;
   SCTL_TRY(device_info(&dev));
   const int cus = std::max(dev.num_cus, 1);
-  std::vector<int64_t> mat(nb), gemv(nb), src(nb), cols(nb), cost_m(nb), cost_g(nb), part_dsp(nb, -1);
+  std::vector<int64_t> mat(nb), gemv(nb), src(nb), cols(nb), cost_m(nb), cost_g(nb);
   for (int64_t b = 0; b < nb; b++) {
     const int64_t tc = p->trg_cnt[b], sc = p->src_cnt[b];
     mat[b] = (off[b] >= 0 && tc > 0 && sc > 0) ? (tc + MAT_ST - 1) / MAT_ST : 0;
     gemv[b] = tc > 0 ? (tc * dof + GEMV_GR - 1) / GEMV_GR : 0;
     src[b] = off[b] >= 0 ? sc : 0;
-    cols[b] = src[b] * p->K0;
+    cols[b] = src[b] * p->K0;  // none: zero rows, in one piece
   }
   const std::vector<int32_t> mat_piece = near_pieces(src, mat, (int64_t)MAT_ST * dof * p->K0, 128,
                                                        dof * p->K0 == 1 ? 1 : 2, cus);
-  std::vector<int32_t> gemv_piece = near_pieces(cols, gemv, GEMV_GR, 512, 4, cus);
-  std::vector<SplitRows> split;
-  int64_t part_words = 0;
+  const GemvPieces gp = gemv_tiles(cols, near_pieces(cols, gemv, GEMV_GR, 512, 4, cus));
   for (int64_t b = 0; b < nb; b++) {
     mat[b] *= std::max<int64_t>(1, (src[b] + mat_piece[b] - 1) / mat_piece[b]);
     cost_m[b] = std::min<int64_t>(src[b], mat_piece[b]);
-    if (off[b] < 0) gemv_piece[b] = 0x7fffffff;  // zero rows, in one piece
-    const int64_t n = std::max<int64_t>(1, (cols[b] + gemv_piece[b] - 1) / gemv_piece[b]);
-    cost_g[b] = std::min<int64_t>(cols[b], gemv_piece[b]);
-    gemv[b] *= n;
-    if (n > 1) {
-      part_dsp[b] = part_words;
-      const int64_t rows = p->trg_cnt[b] * dof;
-      for (int64_t r = 0; r < rows; r += NWG)
-        split.push_back(SplitRows{p->trg_dsp[b] * dof + r, part_words + r * n, (int32_t)std::min<int64_t>(NWG, rows - r),
-                                  (int32_t)n});
-      part_words += rows * n;
-    }
+    gemv[b] *= gp.count[b];
+    cost_g[b] = std::min<int64_t>(cols[b], gp.code[b] & ~63);
   }
-  SCTL_CHECK_ARG(split.size() < 0x7fffffffULL, "near-field layout has too many rows");
   p->free_near();
   int rc = dev_upload(&p->d_near_off, off);
   if (!rc) rc = build_tiles(mat, cost_m, mat_piece, &p->mat_tiles);
-  if (!rc) rc = build_tiles(gemv, cost_g, gemv_piece, &p->gemv_tiles);
-  if (!rc) rc = dev_upload(&p->d_gemv_part_dsp, part_dsp);
-  if (!rc) rc = dev_upload(&p->d_gemv_split, split);
-  if (!rc && part_words && hipMalloc(&p->d_gemv_part, sizeof(double) * part_words) != hipSuccess) {
-    set_error("hipMalloc of the near-field partial sums failed");
-    rc = SCTL_AMD_ERROR_OUT_OF_MEMORY;
-  }
+  if (!rc) rc = build_tiles(gemv, cost_g, gp.code, &p->gemv_tiles, &gp.count);
   if (rc) {
     p->free_near();
     return rc;
   }
-  p->gemv_nsplit = (int)split.size();
+  p->gemv_waves = gp.waves;
+  p->gemv_cut = gp.cut;
   p->near_off = off;
   p->near_dof = dof;
   p->near_ndot = trg_normal_dot != 0;

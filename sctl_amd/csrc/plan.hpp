@@ -34,19 +34,13 @@ struct SplitChunk {
 // Wave tiles of the near-field operators, as a flattened list: tile i
 // belongs to block tile_blk[i] and is the (i - tile_dsp[block])-th tile of
 // that block: row groups, each cut into pieces of piece[block] columns
-// (sources for the matrix kernel, matrix columns for the GEMV).
+// (sources for the matrix kernel; for the GEMV, whose pieces are a power of two,
+// matrix columns with log2 of the number of pieces in the low six bits).
 struct TileList {
   int64_t ntiles = 0;
   int32_t* d_tile_blk = nullptr;
   int64_t* d_tile_dsp = nullptr;  // nblocks entries
   int32_t* d_piece = nullptr;     // nblocks entries
-};
-
-// Rows of the GEMV whose columns were cut: U[u + i] is the sum of the `pieces`
-// partial sums part[p + i * pieces ...], i < rows.
-struct SplitRows {
-  int64_t u, p;
-  int32_t rows, pieces;
 };
 
 template <class T> int dev_upload(T** dst, const std::vector<T>& v) {
@@ -93,23 +87,18 @@ struct sctl_amd_plan_s {
   std::vector<int64_t> near_off;
   int64_t* d_near_off = nullptr;
   sctl_amd::TileList mat_tiles, gemv_tiles;
-  int64_t* d_gemv_part_dsp = nullptr;        // per block: its rows' partial sums (-1: rows not cut)
-  sctl_amd::SplitRows* d_gemv_split = nullptr;
-  int gemv_nsplit = 0;
-  double* d_gemv_part = nullptr;
+  int gemv_waves = 4;     // waves per workgroup of the GEMV
+  bool gemv_cut = false;  // some of its row groups are cut into pieces
 
   void free_near() {
     void* ptrs[] = {d_near_off, mat_tiles.d_tile_blk, mat_tiles.d_tile_dsp, mat_tiles.d_piece, gemv_tiles.d_tile_blk,
-                    gemv_tiles.d_tile_dsp, gemv_tiles.d_piece, d_gemv_part_dsp, d_gemv_split, d_gemv_part};
+                    gemv_tiles.d_tile_dsp, gemv_tiles.d_piece};
     for (void* p : ptrs)
       if (p) (void)hipFree(p);
     d_near_off = nullptr;
     mat_tiles = sctl_amd::TileList();
     gemv_tiles = sctl_amd::TileList();
-    d_gemv_part_dsp = nullptr;
-    d_gemv_split = nullptr;
-    d_gemv_part = nullptr;
-    gemv_nsplit = 0;
+    gemv_cut = false;
     has_near = false;
   }
 
