@@ -183,7 +183,8 @@ struct sctl_amd_near_list_s {
   int device = 0;
   int64_t ntrg = 0, nelem = 0, n_near = 0;
   bool has_normal = false;
-  sctl_amd::Block buf;  // all results; its event: the latest read of them, on whichever stream
+  sctl_amd::Block buf;  // all results; its event: after every read so far, whichever their streams
+  std::mutex read;      // a read's wait, launch and record are one step
   double *d_xtn = nullptr, *d_xntn = nullptr;
   int64_t *d_ecnt = nullptr, *d_edsp = nullptr, *d_scatter = nullptr, *d_tcnt = nullptr, *d_tdsp = nullptr;
   ~sctl_amd_near_list_s() { sctl_amd::block_give(buf); }
@@ -852,16 +853,22 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
             {near_elem_cnt, list->d_ecnt, ne},        {near_elem_dsp, list->d_edsp, ne},
             {near_scatter_index, list->d_scatter, n}, {near_trg_cnt, list->d_tcnt, nt},
             {near_trg_dsp, list->d_tdsp, nt}};
-  // Reads of the results follow each other whatever their streams, so that the
-  // list can be destroyed after the last one (a captured read runs later: its
-  // graph needs the list to live, as any graph its buffers).
-  const bool capturing = stream_capturing(s);
-  if (!capturing && list->buf.used) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->buf.used, 0));
-  if (flags & SCTL_AMD_HOST_PTRS) {
+  if (flags & SCTL_AMD_HOST_PTRS) {  // done on return: nothing to order
     for (const auto& x : a)
       if (x.dst && x.src && x.words)
         SCTL_HIP_TRY(hipMemcpyAsync(x.dst, x.src, 8 * (size_t)x.words, hipMemcpyDeviceToHost, s));
-  } else {
+    SCTL_HIP_TRY(hipStreamSynchronize(s));
+    return SCTL_AMD_SUCCESS;
+  }
+  // Reads of the results follow each other whatever their streams and threads, so
+  // that the list's event, recorded after the latest, is after all of them: a
+  // list destroyed then gives its buffer to the next build behind that event
+  // (a captured read runs later: its graph needs the list to live, as any graph
+  // its buffers).
+  std::lock_guard<std::mutex> lock(list->read);
+  const bool capturing = stream_capturing(s);
+  if (!capturing && list->buf.used) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->buf.used, 0));
+  {
     CopyList c;
     int64_t words = 0;
     for (int k = 0; k < 7; k++) {
@@ -876,7 +883,6 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
     }
   }
   if (!capturing && list->buf.used) SCTL_HIP_TRY(hipEventRecord(list->buf.used, s));
-  if (flags & SCTL_AMD_HOST_PTRS) SCTL_HIP_TRY(hipStreamSynchronize(s));
   return SCTL_AMD_SUCCESS;
 }
 
