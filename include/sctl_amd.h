@@ -329,7 +329,9 @@ int sctl_amd_near_list_build(sctl_amd_near_list* list, const double* Xtrg, int64
 /* Number of near pairs (length of near_scatter_index; Xtrg_near has 3x). */
 int sctl_amd_near_list_size(sctl_amd_near_list list, int64_t* n_near);
 /* Copies the results out (host with SCTL_AMD_HOST_PTRS, else device); any
- * output may be NULL.  Xn_trg_near needs a list built with Xn_trg. */
+ * output may be NULL.  Xn_trg_near needs a list built with Xn_trg.  A read into
+ * device memory may be captured into a hipGraph, whose launches need the list:
+ * it may be destroyed once the last of them has been submitted. */
 int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* Xn_trg_near, int64_t* near_elem_cnt,
                            int64_t* near_elem_dsp, int64_t* near_scatter_index, int64_t* near_trg_cnt,
                            int64_t* near_trg_dsp, uint32_t flags, void* stream);

@@ -185,9 +185,13 @@ struct sctl_amd_near_list_s {
   bool has_normal = false;
   sctl_amd::Block buf;  // all results; its event: after every read so far, whichever their streams
   std::mutex read;      // a read's wait, launch and record are one step
+  bool captured = false;  // some read was captured: its graph's launches have no event
   double *d_xtn = nullptr, *d_xntn = nullptr;
   int64_t *d_ecnt = nullptr, *d_edsp = nullptr, *d_scatter = nullptr, *d_tcnt = nullptr, *d_tdsp = nullptr;
-  ~sctl_amd_near_list_s() { sctl_amd::block_give(buf); }
+  ~sctl_amd_near_list_s() {
+    if (captured) sctl_amd::block_drop(buf);  // hipFree waits for a launch under way
+    else sctl_amd::block_give(buf);
+  }
 };
 
 namespace sctl_amd {
@@ -862,11 +866,13 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
   }
   // Reads of the results follow each other whatever their streams and threads, so
   // that the list's event, recorded after the latest, is after all of them: a
-  // list destroyed then gives its buffer to the next build behind that event
-  // (a captured read runs later: its graph needs the list to live, as any graph
-  // its buffers).
+  // list destroyed then gives its buffer to the next build behind that event.  A
+  // captured read runs when its graph does, as often as that is launched, so the
+  // buffer of such a list is freed and not given on (destroy waits for launches
+  // under way; the graph needs the list for others, as any graph its buffers).
   std::lock_guard<std::mutex> lock(list->read);
   const bool capturing = stream_capturing(s);
+  list->captured |= capturing;
   if (!capturing && list->buf.used) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->buf.used, 0));
   {
     CopyList c;

@@ -89,3 +89,41 @@ def test_some_outputs(gpu):
         assert np.array_equal(out[only].download(), want[KEYS[only]])
     lst.get([None] * 6)
     lst.destroy()
+
+
+def test_captured_read(gpu):
+    """A read captured into a graph and replayed between eager reads; the list is destroyed with a launch under way
+    and others are built at once."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def ok(status):
+        assert status == 0
+
+    c = case(4, 300, 40000)
+    want = gpu.near_list(*c)
+    d, other = arrays(gpu, c), arrays(gpu, case(5, 300, 40000))
+    (q,) = streams(gpu, 1)
+    for _ in range(5):
+        lst = Built(gpu, d)
+        out, eager = lst.outputs(), lst.outputs()
+        graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+        ok(hip.hipStreamBeginCapture(q, 2))  # relaxed
+        lst.get(out, q)
+        ok(hip.hipStreamEndCapture(q, ctypes.byref(graph)))
+        ok(hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)))
+        for last in (False, False, True):
+            for o in out:
+                o.upload(np.full(o.shape, -1, o.dtype))
+            ok(hip.hipGraphLaunch(run, q))
+            if last:
+                lst.destroy()
+                for _ in range(2):
+                    Built(gpu, other).destroy()
+            else:
+                lst.get(eager, q)
+            gpu.synchronize(q)
+            for key, o, e in zip(KEYS, out, eager):
+                assert np.array_equal(o.download(), want[key]) and np.array_equal(e.download(), want[key]), key
+        ok(hip.hipGraphExecDestroy(run))
+        ok(hip.hipGraphDestroy(graph))
+    gpu.check(gpu.lib().sctl_amd_stream_destroy(q))
