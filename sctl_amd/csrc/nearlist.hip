@@ -104,8 +104,11 @@ int block_take(size_t bytes, hipStream_t s, Block* out) {
     }
   }
   if (out->p) {
-    SCTL_HIP_TRY(hipStreamWaitEvent(s, out->used, 0));
-    return SCTL_AMD_SUCCESS;
+    const hipError_t e = hipStreamWaitEvent(s, out->used, 0);
+    if (e == hipSuccess) return SCTL_AMD_SUCCESS;
+    block_drop(*out);  // uses that stream s does not wait for
+    *out = Block();
+    SCTL_HIP_TRY(e);
   }
   size_t step = (size_t)1 << 16;  // an eighth of the size's power of two, so that sizes that differ a little reuse
   while (step * 16 <= bytes) step *= 2;
@@ -122,7 +125,13 @@ int block_take(size_t bytes, hipStream_t s, Block* out) {
     out->p = nullptr;
     SCTL_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&out->p), out->bytes));
   }
-  SCTL_HIP_TRY(hipEventCreateWithFlags(&out->used, hipEventDisableTiming));
+  const hipError_t e = hipEventCreateWithFlags(&out->used, hipEventDisableTiming);
+  if (e != hipSuccess) {
+    out->used = nullptr;
+    block_drop(*out);
+    *out = Block();
+  }
+  SCTL_HIP_TRY(e);
   return SCTL_AMD_SUCCESS;
 }
 
@@ -185,11 +194,13 @@ struct sctl_amd_near_list_s {
   bool has_normal = false;
   sctl_amd::Block buf;  // all results; its event: after every read so far, whichever their streams
   std::mutex read;      // a read's wait, launch and record are one step
-  bool captured = false;  // some read was captured: its graph's launches have no event
+  // Some use is not behind buf's event: a captured read (its graph's launches
+  // have none), kernels of a build that failed, a read that failed half-way.
+  bool loose = false;
   double *d_xtn = nullptr, *d_xntn = nullptr;
   int64_t *d_ecnt = nullptr, *d_edsp = nullptr, *d_scatter = nullptr, *d_tcnt = nullptr, *d_tdsp = nullptr;
   ~sctl_amd_near_list_s() {
-    if (captured) sctl_amd::block_drop(buf);  // hipFree waits for a launch under way
+    if (loose) sctl_amd::block_drop(buf);  // hipFree waits for what is under way
     else sctl_amd::block_give(buf);
   }
 };
@@ -650,8 +661,6 @@ int list_alloc(sctl_amd_near_list_s* L, int64_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_nl_zero, dim3(grid_of(words)), dim3(NL_WG), 0, s, L->d_ecnt, words);
     SCTL_HIP_TRY(hipGetLastError());
   }
-  // Until a read is recorded: a failed build destroys its list here.
-  SCTL_HIP_TRY(hipEventRecord(L->buf.used, s));
   return SCTL_AMD_SUCCESS;
 }
 
@@ -827,7 +836,12 @@ int sctl_amd_near_list_build(sctl_amd_near_list* list, const double* Xtrg, int64
                       d.as<double>(), nelem, e.as<int64_t>(), f.as<int64_t>(), s);
     if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = SCTL_AMD_ERROR_HIP;
   }
+  if (!rc && L->buf.used && hipEventRecord(L->buf.used, s) != hipSuccess) {
+    set_error("hipEventRecord failed after a near-list build");
+    rc = SCTL_AMD_ERROR_HIP;
+  }
   if (rc) {
+    L->loose = true;
     delete L;
     return rc;
   }
@@ -858,12 +872,28 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
             {near_scatter_index, list->d_scatter, n}, {near_trg_cnt, list->d_tcnt, nt},
             {near_trg_dsp, list->d_tdsp, nt}};
   if (flags & SCTL_AMD_HOST_PTRS) {  // done on return: nothing to order
+    hipError_t e = hipSuccess;
     for (const auto& x : a)
-      if (x.dst && x.src && x.words)
-        SCTL_HIP_TRY(hipMemcpyAsync(x.dst, x.src, 8 * (size_t)x.words, hipMemcpyDeviceToHost, s));
-    SCTL_HIP_TRY(hipStreamSynchronize(s));
+      if (e == hipSuccess && x.dst && x.src && x.words)
+        e = hipMemcpyAsync(x.dst, x.src, 8 * (size_t)x.words, hipMemcpyDeviceToHost, s);
+    const hipError_t done = hipStreamSynchronize(s);  // also after a failure: copies may be in flight
+    if (done != hipSuccess) {
+      std::lock_guard<std::mutex> lock(list->read);
+      list->loose = true;
+    }
+    SCTL_HIP_TRY(e);
+    SCTL_HIP_TRY(done);
     return SCTL_AMD_SUCCESS;
   }
+  CopyList c;
+  int64_t words = 0;
+  for (int k = 0; k < 7; k++) {
+    words += a[k].dst && a[k].src ? a[k].words : 0;
+    c.src[k] = static_cast<const uint64_t*>(a[k].src);
+    c.dst[k] = static_cast<uint64_t*>(a[k].dst);
+    c.end[k] = words;
+  }
+  if (!words) return SCTL_AMD_SUCCESS;
   // Reads of the results follow each other whatever their streams and threads, so
   // that the list's event, recorded after the latest, is after all of them: a
   // list destroyed then gives its buffer to the next build behind that event.  A
@@ -872,23 +902,14 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
   // under way; the graph needs the list for others, as any graph its buffers).
   std::lock_guard<std::mutex> lock(list->read);
   const bool capturing = stream_capturing(s);
-  list->captured |= capturing;
-  if (!capturing && list->buf.used) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->buf.used, 0));
-  {
-    CopyList c;
-    int64_t words = 0;
-    for (int k = 0; k < 7; k++) {
-      words += a[k].dst && a[k].src ? a[k].words : 0;
-      c.src[k] = static_cast<const uint64_t*>(a[k].src);
-      c.dst[k] = static_cast<uint64_t*>(a[k].dst);
-      c.end[k] = words;
-    }
-    if (words) {
-      hipLaunchKernelGGL(k_nl_copy, dim3(std::min<unsigned>(grid_of(words), 4096)), dim3(NL_WG), 0, s, c);
-      SCTL_HIP_TRY(hipGetLastError());
-    }
-  }
-  if (!capturing && list->buf.used) SCTL_HIP_TRY(hipEventRecord(list->buf.used, s));
+  if (!capturing) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->buf.used, 0));
+  const bool loose = list->loose;
+  list->loose = true;
+  hipLaunchKernelGGL(k_nl_copy, dim3(std::min<unsigned>(grid_of(words), 4096)), dim3(NL_WG), 0, s, c);
+  SCTL_HIP_TRY(hipGetLastError());
+  if (capturing) return SCTL_AMD_SUCCESS;
+  SCTL_HIP_TRY(hipEventRecord(list->buf.used, s));
+  list->loose = loose;
   return SCTL_AMD_SUCCESS;
 }
 
