@@ -631,6 +631,16 @@ __global__ void __launch_bounds__(NL_WG) k_nl_copy(CopyList c) {
   }
 }
 
+// Whether kernels on `device` may write p: memory of another GPU may not be mapped there.
+bool on_device(const void* p, int device) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == device;
+}
+
 unsigned grid_of(int64_t n) { return (unsigned)((n + NL_WG - 1) / NL_WG); }
 
 int bits_for(int64_t n) {
@@ -885,9 +895,15 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
     SCTL_HIP_TRY(done);
     return SCTL_AMD_SUCCESS;
   }
+  // One launch copies all that lies on the list's GPU; outputs elsewhere (another
+  // GPU's memory) take the runtime's copies.
+  int cur = -1;
+  (void)hipGetDevice(&cur);
+  bool here = cur == list->device;
   CopyList c;
   int64_t words = 0;
   for (int k = 0; k < 7; k++) {
+    if (here && a[k].dst && a[k].src && a[k].words) here = on_device(a[k].dst, list->device);
     words += a[k].dst && a[k].src ? a[k].words : 0;
     c.src[k] = static_cast<const uint64_t*>(a[k].src);
     c.dst[k] = static_cast<uint64_t*>(a[k].dst);
@@ -905,8 +921,14 @@ int sctl_amd_near_list_get(sctl_amd_near_list list, double* Xtrg_near, double* X
   if (!capturing) SCTL_HIP_TRY(hipStreamWaitEvent(s, list->buf.used, 0));
   const bool loose = list->loose;
   list->loose = true;
-  hipLaunchKernelGGL(k_nl_copy, dim3(std::min<unsigned>(grid_of(words), 4096)), dim3(NL_WG), 0, s, c);
-  SCTL_HIP_TRY(hipGetLastError());
+  if (here) {
+    hipLaunchKernelGGL(k_nl_copy, dim3(std::min<unsigned>(grid_of(words), 4096)), dim3(NL_WG), 0, s, c);
+    SCTL_HIP_TRY(hipGetLastError());
+  } else {
+    for (const auto& x : a)
+      if (x.dst && x.src && x.words)
+        SCTL_HIP_TRY(hipMemcpyAsync(x.dst, x.src, 8 * (size_t)x.words, hipMemcpyDeviceToDevice, s));
+  }
   if (capturing) return SCTL_AMD_SUCCESS;
   SCTL_HIP_TRY(hipEventRecord(list->buf.used, s));
   list->loose = loose;

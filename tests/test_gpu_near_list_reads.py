@@ -127,3 +127,24 @@ def test_captured_read(gpu):
         ok(hip.hipGraphExecDestroy(run))
         ok(hip.hipGraphDestroy(graph))
     gpu.check(gpu.lib().sctl_amd_stream_destroy(q))
+
+
+def test_outputs_not_on_the_lists_gpu(gpu):
+    """Outputs that are not memory of the list's GPU (one of them here: page-locked host memory) take the runtime's
+    copies instead of the copy kernel."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    c = case(6, 50, 3000)
+    want = gpu.near_list(*c)
+    lst = Built(gpu, arrays(gpu, c))
+    out, p = lst.outputs(), ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(8 * lst.n), 0) == 0
+    ptrs = [o.ptr for o in out]
+    ptrs[3] = p
+    gpu.check(gpu.lib().sctl_amd_near_list_get(lst.h, ptrs[0], None, *ptrs[1:], 0, None))
+    gpu.synchronize()
+    got = [o.download() for o in out]
+    got[3] = np.array((ctypes.c_int64 * lst.n).from_address(p.value))
+    for key, g in zip(KEYS, got):
+        assert np.array_equal(g, want[key]), key
+    lst.destroy()
+    assert hip.hipHostFree(p) == 0
