@@ -382,9 +382,10 @@ k_nl_elements(const int64_t* __restrict__ ecnt, const int64_t* __restrict__ edsp
   int64_t cells = 1;
   for (int d = MAX_DEPTH; d >= 0; d--) {
     shift = MAX_DEPTH - d;
-    cells = 1;
-#pragma unroll
-    for (int k = 0; k < 3; k++) cells *= (int64_t)(qhi[k] >> shift) - (qlo[k] >> shift) + 1;
+    auto span = [&](int k) { return (int64_t)(qhi[k] >> shift) - (qlo[k] >> shift) + 1; };
+    cells = span(0) * span(1);
+    if (cells > MAX_CELLS) continue;  // times span(2) it may wrap: 2^63 for a box that spans the cube
+    cells *= span(2);
     if (cells <= MAX_CELLS) break;
   }
   // Targets of the cells, one cell per lane of wave 0: two binary searches.
