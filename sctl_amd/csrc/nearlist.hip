@@ -716,11 +716,12 @@ int build_pairs(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const dou
                                          (uint32_t*)nullptr, (uint32_t*)nullptr, (size_t)nt, 0, 63, s));
   PairScratch<Key> ps;
   SCTL_TRY(pair_scratch(nt, nelem, usual, &ps));
+  const size_t later_bytes = ps.bytes;
   Carve c;
   const size_t o_cube = c.take(sizeof(double) * 6), o_part = c.take(bounding_box_bytes(nt, ns)),
                o_counter = c.take(sizeof(int64_t)), o_keys_in = c.take(8 * nt), o_keys = c.take(8 * nt),
                o_idx_in = c.take(4 * nt), o_idx = c.take(4 * nt), o_x = c.take(24 * nt), o_tmp = c.take(sort_bytes),
-               o_found = c.take(sizeof(Key) * cap), o_later = c.take(ps.bytes);
+               o_found = c.take(sizeof(Key) * cap), o_later = c.take(later_bytes);
   BlockScratch work, more, later;
   SCTL_TRY(work.alloc(c.bytes, s));
   char* w = work.b.p;
@@ -757,7 +758,7 @@ int build_pairs(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const dou
   }
   char* l = w + o_later;
   SCTL_TRY(pair_scratch(nt, nelem, n, &ps));
-  if (n > usual) {
+  if (ps.bytes > later_bytes) {  // not n > usual: the sorts' shares need not grow with n
     SCTL_TRY(later.alloc(ps.bytes, s));
     l = later.b.p;
   }
