@@ -25,8 +25,9 @@
 //   3. the near ones go out as (element, target) keys, gathered in LDS and
 //      appended through an atomic counter once per element (one atomic per
 //      batch of 64 tests was most of this kernel's time: a single address
-//      takes ~75 per microsecond); the buffer holds 24 pairs per target, and a
-//      list that has more is filled again into one of the size then known;
+//      takes ~75 per microsecond); the buffer holds 24 pairs per target (fewer from
+//      256 MiB on), and a list that has more is filled again into one of the
+//      size then known;
 //   4. the keys are radix sorted (so the list does not depend on the order of
 //      the appends), in 32 bits where an element and a target number fit; each
 //      element's range is found by binary search, and a stable sort of the
@@ -86,6 +87,16 @@ void block_drop(Block b) {  // hipFree waits for the device
   if (cur >= 0 && cur != b.device) (void)hipSetDevice(cur);
 }
 
+// Frees the blocks that are kept.
+void blocks_release() {
+  std::vector<Block> all;
+  {
+    std::lock_guard<std::mutex> lock(g_blocks_mutex);
+    all.swap(free_blocks());
+  }
+  for (Block& b : all) block_drop(b);
+}
+
 // A block of at least `bytes` on the current device, usable on stream s.
 int block_take(size_t bytes, hipStream_t s, Block* out) {
   DeviceInfo dev;
@@ -115,15 +126,15 @@ int block_take(size_t bytes, hipStream_t s, Block* out) {
   out->device = dev.device;
   out->bytes = (bytes + step - 1) / step * step;
   if (hipMalloc(reinterpret_cast<void**>(&out->p), out->bytes) != hipSuccess) {
-    (void)hipGetLastError();  // give back what is kept and try once more
-    std::vector<Block> all;
-    {
-      std::lock_guard<std::mutex> lock(g_blocks_mutex);
-      all.swap(free_blocks());
-    }
-    for (Block& b : all) block_drop(b);
+    (void)hipGetLastError();
+    blocks_release();
     out->p = nullptr;
-    SCTL_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&out->p), out->bytes));
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&out->p), out->bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // the caller may ask for less
+      *out = Block();
+      SCTL_HIP_TRY(e);
+    }
   }
   const hipError_t e = hipEventCreateWithFlags(&out->used, hipEventDisableTiming);
   if (e != hipSuccess) {
@@ -699,42 +710,52 @@ template <class Key> int pair_scratch(int64_t nt, int64_t nelem, int64_t n, Pair
 }
 
 // The build on device arrays of at least one target, node and element.  One
-// scratch allocation as long as the pairs are at most USUAL per target, which
-// the later steps' share of it is sized for: each stream-ordered free costs
-// the host some hundred microseconds here.
+// scratch allocation holds the targets' sort, the pairs found and the steps that
+// follow, as long as the list has at most ROOM and USUAL pairs per target; their
+// shares are bounded (ROOM_BYTES, at least LEAST pairs per target, and
+// USUAL_BYTES).  !reserve (the device's memory did not suffice): no such shares;
+// the first pass over the elements only counts, and what is needed is allocated
+// by size.  The later steps reuse the memory of the targets' sort.
 template <class Key>
 int build_pairs(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const double* xn, const double* xs, int64_t ns,
-                const double* rad, int64_t nelem, const int64_t* ecnt, const int64_t* edsp, hipStream_t s) {
-  constexpr double ROOM = 24, USUAL = 8;  // pairs per target
+                const double* rad, int64_t nelem, const int64_t* ecnt, const int64_t* edsp, bool reserve,
+                hipStream_t s) {
+  constexpr double ROOM = 24, LEAST = 4, USUAL = 8;  // pairs per target
+  constexpr int64_t ROOM_BYTES = (int64_t)256 << 20, USUAL_BYTES = (int64_t)256 << 20;
   auto at_most = [&](double per_target) {
     return (int64_t)std::min<double>((double)nt * (double)nelem, std::max(per_target * (double)nt, 65536.0));
   };
-  int64_t cap = at_most(ROOM), n = 0;
-  const int64_t usual = at_most(USUAL);
   size_t sort_bytes = 0;
   SCTL_HIP_TRY(rocprim::radix_sort_pairs(nullptr, sort_bytes, (uint64_t*)nullptr, (uint64_t*)nullptr,
                                          (uint32_t*)nullptr, (uint32_t*)nullptr, (size_t)nt, 0, 63, s));
+  // The sort of the targets, then their sorted coordinates in place of its inputs.
+  Carve sort;
+  const size_t o_keys_in = sort.take(8 * nt), o_idx_in = sort.take(4 * nt), o_tmp = sort.take(sort_bytes);
+  const size_t sort_region = std::max<size_t>(sort.bytes, 24 * nt);
+  int64_t cap = std::min(at_most(ROOM), std::max<int64_t>(at_most(LEAST), ROOM_BYTES / (int64_t)sizeof(Key))), n = 0;
+  int64_t usual = std::min<int64_t>(at_most(USUAL), USUAL_BYTES / (2 * sizeof(Key) + 24));
+  if (!reserve) cap = usual = 1;
   PairScratch<Key> ps;
   SCTL_TRY(pair_scratch(nt, nelem, usual, &ps));
-  const size_t later_bytes = ps.bytes;
   Carve c;
   const size_t o_cube = c.take(sizeof(double) * 6), o_part = c.take(bounding_box_bytes(nt, ns)),
-               o_counter = c.take(sizeof(int64_t)), o_keys_in = c.take(8 * nt), o_keys = c.take(8 * nt),
-               o_idx_in = c.take(4 * nt), o_idx = c.take(4 * nt), o_x = c.take(24 * nt), o_tmp = c.take(sort_bytes),
-               o_found = c.take(sizeof(Key) * cap), o_later = c.take(later_bytes);
+               o_counter = c.take(sizeof(int64_t)), o_found = c.take(sizeof(Key) * cap),
+               o_keys = c.take(8 * nt),  // from here on the later steps'
+               o_idx = c.take(4 * nt), o_sort = c.take(sort_region);
+  const size_t later_bytes = std::max(ps.bytes, c.bytes - o_keys);
   BlockScratch work, more, later;
-  SCTL_TRY(work.alloc(c.bytes, s));
-  char* w = work.b.p;
-  double *cube = reinterpret_cast<double*>(w + o_cube), *xsorted = reinterpret_cast<double*>(w + o_x);
-  uint64_t *keys_in = reinterpret_cast<uint64_t*>(w + o_keys_in), *keys = reinterpret_cast<uint64_t*>(w + o_keys);
-  uint32_t *idx_in = reinterpret_cast<uint32_t*>(w + o_idx_in), *idx = reinterpret_cast<uint32_t*>(w + o_idx);
+  SCTL_TRY(work.alloc(o_keys + later_bytes, s));
+  char *w = work.b.p, *a = w + o_sort;
+  double *cube = reinterpret_cast<double*>(w + o_cube), *xsorted = reinterpret_cast<double*>(a);
+  uint64_t *keys_in = reinterpret_cast<uint64_t*>(a + o_keys_in), *keys = reinterpret_cast<uint64_t*>(w + o_keys);
+  uint32_t *idx_in = reinterpret_cast<uint32_t*>(a + o_idx_in), *idx = reinterpret_cast<uint32_t*>(w + o_idx);
   int64_t* counter = reinterpret_cast<int64_t*>(w + o_counter);
   Key* found = reinterpret_cast<Key*>(w + o_found);
   SCTL_TRY(bounding_box(xt, nt, xs, ns, cube, w + o_part, s));
   hipLaunchKernelGGL(k_nl_cube, dim3(1), dim3(64), 0, s, cube, cube);
   hipLaunchKernelGGL(k_nl_keys, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, cube, keys_in, idx_in);
   SCTL_HIP_TRY(hipGetLastError());
-  SCTL_HIP_TRY(rocprim::radix_sort_pairs(w + o_tmp, sort_bytes, keys_in, keys, idx_in, idx, (size_t)nt, 0, 63, s));
+  SCTL_HIP_TRY(rocprim::radix_sort_pairs(a + o_tmp, sort_bytes, keys_in, keys, idx_in, idx, (size_t)nt, 0, 63, s));
   hipLaunchKernelGGL(k_nl_gather, dim3(grid_of(nt)), dim3(NL_WG), 0, s, xt, nt, idx, xsorted);
   SCTL_HIP_TRY(hipGetLastError());
   for (int pass = 0; pass < 2; pass++) {
@@ -756,7 +777,7 @@ int build_pairs(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const dou
     SCTL_HIP_TRY(hipStreamSynchronize(s));
     return SCTL_AMD_SUCCESS;
   }
-  char* l = w + o_later;
+  char* l = w + o_keys;
   SCTL_TRY(pair_scratch(nt, nelem, n, &ps));
   if (ps.bytes > later_bytes) {  // not n > usual: the sorts' shares need not grow with n
     SCTL_TRY(later.alloc(ps.bytes, s));
@@ -788,9 +809,13 @@ int build_list(sctl_amd_near_list_s* L, const double* xt, int64_t nt, const doub
     SCTL_HIP_TRY(hipStreamSynchronize(s));
     return SCTL_AMD_SUCCESS;
   }
-  if (bits_for(nt) < 32 && bits_for(nt) + bits_for(nelem) <= 32)
-    return build_pairs<uint32_t>(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, s);
-  return build_pairs<uint64_t>(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, s);
+  auto build = bits_for(nt) < 32 && bits_for(nt) + bits_for(nelem) <= 32 ? build_pairs<uint32_t> : build_pairs<uint64_t>;
+  const int rc = build(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, true, s);
+  if (rc != SCTL_AMD_ERROR_OUT_OF_MEMORY) return rc;
+  block_drop(L->buf);  // hipFree waits for what is under way
+  L->buf = Block();
+  blocks_release();
+  return build(L, xt, nt, xn, xs, ns, rad, nelem, ecnt, edsp, false, s);
 }
 
 }  // namespace
