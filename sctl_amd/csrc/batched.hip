@@ -577,7 +577,7 @@ int plan_configure(sctl_amd_plan_s* p, PlanShape s) {
       if (q) SCTL_HIP_TRY(hipFree(q));
     SCTL_TRY(dev_upload(&p->d_items, w.items));
     SCTL_TRY(dev_upload(&p->d_split, w.split));
-    if (w.part_words) SCTL_HIP_TRY(hipMalloc(&p->d_part, sizeof(double) * w.part_words));
+    if (w.part_words) SCTL_TRY(device_malloc(reinterpret_cast<void**>(&p->d_part), sizeof(double) * w.part_words));
     p->nitems = (int)w.items.size();
     p->nsplit = (int)w.split.size();
   }
@@ -730,7 +730,7 @@ int sctl_amd_plan_set_geometry(sctl_amd_plan p, const double* r_trg, const doubl
   const hipMemcpyKind kind = (flags & SCTL_AMD_HOST_PTRS) ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
   auto copy = [&](double** dst, const double* src, int64_t n) -> int {
     if (n <= 0) return SCTL_AMD_SUCCESS;
-    if (!*dst) SCTL_HIP_TRY(hipMalloc(dst, sizeof(double) * n));
+    if (!*dst) SCTL_TRY(device_malloc(reinterpret_cast<void**>(dst), sizeof(double) * n));
     SCTL_HIP_TRY(hipMemcpyAsync(*dst, src, sizeof(double) * n, kind, s));
     return SCTL_AMD_SUCCESS;
   };

@@ -82,6 +82,18 @@ double kernel_scale(int ker) {
   return 0;
 }
 
+int device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    blocks_release();
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) *p = nullptr;
+  SCTL_HIP_TRY(e);
+  return SCTL_AMD_SUCCESS;
+}
+
 bool kernel_needs_ctx(int ker) { return needs_ctx(ker); }
 
 int kernel_max_tpl(int ker) {
@@ -475,8 +487,7 @@ int sctl_amd_malloc(void** ptr, size_t bytes) {
   DeviceInfo dev;
   SCTL_TRY(device_info(&dev));
   if (!bytes) return SCTL_AMD_SUCCESS;
-  SCTL_HIP_TRY(hipMalloc(ptr, bytes));
-  return SCTL_AMD_SUCCESS;
+  return device_malloc(ptr, bytes);
 }
 
 int sctl_amd_free(void* ptr) {

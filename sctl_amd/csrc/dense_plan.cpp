@@ -51,8 +51,7 @@ namespace {
 int dev_alloc(void** p, size_t bytes) {
   *p = nullptr;
   if (!bytes) return SCTL_AMD_SUCCESS;
-  SCTL_HIP_TRY(hipMalloc(p, bytes));
-  return SCTL_AMD_SUCCESS;
+  return device_malloc(p, bytes);
 }
 
 int dense_plan_apply_dev(sctl_amd_dense_plan_s* p, const double* v_src, double* v_trg, hipStream_t s) {

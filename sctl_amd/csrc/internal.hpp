@@ -50,6 +50,11 @@ int device_info(DeviceInfo* out);  // for the current device
 // threshold); beyond it, memory goes back to the driver at synchronisation.
 constexpr uint64_t POOL_KEEP_BYTES = (uint64_t)4 << 30;
 
+// Memory that the library keeps without using it (near lists' blocks), freed:
+// called where an allocation failed, before it is tried once more.
+void blocks_release();
+int device_malloc(void** p, size_t bytes);  // hipMalloc
+
 // Stream-ordered device scratch: allocated from the library's pool on the
 // current device, freed on the same stream.
 class Scratch {
@@ -64,7 +69,14 @@ class Scratch {
     if (!bytes) return SCTL_AMD_SUCCESS;
     DeviceInfo dev;
     SCTL_TRY(device_info(&dev));
-    SCTL_HIP_TRY(hipMallocFromPoolAsync(&ptr_, bytes, dev.pool, s));
+    hipError_t e = hipMallocFromPoolAsync(&ptr_, bytes, dev.pool, s);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      blocks_release();
+      e = hipMallocFromPoolAsync(&ptr_, bytes, dev.pool, s);
+    }
+    if (e != hipSuccess) ptr_ = nullptr;
+    SCTL_HIP_TRY(e);
     bytes_ = bytes;
     return SCTL_AMD_SUCCESS;
   }

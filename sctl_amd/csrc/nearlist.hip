@@ -58,7 +58,8 @@ namespace {
 
 // Device memory of near lists (a build's scratch, a list's results) kept for
 // the next build: up to KEEP_BLOCKS blocks and KEEP_BYTES per device, the
-// oldest given back beyond that.  A block carries an event recorded after its
+// oldest given back beyond that, all of them where an allocation of the library
+// fails (blocks_release).  A block carries an event recorded after its
 // last use; whoever takes it makes its stream wait for that event, so threads
 // and streams share the blocks freely.  (The stream-ordered pool, asked for
 // such buffers again while the last read of the previous ones was under way,
@@ -87,7 +88,8 @@ void block_drop(Block b) {  // hipFree waits for the device
   if (cur >= 0 && cur != b.device) (void)hipSetDevice(cur);
 }
 
-// Frees the blocks that are kept.
+}  // namespace
+
 void blocks_release() {
   std::vector<Block> all;
   {
@@ -96,6 +98,8 @@ void blocks_release() {
   }
   for (Block& b : all) block_drop(b);
 }
+
+namespace {
 
 // A block of at least `bytes` on the current device, usable on stream s.
 int block_take(size_t bytes, hipStream_t s, Block* out) {

@@ -46,7 +46,7 @@ struct TileList {
 template <class T> int dev_upload(T** dst, const std::vector<T>& v) {
   *dst = nullptr;
   if (v.empty()) return SCTL_AMD_SUCCESS;
-  SCTL_HIP_TRY(hipMalloc(dst, sizeof(T) * v.size()));
+  SCTL_TRY(device_malloc(reinterpret_cast<void**>(dst), sizeof(T) * v.size()));
   SCTL_HIP_TRY(hipMemcpy(*dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
   return SCTL_AMD_SUCCESS;
 }

@@ -16,6 +16,24 @@ pytestmark = pytest.mark.gpu
 NT, NEAR, NELEM = 30_000_000, 1200, 200
 
 
+def fill_but(hip, free):
+    """Takes the device's memory but for `free` bytes; returns the blocks."""
+    have, total, hold, fill = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_void_p(), []
+    assert hip.hipMemGetInfo(ctypes.byref(have), ctypes.byref(total)) == 0
+    if free:
+        assert hip.hipMalloc(ctypes.byref(hold), ctypes.c_size_t(int(free))) == 0
+    size = have.value
+    while size >= 1 << 24:  # the rest, in blocks of halving size
+        p = ctypes.c_void_p()
+        if hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size)) == 0:
+            fill.append(p)
+        else:
+            size //= 2
+    if free:
+        assert hip.hipFree(hold) == 0
+    return fill
+
+
 @pytest.mark.parametrize("free", [2.0e9, 2.4e9, 5.0e9])
 def test_little_memory(gpu, free):
     hip = ctypes.CDLL("libamdhip64.so")
@@ -29,17 +47,7 @@ def test_little_memory(gpu, free):
     d = [gpu.DeviceArray.from_host(a.ravel()) for a in (xt, xs, rad)]
     d += [gpu.DeviceArray.from_host(a, dtype=np.int64) for a in (cnt, dsp)]
     gpu.synchronize()
-    have, total, hold, fill = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_void_p(), []
-    assert hip.hipMemGetInfo(ctypes.byref(have), ctypes.byref(total)) == 0
-    assert hip.hipMalloc(ctypes.byref(hold), ctypes.c_size_t(int(free))) == 0
-    size = have.value
-    while size >= 1 << 24:  # the rest, in blocks of halving size
-        p = ctypes.c_void_p()
-        if hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size)) == 0:
-            fill.append(p)
-        else:
-            size //= 2
-    assert hip.hipFree(hold) == 0
+    fill = fill_but(hip, free)
     try:
         got = gpu.near_list(*d)
     finally:
@@ -51,3 +59,19 @@ def test_little_memory(gpu, free):
     for key in ("near_trg_cnt", "near_trg_dsp"):
         assert np.array_equal(got[key][at], want[key]), key
         assert np.count_nonzero(got[key]) == np.count_nonzero(want[key]), key
+
+
+def test_kept_memory_goes_to_other_allocations(gpu):
+    """The blocks kept between builds, more than a gigabyte here, are freed when another allocation fails."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(2)
+    d = [gpu.DeviceArray.from_host(a) for a in (2.0 + rng.random(3 * NT), rng.random(3), np.array([0.1]))]
+    d += [gpu.DeviceArray.from_host(np.array([a]), dtype=np.int64) for a in (1, 0)]
+    assert gpu.near_list(*d)["near_scatter_index"].size == 0
+    fill = fill_but(hip, 0)
+    try:
+        a = gpu.DeviceArray(1 << 30, np.uint8)
+        a.free()
+    finally:
+        for p in fill:
+            assert hip.hipFree(p) == 0
