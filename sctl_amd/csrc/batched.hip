@@ -558,32 +558,36 @@ BlocksFn plan_fn(const sctl_amd_plan_s* p, const PlanShape& s) {
 }  // namespace
 
 // Applies knobs to a plan: rebuilds the work items for the targets per lane
-// and sizes the dynamic LDS that enforces the cap on resident workgroups.
+// and sizes the dynamic LDS that enforces the cap on resident workgroups.  A plan
+// that cannot have them stays as it was.
 int plan_configure(sctl_amd_plan_s* p, PlanShape s) {
   DeviceInfo dev;
   SCTL_TRY(device_info(&dev));
   s.spl = s.spl >= 4 ? 4 : (s.spl >= 2 ? 2 : 1);
   s.tpl = s.tpl >= 2 && plan_max_tpl(p->kernel) >= 2 ? 2 : 1;
   s.occ = std::max(0, s.occ);
+  size_t dyn = 0;
+  SCTL_TRY(occupancy_lds((const void*)plan_fn(p, s), s.occ, blocks_lds(p->kernel, p->precision, s.spl), &dyn));
   if (!p->d_items || s.tpl != p->shape.tpl) {
     const WorkList w = build_items(p, s.tpl, std::max(dev.num_cus, 1));
     SCTL_CHECK_ARG(w.items.size() < 0x7fffffffULL, "too many work items");
-    p->nitems = p->nsplit = 0;
-    void* old[] = {p->d_items, p->d_split, p->d_part};
-    p->d_items = nullptr;
-    p->d_split = nullptr;
-    p->d_part = nullptr;
-    for (void* q : old)
-      if (q) SCTL_HIP_TRY(hipFree(q));
-    SCTL_TRY(dev_upload(&p->d_items, w.items));
-    SCTL_TRY(dev_upload(&p->d_split, w.split));
-    if (w.part_words) SCTL_TRY(device_malloc(reinterpret_cast<void**>(&p->d_part), sizeof(double) * w.part_words));
-    p->nitems = (int)w.items.size();
-    p->nsplit = (int)w.split.size();
+    Item* items = nullptr;
+    SplitChunk* split = nullptr;
+    double* part = nullptr;
+    int rc = dev_upload(&items, w.items);
+    if (!rc) rc = dev_upload(&split, w.split);
+    if (!rc && w.part_words) rc = device_malloc(reinterpret_cast<void**>(&part), sizeof(double) * w.part_words);
+    if (!rc) {
+      std::swap(p->d_items, items);
+      std::swap(p->d_split, split);
+      std::swap(p->d_part, part);
+      p->nitems = (int)w.items.size();
+      p->nsplit = (int)w.split.size();
+    }
+    for (void* q : {(void*)items, (void*)split, (void*)part})  // the old ones, or what could be had of the new
+      if (q) (void)hipFree(q);
+    if (rc) return rc;
   }
-  const BlocksFn fn = plan_fn(p, s);
-  size_t dyn = 0;
-  SCTL_TRY(occupancy_lds((const void*)fn, s.occ, blocks_lds(p->kernel, p->precision, s.spl), &dyn));
   p->dyn_lds = dyn;
   p->shape = s;
   p->generation++;

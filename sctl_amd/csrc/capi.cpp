@@ -89,7 +89,10 @@ int device_malloc(void** p, size_t bytes) {
     blocks_release();
     e = hipMalloc(p, bytes);
   }
-  if (e != hipSuccess) *p = nullptr;
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();  // reported here, and not by the next launch's check
+  }
   SCTL_HIP_TRY(e);
   return SCTL_AMD_SUCCESS;
 }

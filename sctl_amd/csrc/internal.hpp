@@ -75,7 +75,10 @@ class Scratch {
       blocks_release();
       e = hipMallocFromPoolAsync(&ptr_, bytes, dev.pool, s);
     }
-    if (e != hipSuccess) ptr_ = nullptr;
+    if (e != hipSuccess) {
+      ptr_ = nullptr;
+      (void)hipGetLastError();  // reported here, and not by the next launch's check
+    }
     SCTL_HIP_TRY(e);
     bytes_ = bytes;
     return SCTL_AMD_SUCCESS;

@@ -47,7 +47,12 @@ template <class T> int dev_upload(T** dst, const std::vector<T>& v) {
   *dst = nullptr;
   if (v.empty()) return SCTL_AMD_SUCCESS;
   SCTL_TRY(device_malloc(reinterpret_cast<void**>(dst), sizeof(T) * v.size()));
-  SCTL_HIP_TRY(hipMemcpy(*dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+  const hipError_t e = hipMemcpy(*dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    (void)hipFree(*dst);
+    *dst = nullptr;
+  }
+  SCTL_HIP_TRY(e);
   return SCTL_AMD_SUCCESS;
 }
 

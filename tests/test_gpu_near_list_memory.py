@@ -29,6 +29,7 @@ def fill_but(hip, free):
             fill.append(p)
         else:
             size //= 2
+    hip.hipGetLastError()  # the failed attempts'
     if free:
         assert hip.hipFree(hold) == 0
     return fill
