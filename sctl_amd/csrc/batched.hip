@@ -485,10 +485,7 @@ size_t blocks_lds(int ker, int precision, int spl) {
   int K0, K1, ND;
   kernel_dims(ker, &K0, &K1, &ND);
   const size_t stage = 64 * (size_t)spl * (BWG / 64);
-  if (precision == SCTL_AMD_MIXED) {
-    if (ker == LAP_DXU) return stage * (6 * sizeof(double) + sizeof(float));  // s, f n; one unused float
-    return stage * (4 * sizeof(double) + (((ND + K0) + 3) & ~3) * sizeof(float));
-  }
+  if (precision == SCTL_AMD_MIXED) return stage * (4 * sizeof(double) + (((ND + K0) + 3) & ~3) * sizeof(float));
   return stage * (ker == LAP_DXU ? 6 : ((3 + ND + K0) + 1) & ~1) * sizeof(double);
 }
 }  // namespace
