@@ -106,7 +106,7 @@ k_blocks_f64(const Item* __restrict__ items, int nitems,
              const double* __restrict__ fs, double* __restrict__ out, double* __restrict__ part, double scale,
              double mu) {
   using K = Ker<KER>;
-  constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, R = rec_f64<KER>(), STAGE = 64 * SPL;
+  constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, R = rec_f64<KER, KER == LAP_DXU>(), STAGE = 64 * SPL;
   __shared__ double lds_all[(BWG / 64) * STAGE * R];
   const int lane = threadIdx.x & 63;
   double* lds = lds_all + (threadIdx.x >> 6) * (STAGE * R);

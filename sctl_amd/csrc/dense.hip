@@ -42,7 +42,11 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
            const double* __restrict__ fs, int64_t ns, int64_t chunk, double* __restrict__ out, int direct,
            double scale, double mu) {
   using K = Ker<KER>;
-  constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, R = rec_f64<KER>();
+  // The double layer stages f n, one multiplication per pair fewer, but for the
+  // full-precision sums of few sources (FOLD_SOURCES): f n is rounded, which
+  // n.r near 0 enlarges.
+  constexpr bool FN = KER == LAP_DXU && NEWTON != 2;
+  constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, R = rec_f64<KER, FN>();
   // Sources per tile.  The Helmholtz kernels' loop runs whole tiles (below), so
   // theirs are as long as the shortest split.
   constexpr int TS = needs_ctx(KER) ? 64 : TILE;
@@ -76,7 +80,7 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
         rec[0] = xs[s * 3 + 0];
         rec[1] = xs[s * 3 + 1];
         rec[2] = xs[s * 3 + 2];
-        if constexpr (KER == LAP_DXU) {
+        if constexpr (FN) {
           const double f = fs[s];
 #pragma unroll
           for (int k = 0; k < 3; k++) rec[3 + k] = f * xn[s * 3 + k];
@@ -111,15 +115,15 @@ k_eval_f64(const double* __restrict__ xt, int64_t nt, const double* __restrict__
 #pragma unroll
       for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
 #pragma unroll
-      for (int k = 0; k < (KER == LAP_DXU ? 0 : K0); k++) f[k] = rec[3 + ND + k];
-      if constexpr (KER == LAP_DXU && MASK) {
+      for (int k = 0; k < (FN ? 0 : K0); k++) f[k] = rec[3 + ND + k];
+      if constexpr (FN && MASK) {
 #pragma unroll
         for (int k = 0; k < 3; k++) n[k] = xn[(sb + i) * 3 + k];
         f[0] = fs[sb + i];
       }
 #pragma unroll
       for (int j = 0; j < TPL; j++) {
-        if constexpr (KER == LAP_DXU && !MASK)
+        if constexpr (FN && !MASK)
           lap_dxu_fn<NEWTON, false>(acc[j][0], tx[j] - sx, ty[j] - sy, tz[j] - sz, n);
         else interact<KER, NEWTON, MASK>(acc[j], tx[j] - sx, ty[j] - sy, tz[j] - sz, n, f, mu);
       }
@@ -299,11 +303,25 @@ template <int KER, int NEWTON> EvalF64Fn f64_fn(int ti) {
 EvalF64Fn f64_fn(int ker, int newton, int ti) {
   return with_kernel(ker, [&](auto kc) {
     constexpr int K = decltype(kc)::value;
+    if constexpr (Ker<K>::POW != 0) {
+      if (newton == FOLDED) return f64_fn<K, FOLDED>(ti);
+    }
     return newton == 0 ? f64_fn<K, 0>(ti) : (newton == 1 ? f64_fn<K, 1>(ti) : f64_fn<K, 2>(ti));
   });
 }
-int rec_words_f64(int ker) {
-  return with_kernel(ker, [](auto kc) { return rec_f64<decltype(kc)::value>(); });
+// The full-precision kernels of one power of 1/r take the shorter form of the
+// rsqrt (FOLDED) and the double layer's f n from this many sources on.  Below, a
+// target's sum is at most two tiles' and their roundings show in it; above, the
+// sums by tiles round less than the one running sum of all sources that they
+// replaced.  rms error over the sum of magnitudes in 1e-16, the longer forms in
+// one running sum / the shorter ones, 2000 to 20000 targets:
+//   Laplace DxU  4 sources 1.69 / 1.99, 64 1.20 / 1.28, 512 1.65 / 0.84, 16384 1.21 / 0.49
+//   Stokes DxU   4 2.79 / 3.36, 64 1.62 / 1.86, 512 1.83 / 1.17, 16384 0.88 / 0.47
+//   Laplace FxdU 4 1.59 / 1.90, 64 1.17 / 1.26, 512 1.68 / 0.80, 16384 0.93 / 0.37
+constexpr int64_t FOLD_SOURCES = 512;
+int f64_step(int ker, int newton, int64_t ns) {
+  const bool one_power = with_kernel(ker, [](auto kc) { return Ker<decltype(kc)::value>::POW != 0; });
+  return newton == 2 && one_power && ns >= FOLD_SOURCES ? FOLDED : newton;
 }
 int max_tpl_index(int ker) {
   return with_kernel(ker, [](auto kc) { return tpl_index(max_tpl<decltype(kc)::value>()); });
@@ -381,10 +399,11 @@ int f64_apply(int ker, int newton, const double* r_trg, int64_t nt, const double
   split_sources(tb, ns, dev.num_cus, &nsplit, &chunk);
   const int64_t group = split_group(nsplit, sizeof(double) * (size_t)nt * K1, part_budget);
   SCTL_CHECK_ARG(group <= 1 || part, "no buffer for the split partial sums");
-  const double scale = (double)(kernel_scale(ker) * fold_factor(ker, newton));
-  const EvalF64Fn fn = f64_fn(ker, newton, ti);
+  const int step = f64_step(ker, newton, ns);
+  const double scale = (double)(kernel_scale(ker) * fold_factor(ker, step));
+  const EvalF64Fn fn = f64_fn(ker, step, ti);
   size_t dyn = 0;
-  SCTL_TRY(occupancy_lds((const void*)fn, shape.occ, sizeof(double) * TILE * rec_words_f64(ker), &dyn));
+  SCTL_TRY(occupancy_lds((const void*)fn, shape.occ, 0, &dyn));
   if (!stream_capturing(stream)) profile_count(ker, nt * ns);
   // Groups of `group` splits: sources [y0*chunk, (y0+gy)*chunk) per launch.
   for (int64_t y0 = 0; y0 < nsplit; y0 += group) {

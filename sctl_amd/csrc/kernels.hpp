@@ -98,9 +98,8 @@ template <int KER> constexpr int max_tpl() { return Ker<KER>::K1 <= 3 ? 4 : (Ker
 // Words per packed source record: position, normal (if any), density.
 template <int KER> constexpr int src_words() { return 3 + Ker<KER>::ND + Ker<KER>::K0; }
 // Record widths padded to 16 bytes (LDS reads of 128 bits).
-// The Laplace double layer's FP64 record holds f n in place of n and f
-// (lap_dxu_fn).
-template <int KER> constexpr int rec_f64() { return KER == LAP_DXU ? 6 : (src_words<KER>() + 1) & ~1; }
+// FN: the Laplace double layer's record with f n in place of n and f (lap_dxu_fn).
+template <int KER, bool FN = false> constexpr int rec_f64() { return FN ? 6 : (src_words<KER>() + 1) & ~1; }
 template <int KER> constexpr int rec_f32() { return (src_words<KER>() + 3) & ~3; }
 
 __device__ __forceinline__ double hw_rsq(double x) { return __builtin_amdgcn_rsq(x); }
@@ -272,37 +271,40 @@ __device__ __forceinline__ void helmholtz_factor(T r2, T z, T mu, T* G0, T* G1) 
 
 // Deferred-scaling constants.  NEWTON = 1: intrin-wrapper.hpp:540-559.
 // NEWTON = 2 (full FP64 precision) is not two deferred steps here but one
-// third-order step in one of two forms (rsq_deferred): FOLD = true leaves the
-// factor 1 / h0 of the completed square to the caller, FOLD = false needs no
-// factor.
+// third-order step, which needs no factor; NEWTON = FOLDED is that step in a form
+// that leaves the factor 1 / h0 to the caller (rsq_deferred).
+constexpr int FOLDED = 3;
 constexpr double CUBIC_E = 5.0 / 3.0, CUBIC_H = 20.0 / 9.0;
 __host__ __device__ constexpr double newton_c1(int j) { return j == 0 ? -3.0 : (j == 1 ? -12.0 : -768.0); }
 __host__ __device__ constexpr double newton_c2(int n) { return n == 1 ? -0.5 : 1.0; }
 __host__ __device__ constexpr long double ipow(long double x, int p) { return p == 0 ? 1.0L : x * ipow(x, p - 1); }
 
 // Unscaled rsqrt: equals c^-1 / sqrt(x) up to rounding, with c =
-// newton_c2(NEWTON), or 1 / h0 for NEWTON 2 with FOLD.
+// newton_c2(NEWTON), or 1 / h0 for FOLDED.
 //   NEWTON 0: the hardware estimate (v_rsq_f64 / v_rsq_f32, ~2^-23 relative);
 //   NEWTON 1: one deferred Newton step z (x z^2 - 3) (= -2 / sqrt(x), ~2^-47);
 //   NEWTON 2: the third-order step z (1 + e/2 + 3 e^2 / 8), e = 1 - x z^2,
 //             the first terms of (1 - e)^(-1/2) (Householder's method of
 //             order 3): error ~ (5/16) e^3 ~ 2^-70, i.e. rounding only, in 5
-//             operations instead of the 6 of two deferred Newton steps.
-//             With FOLD the polynomial's square is completed,
+//             operations instead of the 6 of two deferred Newton steps;
+//   FOLDED:   the same with the polynomial's square completed,
 //               1 + e/2 + 3 e^2 / 8 = ((e + 2/3)^2 + 20/9) 3/8,
 //             and the 3/8 left out: 4 operations (x z, e + 2/3 in one FMA,
 //             the square in another, the product).  Its value at e = 0, h0 =
 //             (CUBIC_E - 1)^2 + CUBIC_H = 8/3 up to rounding, is divided out
 //             by fold_factor.  The FP64 kernels of one power of 1/r are bound
 //             by VALU issue, so the operation counts in time: Laplace FxU 16
-//             -> 15 issue slots per pair (v_rsq_f64 takes four).
-template <int NEWTON, bool FOLD = false, class T> __device__ __forceinline__ T rsq_deferred(T x) {
+//             -> 15 issue slots per pair (v_rsq_f64 takes four).  It rounds
+//             twice at full size where the other form rounds once (rms error
+//             7.5e-17 instead of 5.1e-17), which only sums of many sources
+//             hide (dense.hip, FOLD_SOURCES).
+template <int NEWTON, class T> __device__ __forceinline__ T rsq_deferred(T x) {
   T z = hw_rsq(x);
   if constexpr (NEWTON == 1) z = z * fmad(x, z * z, (T)newton_c1(0));
-  if constexpr (NEWTON >= 2 && FOLD) {
+  if constexpr (NEWTON == FOLDED) {
     const T e = fmad(-(x * z), z, (T)CUBIC_E);
     z = z * fmad(e, e, (T)CUBIC_H);
-  } else if constexpr (NEWTON >= 2) {
+  } else if constexpr (NEWTON == 2) {
     const T e = fmad(-(x * z), z, (T)1);
     z = fmad(z * e, fmad(e, (T)0.375, (T)0.5), z);
   }
@@ -314,12 +316,13 @@ template <int NEWTON, bool FOLD = false, class T> __device__ __forceinline__ T r
 // others (scaled in-loop).
 template <int KER, int NEWTON> __host__ __device__ constexpr long double fold_factor() {
   constexpr long double e0 = (long double)CUBIC_E - 1, h0 = e0 * e0 + (long double)CUBIC_H;
-  return Ker<KER>::POW ? ipow(NEWTON >= 2 ? 1 / h0 : (long double)newton_c2(NEWTON), Ker<KER>::POW) : 1.0L;
+  return Ker<KER>::POW ? ipow(NEWTON == FOLDED ? 1 / h0 : (long double)newton_c2(NEWTON), Ker<KER>::POW) : 1.0L;
 }
 inline long double fold_factor(int ker, int newton) {
   return with_kernel(ker, [&](auto kc) {
     constexpr int K = decltype(kc)::value;
-    return newton == 0 ? fold_factor<K, 0>() : (newton == 1 ? fold_factor<K, 1>() : fold_factor<K, 2>());
+    return newton == 0 ? fold_factor<K, 0>()
+                       : (newton == 1 ? fold_factor<K, 1>() : (newton == 2 ? fold_factor<K, 2>() : fold_factor<K, FOLDED>()));
   });
 }
 
@@ -328,7 +331,7 @@ inline long double fold_factor(int ker, int newton) {
 template <int NEWTON, bool MASK>
 __device__ __forceinline__ void lap_dxu_fn(double& acc, double rx, double ry, double rz, const double* fn) {
   const double r2 = fmad(rz, rz, fmad(ry, ry, rx * rx));
-  double z = rsq_deferred<NEWTON, true>(r2);
+  double z = rsq_deferred<NEWTON>(r2);
   if constexpr (MASK) z = r2 > 0.0 ? z : 0.0;
   const double nd = fmad(rz, fn[2], fmad(ry, fn[1], rx * fn[0]));
   acc = fmad(nd, z * z * z, acc);
@@ -340,7 +343,8 @@ __device__ __forceinline__ void lap_dxu_fn(double& acc, double rx, double ry, do
 template <int KER, int NEWTON, bool MASK, class T>
 __device__ __forceinline__ void interact(T* acc, T rx, T ry, T rz, const T* n, const T* f, T mu = (T)0) {
   const T r2 = fmad(rz, rz, fmad(ry, ry, rx * rx));
-  T z = rsq_deferred<NEWTON, Ker<KER>::POW != 0>(r2);
+  static_assert(NEWTON != FOLDED || Ker<KER>::POW != 0, "the factor would have to be applied per pair");
+  T z = rsq_deferred<NEWTON>(r2);
   if constexpr (MASK) z = (r2 > (T)0) ? z : (T)0;
   if constexpr (KER == LAP_FXU) {
     acc[0] = fmad(z, f[0], acc[0]);
