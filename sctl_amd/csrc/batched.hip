@@ -104,8 +104,9 @@ k_blocks_f64(const Item* __restrict__ items, int nitems,
              const int64_t* __restrict__ trg_dsp, const int64_t* __restrict__ src_dsp,
              const double* __restrict__ xt, const double* __restrict__ xs, const double* __restrict__ xn,
              const double* __restrict__ fs, double* __restrict__ out, double* __restrict__ part, double scale,
-             double mu) {
+             double scale_folded, double mu) {
   using K = Ker<KER>;
+  constexpr bool FOLDS = NEWTON == 2 && K::POW != 0;  // items with ITEM_FOLDED have the FOLDED rsqrt
   constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, R = rec_f64<KER, KER == LAP_DXU>(), STAGE = 64 * SPL;
   __shared__ double lds_all[(BWG / 64) * STAGE * R];
   const int lane = threadIdx.x & 63;
@@ -114,7 +115,8 @@ k_blocks_f64(const Item* __restrict__ items, int nitems,
   const int first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (BWG / 64) + (threadIdx.x >> 6)));
   for (int64_t it = first; it < nitems; it += (int64_t)gridDim.x * (BWG / 64)) {
     const Item I = items[it];
-    const int lg = I.lg, G = 1 << lg, L = 64 >> lg;
+    const bool folded = FOLDS && (I.lg & ITEM_FOLDED);
+    const int lg = FOLDS ? I.lg & (ITEM_FOLDED - 1) : I.lg, G = 1 << lg, L = 64 >> lg;
     const int g = lane >> (6 - lg), tl = lane & (L - 1);
     const int64_t tb = trg_dsp[I.block] + I.t_off;
     bool tv[TPL];
@@ -159,23 +161,32 @@ k_blocks_f64(const Item* __restrict__ items, int nitems,
       for (int j = 0; j < TPL; j++)
 #pragma unroll
         for (int k = 0; k < K1; k++) acc[j][k] = 0.0;
-      group_sources<STAGE>(lg, g, len, [&](int i) {
-        const double* rec = lds + i * R;
-        if constexpr (KER == LAP_DXU) {
-#pragma unroll
-          for (int j = 0; j < TPL; j++)
-            lap_dxu_fn<NEWTON, false>(acc[j][0], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], rec + 3);
-        } else {
-          double n[3] = {0, 0, 0}, f[K0];
-#pragma unroll
-          for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
-#pragma unroll
-          for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
-#pragma unroll
-          for (int j = 0; j < TPL; j++)
-            interact<KER, NEWTON, false>(acc[j], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], n, f, mu);
-        }
-      });
+      auto sum = [&](auto step) {
+        constexpr int N = decltype(step)::value;
+        group_sources<STAGE>(lg, g, len, [&](int i) {
+          const double* rec = lds + i * R;
+          if constexpr (KER == LAP_DXU) {
+  #pragma unroll
+            for (int j = 0; j < TPL; j++)
+              lap_dxu_fn<N, false>(acc[j][0], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], rec + 3);
+          } else {
+            double n[3] = {0, 0, 0}, f[K0];
+  #pragma unroll
+            for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
+  #pragma unroll
+            for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
+  #pragma unroll
+            for (int j = 0; j < TPL; j++)
+              interact<KER, N, false>(acc[j], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], n, f, mu);
+          }
+        });
+      };
+      if constexpr (FOLDS) {
+        if (folded) sum(std::integral_constant<int, FOLDED>());
+        else sum(std::integral_constant<int, NEWTON>());
+      } else {
+        sum(std::integral_constant<int, NEWTON>());
+      }
       bool bad = false;
 #pragma unroll
       for (int j = 0; j < TPL; j++)
@@ -186,20 +197,29 @@ k_blocks_f64(const Item* __restrict__ items, int nitems,
         for (int j = 0; j < TPL; j++)
 #pragma unroll
           for (int k = 0; k < K1; k++) acc[j][k] = 0.0;
-        for (int i = g; i < len; i += G) {
-          const double* rec = lds + i * R;
-          if constexpr (KER == LAP_DXU) {
-#pragma unroll
-            for (int j = 0; j < TPL; j++)
-              lap_dxu_fn<NEWTON, true>(acc[j][0], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], rec + 3);
-          } else {
-            double n[3] = {0, 0, 0}, f[K0];
-            for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
-            for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
-#pragma unroll
-            for (int j = 0; j < TPL; j++)
-              interact<KER, NEWTON, true>(acc[j], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], n, f, mu);
+        auto redo = [&](auto step) {
+          constexpr int N = decltype(step)::value;
+          for (int i = g; i < len; i += G) {
+            const double* rec = lds + i * R;
+            if constexpr (KER == LAP_DXU) {
+  #pragma unroll
+              for (int j = 0; j < TPL; j++)
+                lap_dxu_fn<N, true>(acc[j][0], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], rec + 3);
+            } else {
+              double n[3] = {0, 0, 0}, f[K0];
+              for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
+              for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
+  #pragma unroll
+              for (int j = 0; j < TPL; j++)
+                interact<KER, N, true>(acc[j], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], n, f, mu);
+            }
           }
+        };
+        if constexpr (FOLDS) {
+          if (folded) redo(std::integral_constant<int, FOLDED>());
+          else redo(std::integral_constant<int, NEWTON>());
+        } else {
+          redo(std::integral_constant<int, NEWTON>());
         }
       }
 #pragma unroll
@@ -215,7 +235,7 @@ k_blocks_f64(const Item* __restrict__ items, int nitems,
       if (g == 0 && tv[j]) {
 #pragma unroll
         for (int k = 0; k < K1; k++) {
-          if (I.part < 0) out[t[j] * K1 + k] += tot[j][k] * scale;
+          if (I.part < 0) out[t[j] * K1 + k] += tot[j][k] * (folded ? scale_folded : scale);
           else part[I.part + (int64_t)(tl + j * L) * K1 + k] = tot[j][k];
         }
       }
@@ -269,7 +289,7 @@ k_blocks_mixed(const Item* __restrict__ items, int nitems,
                const int64_t* __restrict__ trg_dsp, const int64_t* __restrict__ src_dsp,
                const double* __restrict__ xt, const double* __restrict__ xs, const double* __restrict__ xn,
                const double* __restrict__ fs, double* __restrict__ out, double* __restrict__ part, double scale,
-               double ctx) {
+               double, double ctx) {
   const float mu = (float)ctx;
   using K = Ker<KER>;
   constexpr int K0 = K::K0, K1 = K::K1, ND = K::ND, STAGE = 64 * SPL;
@@ -414,9 +434,10 @@ k_blocks_mixed(const Item* __restrict__ items, int nitems,
 // One workgroup per chunk that was cut into pieces: out += scale * (the sum of
 // the pieces' partial sums, in piece order).
 __global__ void __launch_bounds__(SWG)
-k_sum_pieces(const SplitChunk* __restrict__ chunks, int K1, const double* __restrict__ part, double* __restrict__ out,
-             double scale) {
+k_sum_pieces(const SplitChunk* __restrict__ chunks, int K1, const double* __restrict__ part,
+             double* __restrict__ out) {
   const SplitChunk C = chunks[blockIdx.x];
+  const double scale = C.scale;
   const int n = C.t_cnt * K1;
   if (C.pieces > 32) {  // few targets, many pieces: four lanes per value
     for (int i0 = 0; i0 < n; i0 += SWG / 4) {
@@ -441,7 +462,7 @@ k_sum_pieces(const SplitChunk* __restrict__ chunks, int K1, const double* __rest
 }
 
 using BlocksFn = void (*)(const Item*, int, const int64_t*, const int64_t*, const double*, const double*,
-                          const double*, const double*, double*, double*, double, double);
+                          const double*, const double*, double*, double*, double, double, double);
 
 // Targets per lane: 1 or 2 (2 only where max_tpl allows it).
 template <int KER, int NEWTON, int SPL> BlocksFn f64_blocks_t(int tpl) {
@@ -509,8 +530,13 @@ struct WorkList {
   std::vector<SplitChunk> split;
   int64_t part_words = 0;
 };
+double plan_scale(const sctl_amd_plan_s* p, bool folded) {
+  return (double)(kernel_scale(p->kernel) * fold_factor(p->kernel, folded ? FOLDED : p->newton));
+}
+
 WorkList build_items(const sctl_amd_plan_s* p, int tpl, int num_cus) {
   WorkList w;
+  const bool folds = p->precision != SCTL_AMD_MIXED && p->newton == 2 && one_power(p->kernel);
   const int64_t chunk = 64LL * tpl;
   auto groups = [&](int64_t cnt) { return cnt <= 16 * tpl ? 2 : (cnt <= 32 * tpl ? 1 : 0); };
   int64_t total = 0;
@@ -530,10 +556,13 @@ WorkList build_items(const sctl_amd_plan_s* p, int tpl, int num_cus) {
       int64_t n = (lanes * sc + piece_cost - 1) / piece_cost;
       const int64_t len = ((sc + n - 1) / n + 63) / 64 * 64;
       n = (sc + len - 1) / len;
-      if (n > 1) w.split.push_back(SplitChunk{p->trg_dsp[b] + t0, w.part_words, cnt, (int32_t)n});
+      const bool folded = folds && (sc >> lg) >= FOLD_SOURCES;
+      if (n > 1)
+        w.split.push_back(SplitChunk{p->trg_dsp[b] + t0, w.part_words, cnt, (int32_t)n, plan_scale(p, folded)});
       for (int64_t i = 0; i < n; i++) {
         const int64_t s0 = i * len, sn = std::min<int64_t>(len, sc - s0);
-        items.push_back(Item{(int32_t)b, (int32_t)t0, cnt, lg, (int32_t)s0, (int32_t)sn, n > 1 ? w.part_words : -1});
+        items.push_back(Item{(int32_t)b, (int32_t)t0, cnt, lg + (folded ? ITEM_FOLDED : 0), (int32_t)s0, (int32_t)sn,
+                             n > 1 ? w.part_words : -1});
         cost.push_back(lanes * sn);
         if (n > 1) w.part_words += (int64_t)cnt * p->K1;
       }
@@ -610,18 +639,18 @@ int plan_launch(sctl_amd_plan_s* p, const double* v_src, double* v_trg, hipStrea
   if (p->nitems == 0) return SCTL_AMD_SUCCESS;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   SCTL_HIP_TRY(hipStreamIsCapturing(s, &cs));
-  const double scale = (double)(kernel_scale(p->kernel) * fold_factor(p->kernel, p->newton));
   // Four items per workgroup; past 2^22 workgroups (a grid of 2^30 threads) they loop.
   const unsigned grid = (unsigned)std::min<int64_t>(1 << 22, ((int64_t)p->nitems + BWG / 64 - 1) / (BWG / 64));
   if (cs == hipStreamCaptureStatusNone) profile_count(p->kernel, p->interactions);  // graphs count per launch
   {
     ProfileScope prof(s);
     hipLaunchKernelGGL(plan_fn(p, p->shape), dim3(grid), dim3(BWG), p->dyn_lds, s, p->d_items, p->nitems,
-                       p->d_trg_dsp, p->d_src_dsp, p->d_xt, p->d_xs, p->d_xn, v_src, v_trg, p->d_part, scale, p->ctx);
+                       p->d_trg_dsp, p->d_src_dsp, p->d_xt, p->d_xs, p->d_xn, v_src, v_trg, p->d_part, plan_scale(p, false),
+                       plan_scale(p, true), p->ctx);
   }
   SCTL_HIP_TRY(hipGetLastError());
   if (p->nsplit) {
-    hipLaunchKernelGGL(k_sum_pieces, dim3(p->nsplit), dim3(SWG), 0, s, p->d_split, p->K1, p->d_part, v_trg, scale);
+    hipLaunchKernelGGL(k_sum_pieces, dim3(p->nsplit), dim3(SWG), 0, s, p->d_split, p->K1, p->d_part, v_trg);
     SCTL_HIP_TRY(hipGetLastError());
   }
   return SCTL_AMD_SUCCESS;

@@ -309,19 +309,8 @@ EvalF64Fn f64_fn(int ker, int newton, int ti) {
     return newton == 0 ? f64_fn<K, 0>(ti) : (newton == 1 ? f64_fn<K, 1>(ti) : f64_fn<K, 2>(ti));
   });
 }
-// The full-precision kernels of one power of 1/r take the shorter form of the
-// rsqrt (FOLDED) and the double layer's f n from this many sources on.  Below, a
-// target's sum is at most two tiles' and their roundings show in it; above, the
-// sums by tiles round less than the one running sum of all sources that they
-// replaced.  rms error over the sum of magnitudes in 1e-16, the longer forms in
-// one running sum / the shorter ones, 2000 to 20000 targets:
-//   Laplace DxU  4 sources 1.69 / 1.99, 64 1.20 / 1.28, 512 1.65 / 0.84, 16384 1.21 / 0.49
-//   Stokes DxU   4 2.79 / 3.36, 64 1.62 / 1.86, 512 1.83 / 1.17, 16384 0.88 / 0.47
-//   Laplace FxdU 4 1.59 / 1.90, 64 1.17 / 1.26, 512 1.68 / 0.80, 16384 0.93 / 0.37
-constexpr int64_t FOLD_SOURCES = 512;
 int f64_step(int ker, int newton, int64_t ns) {
-  const bool one_power = with_kernel(ker, [](auto kc) { return Ker<decltype(kc)::value>::POW != 0; });
-  return newton == 2 && one_power && ns >= FOLD_SOURCES ? FOLDED : newton;
+  return newton == 2 && one_power(ker) && ns >= FOLD_SOURCES ? FOLDED : newton;
 }
 int max_tpl_index(int ker) {
   return with_kernel(ker, [](auto kc) { return tpl_index(max_tpl<decltype(kc)::value>()); });

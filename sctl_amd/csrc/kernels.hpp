@@ -297,7 +297,7 @@ __host__ __device__ constexpr long double ipow(long double x, int p) { return p 
 //             -> 15 issue slots per pair (v_rsq_f64 takes four).  It rounds
 //             twice at full size where the other form rounds once (rms error
 //             7.5e-17 instead of 5.1e-17), which only sums of many sources
-//             hide (dense.hip, FOLD_SOURCES).
+//             hide (FOLD_SOURCES).
 template <int NEWTON, class T> __device__ __forceinline__ T rsq_deferred(T x) {
   T z = hw_rsq(x);
   if constexpr (NEWTON == 1) z = z * fmad(x, z * z, (T)newton_c1(0));
@@ -317,6 +317,20 @@ template <int NEWTON, class T> __device__ __forceinline__ T rsq_deferred(T x) {
 template <int KER, int NEWTON> __host__ __device__ constexpr long double fold_factor() {
   constexpr long double e0 = (long double)CUBIC_E - 1, h0 = e0 * e0 + (long double)CUBIC_H;
   return Ker<KER>::POW ? ipow(NEWTON == FOLDED ? 1 / h0 : (long double)newton_c2(NEWTON), Ker<KER>::POW) : 1.0L;
+}
+// The full-precision FP64 kernels of one power of 1/r take the shorter form of the
+// rsqrt (FOLDED), and the dense double layer f n, from this many sources per lane
+// on.  Below, a target's sum is at most two tiles' and their roundings show in
+// it; above, the sums by tiles round less than the one running sum of all sources
+// that they replaced.  rms error over the sum of magnitudes in 1e-16, the longer forms in
+// one running sum / the shorter ones, 2000 to 20000 targets:
+//   Laplace DxU  4 sources 1.69 / 1.99, 64 1.20 / 1.28, 512 1.65 / 0.84, 16384 1.21 / 0.49
+//   Stokes DxU   4 2.79 / 3.36, 64 1.62 / 1.86, 512 1.83 / 1.17, 16384 0.88 / 0.47
+//   Laplace FxdU 4 1.59 / 1.90, 64 1.17 / 1.26, 512 1.68 / 0.80, 16384 0.93 / 0.37
+constexpr int64_t FOLD_SOURCES = 512;
+
+inline bool one_power(int ker) {
+  return with_kernel(ker, [](auto kc) { return Ker<decltype(kc)::value>::POW != 0; });
 }
 inline long double fold_factor(int ker, int newton) {
   return with_kernel(ker, [&](auto kc) {

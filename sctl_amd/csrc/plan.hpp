@@ -11,13 +11,14 @@
 
 namespace sctl_amd {
 
+constexpr int32_t ITEM_FOLDED = 4;
 // One work item of the batched Eval: a chunk of one block's targets against a
 // piece of the block's sources.
 struct Item {
   int32_t block;  // block index
   int32_t t_off;  // first target of the chunk, relative to the block
   int32_t t_cnt;  // targets in the chunk (<= 64*TPL)
-  int32_t lg;     // log2 of the number of lane groups
+  int32_t lg;     // log2 of the number of lane groups; + ITEM_FOLDED: the FOLDED rsqrt
   int32_t s_off;  // first source of the piece, relative to the block
   int32_t s_cnt;  // sources in the piece
   int64_t part;   // where the piece's sums go in the partial sums; -1: the only piece, added to the output
@@ -29,6 +30,7 @@ struct SplitChunk {
   int64_t t_base;  // first target of the chunk in the plan's target array
   int64_t part;    // the first piece's partial sums
   int32_t t_cnt, pieces;
+  double scale;    // of the sums
 };
 
 // Wave tiles of the near-field operators, as a flattened list: tile i

@@ -55,3 +55,30 @@ def test_both_forms(gpu, k, ns):
     out = gpu.eval(k, xt, xs, n, v)
     assert np.abs(out - ref).max() <= 2e-14 * size
     assert np.array_equal(gpu.DensePlan(k, xt, xs, n).apply(v), out)
+
+
+@pytest.mark.parametrize("k", [0, 1, 3, 4, 7, 10])
+def test_blocks_of_both_forms(gpu, k):
+    """A plan whose blocks' lanes sum fewer and more sources than that, in one piece and in several, with one, two and
+    four lane groups."""
+    rng = np.random.default_rng(k)
+    _, K0, K1, _, _ = oracle.dims(k)
+    tc = np.array([128, 128, 5, 20, 30, 16, 128, 50, 300])
+    sc = np.array([511, 512, 513, 2047, 2048, 2049, 5000, 1024, 1])
+    td, sd = (np.concatenate(([0], np.cumsum(a)[:-1])) for a in (tc, sc))
+    xt, xs, n = rng.random(3 * tc.sum()), rng.random(3 * sc.sum()), rng.standard_normal(3 * sc.sum())
+    v = rng.standard_normal(K0 * sc.sum())
+    for b in range(tc.size):  # a coincident pair in each block
+        xt[3 * td[b]:3 * td[b] + 3] = xs[3 * (sd[b] + sc[b]) - 3:3 * (sd[b] + sc[b])]
+    P = gpu.Plan(k, td, tc, sd, sc, int(tc.sum()), int(sc.sum()))
+    P.set_geometry(xt, xs, n)
+    for tpl in (2, 1):
+        P.set_shape(2, tpl, 0)
+        out = P.apply(v, np.zeros(K1 * tc.sum()))
+        for b in range(tc.size):
+            t, s = slice(3 * td[b], 3 * (td[b] + tc[b])), slice(3 * sd[b], 3 * (sd[b] + sc[b]))
+            f = v[K0 * sd[b]:K0 * (sd[b] + sc[b])]
+            ref = oracle.eval(k, xt[t], xs[s], n[s], f)
+            size = np.max(np.abs(oracle.kernel_matrix(k, xt[t], xs[s], n[s])).T @ np.abs(f))
+            # 5000 terms in sums of at most 128, their roundings relative to partial sums
+            assert np.abs(out[K1 * td[b]:K1 * (td[b] + tc[b])] - ref).max() <= 2e-14 * size, (tpl, b)
