@@ -462,37 +462,39 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 // A kernel's far form.  NV: dot products with t' - s' beside r^2 (DxU: nq;
 // Stokes: f, and n for the double layer).  GRAD: outputs along r = t' - s',
-// summed as t'_k (sum g) - (sum g s'_k).  NROW: FP32 words per source that the
-// pairs read besides (s' where GRAD, then the densities).
+// summed as t'_k (sum g) - (sum g s'_k).  T64: |t'|^2 is formed in FP64 and rounded
+// once, where 1/r^3 or 1/r^5 would carry its error, one for all of a tile's
+// pairs, into the sum (it costs the single layer 0.2 %).  NROW: FP32 words per
+// source that the pairs read besides (s' where GRAD, then the densities).
 template <int KER> struct FarForm {
   static constexpr bool ON = false;
   static constexpr int NV = 0, NROW = 0;
-  static constexpr bool GRAD = false;
+  static constexpr bool GRAD = false, T64 = false;
 };
 template <> struct FarForm<LAP_FXU> {
   static constexpr bool ON = true;
   static constexpr int NV = 0, NROW = 1;
-  static constexpr bool GRAD = false;
+  static constexpr bool GRAD = false, T64 = false;
 };
 template <> struct FarForm<LAP_DXU> {
   static constexpr bool ON = true;
   static constexpr int NV = 1, NROW = 0;
-  static constexpr bool GRAD = false;
+  static constexpr bool GRAD = false, T64 = true;
 };
 template <> struct FarForm<LAP_FXDU> {
   static constexpr bool ON = true;
   static constexpr int NV = 0, NROW = 4;
-  static constexpr bool GRAD = true;
+  static constexpr bool GRAD = true, T64 = true;
 };
 template <> struct FarForm<STK_FXU> {
   static constexpr bool ON = true;
   static constexpr int NV = 1, NROW = 6;
-  static constexpr bool GRAD = true;
+  static constexpr bool GRAD = true, T64 = false;
 };
 template <> struct FarForm<STK_DXU> {
   static constexpr bool ON = true;
   static constexpr int NV = 2, NROW = 3;
-  static constexpr bool GRAD = true;
+  static constexpr bool GRAD = true, T64 = true;
 };
 template <int KER> constexpr bool far_mfma() { return FarForm<KER>::ON; }
 // |t'|^2 below this takes the FP32 forms: the matrix cores may flush parts
@@ -585,7 +587,7 @@ __device__ __forceinline__ void far_pair(float* p, float& G, float r2, const flo
     const float g = KER == LAP_FXDU ? row(3) * z * z2 : (d[0] * z2) * (d[1] * z2) * z;
 #pragma unroll
     for (int k = 0; k < 3; k++) p[k] = fmad(-g, row(k), p[k]);
-    G += g;
+    G = g;
   }
 }
 
@@ -691,8 +693,10 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
     }
     __syncthreads();
 
-    const float th[3] = {(float)(t64[0] - m.x), (float)(t64[1] - m.y), (float)(t64[2] - m.z)};
-    const float T = fmad(th[2], th[2], fmad(th[1], th[1], th[0] * th[0]));
+    const double t[3] = {t64[0] - m.x, t64[1] - m.y, t64[2] - m.z};
+    const float th[3] = {(float)t[0], (float)t[1], (float)t[2]};
+    const float T = F::T64 ? (float)fmad(t[2], t[2], fmad(t[1], t[1], t[0] * t[0]))
+                           : fmad(th[2], th[2], fmad(th[1], th[1], th[0] * th[0]));
     const float H2 = (float)m.w;
     u32x4 col[GROUPS];  // lane group g: axis g (3: |t'|^2) of the targets q0 + 16 j + (lane & 15)
     float cx[GROUPS] = {th[0], th[1], th[2], T};
@@ -732,13 +736,21 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
           f32x4 dots[NV ? NV : 1];
 #pragma unroll
           for (int v = 0; v < NV; v++) dots[v] = mfma16(av[v], col[j], v4[v]);
+          // The four g of g r are added up first: G's rounding is |t'| / H times that of
+          // the sums of g s' in the outputs.  With T64 and the outputs' FP64 t': error
+          // against FP64 for sets apart (FP32 form / before / now) Stokes DxU 3.6 / 4.0 /
+          // 3.6e-7, Laplace FxdU 3.1 / 3.1 / 2.3e-7; sphere 2.48 / 2.52 / 2.49 and 1.83 /
+          // 1.82 / 1.76e-7; the same time.
+          constexpr bool BY4 = F::GRAD && KER != STK_FXU;
+          float g4[4];
 #pragma unroll
           for (int i = 0; i < 4; i++) {
             float d[NV ? NV : 1];
 #pragma unroll
             for (int v = 0; v < NV; v++) d[v] = i & 1 ? -dots[v][i] : dots[v][i];
-            far_pair<KER, NEWTON>(pf[j], pG[j], r2[i], d, [&](int k) { return w4[k][i]; });
+            far_pair<KER, NEWTON>(pf[j], BY4 ? g4[i] : pG[j], r2[i], d, [&](int k) { return w4[k][i]; });
           }
+          if constexpr (BY4) pG[j] += (g4[0] + g4[1]) + (g4[2] + g4[3]);
         }
       }
     };
@@ -816,9 +828,9 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
     for (int k = 0; k < K1; k++) {
       ptn[k] += sum_rows(pf[0][k], pf[1][k], pf[2][k], pf[3][k]);
       if constexpr (F::GRAD) {
-        float x = th[k];
-        asm volatile("" : "+v"(x));  // or the conversion is done in each pass of the far loop
-        ptn[k] = fmad((double)x, Gt, ptn[k]);
+        double x = t64[k];
+        asm volatile("" : "+v"(x));  // or the difference is held through the far loop
+        ptn[k] = fmad(x - (k == 0 ? m.x : (k == 1 ? m.y : m.z)), Gt, ptn[k]);
       }
       const double y = ptn[k] - comp[k];  // Kahan: acc += ptn
       const double sum = acc[k] + y;
