@@ -131,8 +131,65 @@ __device__ __forceinline__ void mix_near(float* p, const float* th, const float*
   }
 }
 
+// A kernel's far form on the matrix cores (k_eval_mixed_mfma).  NV: dot products
+// with t' - s' beside r^2 (DxU: nq; Stokes: f, and n for the double layer).  GRAD:
+// outputs along r = t' - s', summed as t'_k (sum g) - (sum g s'_k).  T64: |t'|^2 is
+// formed in FP64 and rounded once, and the outputs take t' in FP64, where 1/r^3 or
+// 1/r^5 would carry errors that are one for all of a tile's pairs into the sum (it
+// costs the single layers 0.2-0.4 %, which are exact enough without).  NROW: FP32 words per
+// source that the pairs read besides (s' where GRAD, then the densities).
+template <int KER> struct FarForm {
+  static constexpr bool ON = false;
+  static constexpr int NV = 0, NROW = 0;
+  static constexpr bool GRAD = false, T64 = false;
+};
+template <> struct FarForm<LAP_FXU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 0, NROW = 1;
+  static constexpr bool GRAD = false, T64 = false;
+};
+template <> struct FarForm<LAP_DXU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 1, NROW = 0;
+  static constexpr bool GRAD = false, T64 = true;
+};
+template <> struct FarForm<LAP_FXDU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 0, NROW = 4;
+  static constexpr bool GRAD = true, T64 = true;
+};
+template <> struct FarForm<STK_FXU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 1, NROW = 6;
+  static constexpr bool GRAD = true, T64 = false;
+};
+template <> struct FarForm<STK_DXU> {
+  static constexpr bool ON = true;
+  static constexpr int NV = 2, NROW = 3;
+  static constexpr bool GRAD = true, T64 = true;
+};
+
+// The fourth word of a tile's meta: H^2, and in the eight bits far below its
+// rounding to FP32 the exponent of the least |t'|^2 of the matrix cores
+// (mfma_min_t).  (In a word of its own, H^2 stays in a scalar register, which
+// costs the Stokes kernels 8 to 12 bytes of scratch.)
+__device__ __forceinline__ double meta_word(double h2, float min_t) {
+  return __hiloint2double(__double2hiint(h2), (__double2loint(h2) & ~0xff) | (__float_as_int(min_t) >> 23));
+}
+__device__ __forceinline__ float meta_min_t(double w) { return __int_as_float((__double2loint(w) & 0xff) << 23); }
+// Below the |t'|^2 returned, up to its power of two, a tile's pairs take the FP32
+// forms.  The matrix cores
+// may flush parts and products below 2^-126.  |t'|^2 is cut to parts of 2^-16 of
+// it, and v = f, n (or f n), `largest` the tile's largest, is multiplied with t' in
+// products down to 2^-24 |v| |t'|.  (Stokes FxU densities of 1e-35, 70000 x 30000
+// points: error 2.0e-6 on the matrix cores, 1.5e-7 so.)
+__device__ __forceinline__ float mfma_min_t(float largest) {
+  const float t = 0x1p-102f / largest;
+  return largest > 0.0f ? fmaxf(t * t, 0x1p-100f) : 0x1p-100f;
+}
+
 // One workgroup per tile: tile centre and H^2, then the records, sources in
-// the order perm[].  meta[tile] = {c_x, c_y, c_z, H^2}; sub[4 tile + q] =
+// the order perm[].  meta[tile] = {c_x, c_y, c_z, meta_word}; sub[4 tile + q] =
 // {b_x, b_y, b_z, h^2} of sub-tile q (sources 64q .. 64q + 63, one wave):
 // the centre of its FP32 offsets' bounding box, relative to the tile centre,
 // and the squared radius of its offsets about that centre ({0, 0, 0, 0} for
@@ -147,7 +204,7 @@ k_pack_tiles(const double* __restrict__ xs, const double* __restrict__ xn, const
   constexpr int K0 = K::K0, ND = K::ND, Q = MixLayout<KER>::Q;
   static_assert(TILE == WG, "one source per lane");
   __shared__ double red[WG / 64][6];
-  __shared__ float hred[WG / 64];
+  __shared__ float hred[WG / 64], vred[WG / 64][2];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if ((int64_t)blockIdx.x >= ntiles) {  // the workgroups after the tiles copy the targets into their order
     const int64_t q = ((int64_t)blockIdx.x - ntiles) * WG + tid;
@@ -203,12 +260,24 @@ k_pack_tiles(const double* __restrict__ xs, const double* __restrict__ xn, const
   }
   h2 = wave_max(h2);
   if (lane == 0) hred[wv] = h2;
+  // the largest of the vectors that the matrix cores take, as packed
+  constexpr int NV = FarForm<KER>::NV;
+#pragma unroll
+  for (int v = 0; v < NV; v++) {
+    const float* x = rec + (KER == LAP_DXU ? 4 : 3 + 3 * v);
+    const float m = wave_max(fmaxf(fabsf(x[0]), fmaxf(fabsf(x[1]), fabsf(x[2]))));
+    if (lane == 0) vred[wv][v] = m;
+  }
   __syncthreads();
   if (tid == 0) {
     float hm = hred[0];
 #pragma unroll
     for (int w = 1; w < WG / 64; w++) hm = fmaxf(hm, hred[w]);
-    meta[blockIdx.x] = make_double4(c[0], c[1], c[2], (double)hm * 1.0000001);
+    float min_t = mfma_min_t(1.0f);
+#pragma unroll
+    for (int v = 0; v < NV; v++)
+      min_t = fmaxf(min_t, mfma_min_t(fmaxf(fmaxf(vred[0][v], vred[1][v]), fmaxf(vred[2][v], vred[3][v]))));
+    meta[blockIdx.x] = make_double4(c[0], c[1], c[2], meta_word((double)hm * 1.0000001, min_t));
   }
   {
     float b[3], bh2 = 0.0f;
@@ -459,47 +528,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
-
-// A kernel's far form.  NV: dot products with t' - s' beside r^2 (DxU: nq;
-// Stokes: f, and n for the double layer).  GRAD: outputs along r = t' - s',
-// summed as t'_k (sum g) - (sum g s'_k).  T64: |t'|^2 is formed in FP64 and rounded
-// once, where 1/r^3 or 1/r^5 would carry its error, one for all of a tile's
-// pairs, into the sum (it costs the single layer 0.2 %).  NROW: FP32 words per
-// source that the pairs read besides (s' where GRAD, then the densities).
-template <int KER> struct FarForm {
-  static constexpr bool ON = false;
-  static constexpr int NV = 0, NROW = 0;
-  static constexpr bool GRAD = false, T64 = false;
-};
-template <> struct FarForm<LAP_FXU> {
-  static constexpr bool ON = true;
-  static constexpr int NV = 0, NROW = 1;
-  static constexpr bool GRAD = false, T64 = false;
-};
-template <> struct FarForm<LAP_DXU> {
-  static constexpr bool ON = true;
-  static constexpr int NV = 1, NROW = 0;
-  static constexpr bool GRAD = false, T64 = true;
-};
-template <> struct FarForm<LAP_FXDU> {
-  static constexpr bool ON = true;
-  static constexpr int NV = 0, NROW = 4;
-  static constexpr bool GRAD = true, T64 = true;
-};
-template <> struct FarForm<STK_FXU> {
-  static constexpr bool ON = true;
-  static constexpr int NV = 1, NROW = 6;
-  static constexpr bool GRAD = true, T64 = false;
-};
-template <> struct FarForm<STK_DXU> {
-  static constexpr bool ON = true;
-  static constexpr int NV = 2, NROW = 3;
-  static constexpr bool GRAD = true, T64 = true;
-};
 template <int KER> constexpr bool far_mfma() { return FarForm<KER>::ON; }
-// |t'|^2 below this takes the FP32 forms: the matrix cores may flush parts
-// below 2^-126, which are 2^-16 of |t'|^2.
-constexpr float MFMA_MIN_T = 0x1p-100f;
 
 struct Parts {
   float a, b, c;  // each used by its upper 16 bits
@@ -782,7 +811,7 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
         pn[k] = 0.0f;
       }
     };
-    const bool tiny = __builtin_amdgcn_ballot_w64(T < MFMA_MIN_T) != 0;
+    const bool tiny = __builtin_amdgcn_ballot_w64(T < meta_min_t(m.w)) != 0;
     if (__builtin_amdgcn_ballot_w64(T < 9.0f * H2) == 0 && !tiny) {
       far(0, std::integral_constant<int, CHUNKS>());
     } else {
@@ -828,9 +857,15 @@ k_eval_mixed_mfma(const double* __restrict__ xt, int64_t nt, const uint32_t* __r
     for (int k = 0; k < K1; k++) {
       ptn[k] += sum_rows(pf[0][k], pf[1][k], pf[2][k], pf[3][k]);
       if constexpr (F::GRAD) {
-        double x = t64[k];
-        asm volatile("" : "+v"(x));  // or the difference is held through the far loop
-        ptn[k] = fmad(x - (k == 0 ? m.x : (k == 1 ? m.y : m.z)), Gt, ptn[k]);
+        if constexpr (F::T64) {
+          double x = t64[k];
+          asm volatile("" : "+v"(x));  // or the difference is held through the far loop
+          ptn[k] = fmad(x - (k == 0 ? m.x : (k == 1 ? m.y : m.z)), Gt, ptn[k]);
+        } else {
+          float x = th[k];
+          asm volatile("" : "+v"(x));  // or the conversion is done in each pass of the far loop
+          ptn[k] = fmad((double)x, Gt, ptn[k]);
+        }
       }
       const double y = ptn[k] - comp[k];  // Kahan: acc += ptn
       const double sum = acc[k] + y;
