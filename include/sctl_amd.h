@@ -384,7 +384,8 @@ int sctl_amd_hilbert_order(const double* r_a, int64_t na, uint32_t* perm_a, cons
  * sctl_amd_eval / sctl_amd_plan_create with a matching key use the result. */
 int sctl_amd_tune_db_path(const char* path);
 
-/* Dense Eval: targets per lane {1,2,4} x workgroups-per-CU cap {none,3,2}.
+/* Dense Eval: targets per lane {1,2,4} x workgroups-per-CU cap {none,3,2}; one
+ * target per lane only where the mixed path has no other form.
  * Device pointers only; v_scratch (nt*K1) receives garbage. */
 int sctl_amd_tune_eval(int kernel, int precision, int digits, const double* r_trg, int64_t nt, const double* r_src,
                        const double* n_src, const double* v_src, int64_t ns, double* v_scratch, uint32_t flags,

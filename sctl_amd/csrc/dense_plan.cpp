@@ -121,6 +121,7 @@ int sctl_amd_dense_plan_create(sctl_amd_dense_plan* out, int kernel, int precisi
   p->ns = ns;
   p->ctx = kernel_needs_ctx(kernel) ? *ctx : 0.0;
   p->shape = pick_dense_shape(kernel, precision, p->newton, nt, ns);
+  if (!p->f64 && mixed_runs_mfma(kernel, nt, ns)) p->shape.tpl = 1;  // as it runs
   const hipMemcpyKind kind = (flags & SCTL_AMD_HOST_PTRS) ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
   auto copy = [&](double** dst, const double* src, int64_t n) -> int {
     if (n <= 0) return SCTL_AMD_SUCCESS;

@@ -159,6 +159,9 @@ int f64_apply(int ker, int newton, const double* r_trg, int64_t nt, const double
 // step with SCTL_AMD_MIXED_NEWTON): below a size the mixed path's orders, packing
 // and short tiles cost more than its cheaper pairs save.  mixed.hip.
 bool mixed_runs_f64(int ker, int64_t nt, int64_t ns);
+// Whether a mixed Eval of this size runs the matrix-core kernel, which has one
+// form whatever the targets per lane.
+bool mixed_runs_mfma(int ker, int64_t nt, int64_t ns);
 struct MixedGeometry {
   int ti = 0, Q = 0;
   bool mfma = false;  // the far form on the matrix cores

@@ -983,6 +983,10 @@ bool far_mfma_at(int ker, int64_t nt, int64_t ns) {
   }
 }
 
+bool mixed_runs_mfma(int ker, int64_t nt, int64_t ns) {
+  return !mixed_runs_f64(ker, nt, ns) && far_mfma_at(ker, nt, ns);
+}
+
 // Launch geometry of one mixed Eval: target blocks and the source splits.
 // Split the sources over gridDim.y when the target blocks cannot fill the
 // device (each split one tile at the least), and so that no split exceeds

@@ -181,7 +181,7 @@ DenseShape pick_dense_shape(int ker, int precision, int newton, int64_t nt, int6
   if (precision == SCTL_AMD_FP64)
     s.tpl = (!kernel_needs_ctx(ker) && nt >= (1 << 16)) ? 4 : 1;
   else
-    s.tpl = nt >= 256LL * 2 * 2048 ? 2 : 1;
+    s.tpl = nt >= 256LL * 2 * 2048 && !mixed_runs_mfma(ker, nt, ns) ? 2 : 1;
   return s;
 }
 
@@ -272,8 +272,9 @@ int sctl_amd_tune_eval(int kernel, int precision, int digits, const double* r_tr
   DenseShape bs;
   // The Helmholtz kernels are timed at wavenumber 1 (the shape does not depend on it).
   const double mu = kernel_needs_ctx(kernel) ? 1.0 : 0.0;
+  const bool one_form = precision == SCTL_AMD_MIXED && mixed_runs_mfma(kernel, nt, ns);
   for (int tpl : {1, 2, 4}) {
-    if (tpl > kernel_max_tpl(kernel)) continue;
+    if (tpl > (one_form ? 1 : kernel_max_tpl(kernel))) continue;
     for (int occ : {0, 3, 2}) {
       DenseShape sh;
       sh.tpl = tpl;
