@@ -176,8 +176,10 @@ int stage_in(Scratch& buf, const double* host, int64_t n, hipStream_t s, const d
 // buffers (allocated with hipHostMalloc on first use and reused; PIN_KEEP free
 // ones are kept, more go back to the driver), two per call so that the copy of
 // one chunk into the caller's memory overlaps the DMA of the next.  A host Eval
-// that fits one chunk goes through one (eval_host_small).
-constexpr size_t PIN_CHUNK = (size_t)8 << 20, PIN_KEEP = 32;
+// that fits one chunk goes through one (eval_host_small).  256 chunks (2 GiB, if
+// ever in use at once) serve 128 threads' KernelMatrix calls without allocating:
+// with 32 kept, 64 threads' 400 x 500 matrices took 128 us each, with 256 99.
+constexpr size_t PIN_CHUNK = (size_t)8 << 20, PIN_KEEP = 256;
 std::mutex g_pin_mutex;
 std::vector<void*> g_pin_free;
 
