@@ -24,6 +24,10 @@
  *    stream).  Device-pointer calls are asynchronous on that stream.
  *  - Thread-safe: calls from different host threads on different streams may
  *    overlap.  Plans (sctl_amd_plan) are not shared between threads.
+ *  - A plan (sctl_amd_plan, sctl_amd_dense_plan) holds the scratch of its
+ *    applies: applies of one plan on several streams, and replays of graphs of
+ *    it, must be ordered by the caller.  The near-field matrix and GEMV of a plan
+ *    keep nothing in it and may overlap.
  */
 #ifndef SCTL_AMD_H_
 #define SCTL_AMD_H_
