@@ -192,7 +192,7 @@ int pin_take(void** p) {
       return SCTL_AMD_SUCCESS;
     }
   }
-  SCTL_HIP_TRY(hipHostMalloc(p, PIN_CHUNK, hipHostMallocDefault));
+  SCTL_HIP_TRY(hipHostMalloc(p, PIN_CHUNK, hipHostMallocPortable));  // whichever device takes it next
   return SCTL_AMD_SUCCESS;
 }
 void pin_give(void* p) {
