@@ -389,7 +389,8 @@ int sctl_amd_hilbert_order(const double* r_a, int64_t na, uint32_t* perm_a, cons
 int sctl_amd_tune_db_path(const char* path);
 
 /* Dense Eval: targets per lane {1,2,4} x workgroups-per-CU cap {none,3,2}; one
- * target per lane only where the mixed path has no other form.
+ * target per lane only where the mixed path has no other form.  Each timed
+ * once, the three fastest again; the best of that second pass is recorded.
  * Device pointers only; v_scratch (nt*K1) receives garbage. */
 int sctl_amd_tune_eval(int kernel, int precision, int digits, const double* r_trg, int64_t nt, const double* r_src,
                        const double* n_src, const double* v_src, int64_t ns, double* v_scratch, uint32_t flags,

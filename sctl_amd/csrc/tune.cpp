@@ -268,11 +268,25 @@ int sctl_amd_tune_eval(int kernel, int precision, int digits, const double* r_tr
   SCTL_TRY(device_info(&dev));
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : hipStreamPerThread;
   const int newton = precision == SCTL_AMD_FP64 ? newton_steps_f64(digits) : ((flags & SCTL_AMD_MIXED_NEWTON) ? 1 : 0);
-  double best = 1e300;
-  DenseShape bs;
+  // Every candidate once, then the three fastest again, the best of that second
+  // pass winning: the first one runs before the clock has risen (2^20 x 2^20 mixed,
+  // three candidates timed once: the cap of 3 was taken, 119 ms against 110).
+  struct Cand {
+    double ms;
+    DenseShape sh;
+  };
+  std::vector<Cand> cands;
   // The Helmholtz kernels are timed at wavenumber 1 (the shape does not depend on it).
   const double mu = kernel_needs_ctx(kernel) ? 1.0 : 0.0;
   const bool one_form = precision == SCTL_AMD_MIXED && mixed_runs_mfma(kernel, nt, ns);
+  auto timed = [&](const DenseShape& sh, double* ms) {
+    auto run = [&]() {
+      return precision == SCTL_AMD_FP64
+                 ? launch_eval_f64(kernel, newton, r_trg, nt, r_src, n_src, v_src, ns, v_scratch, sh, mu, s)
+                 : launch_eval_mixed(kernel, newton, r_trg, nt, r_src, n_src, v_src, ns, v_scratch, sh, mu, s);
+    };
+    return time_ms(run, s, 2, ms);
+  };
   for (int tpl : {1, 2, 4}) {
     if (tpl > (one_form ? 1 : kernel_max_tpl(kernel))) continue;
     for (int occ : {0, 3, 2}) {
@@ -280,16 +294,19 @@ int sctl_amd_tune_eval(int kernel, int precision, int digits, const double* r_tr
       sh.tpl = tpl;
       sh.occ = occ;
       double ms = 0;
-      auto run = [&]() {
-        return precision == SCTL_AMD_FP64
-                   ? launch_eval_f64(kernel, newton, r_trg, nt, r_src, n_src, v_src, ns, v_scratch, sh, mu, s)
-                   : launch_eval_mixed(kernel, newton, r_trg, nt, r_src, n_src, v_src, ns, v_scratch, sh, mu, s);
-      };
-      SCTL_TRY(time_ms(run, s, 2, &ms));
-      if (ms < best) {
-        best = ms;
-        bs = sh;
-      }
+      SCTL_TRY(timed(sh, &ms));
+      cands.push_back({ms, sh});
+    }
+  }
+  std::sort(cands.begin(), cands.end(), [](const Cand& a, const Cand& b) { return a.ms < b.ms; });
+  double best = 1e300;
+  DenseShape bs;
+  for (size_t i = 0; i < std::min<size_t>(3, cands.size()); i++) {
+    double ms = 0;
+    SCTL_TRY(timed(cands[i].sh, &ms));
+    if (ms < best) {
+      best = ms;
+      bs = cands[i].sh;
     }
   }
   store(dense_key(kernel, precision, newton, nt, ns), {(double)bs.tpl, (double)bs.occ, best});
