@@ -166,16 +166,16 @@ k_blocks_f64(const Item* __restrict__ items, int nitems,
         group_sources<STAGE>(lg, g, len, [&](int i) {
           const double* rec = lds + i * R;
           if constexpr (KER == LAP_DXU) {
-  #pragma unroll
+#pragma unroll
             for (int j = 0; j < TPL; j++)
               lap_dxu_fn<N, false>(acc[j][0], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], rec + 3);
           } else {
             double n[3] = {0, 0, 0}, f[K0];
-  #pragma unroll
+#pragma unroll
             for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
-  #pragma unroll
+#pragma unroll
             for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
-  #pragma unroll
+#pragma unroll
             for (int j = 0; j < TPL; j++)
               interact<KER, N, false>(acc[j], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], n, f, mu);
           }
@@ -202,14 +202,14 @@ k_blocks_f64(const Item* __restrict__ items, int nitems,
           for (int i = g; i < len; i += G) {
             const double* rec = lds + i * R;
             if constexpr (KER == LAP_DXU) {
-  #pragma unroll
+#pragma unroll
               for (int j = 0; j < TPL; j++)
                 lap_dxu_fn<N, true>(acc[j][0], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], rec + 3);
             } else {
               double n[3] = {0, 0, 0}, f[K0];
               for (int k = 0; k < ND; k++) n[k] = rec[3 + k];
               for (int k = 0; k < K0; k++) f[k] = rec[3 + ND + k];
-  #pragma unroll
+#pragma unroll
               for (int j = 0; j < TPL; j++)
                 interact<KER, N, true>(acc[j], tx[j] - rec[0], ty[j] - rec[1], tz[j] - rec[2], n, f, mu);
             }
